@@ -251,45 +251,191 @@ template <int WT, int MODE> __global__ __launch_bounds__(256) void k_rms_norm_ge
     }
 }
 
-// ggml_norm (LayerNorm without the affine part), one wave per row: the mean
-// from a double sum, the variance from a double sum of the f32 centred values
-// v = x - mean, scale = 1/sqrtf(variance + eps), y = v*scale (ggml-CPU's
-// order of roundings; the sums' order differs, within the tolerance). The
-// row is read three times, the later reads from cache. Sites:
-// qwen3-tts/codec.cpp:216 (ConvNeXt), kokoro/operations.cpp:12,93.
-__global__ __launch_bounds__(256) void k_layer_norm(const NormArgs a) {
-    const int     lane = threadIdx.x % kWave;
-    const int64_t row  = static_cast<int64_t>(blockIdx.x) * (256 / kWave) + threadIdx.x / kWave;
-    if (row >= a.nrows) {
-        return;
+// Sum of a double over the TPR lanes that share a row (TPR a power of two from
+// 64 up, dividing the block): the wave's sum, then for more than one wave the
+// waves' sums through `part` (one slot per wave) in wave order. Every thread
+// of the block takes part; two calls need two `part` arrays.
+template <int TPR> __device__ __forceinline__ double row_sum(double v, double * part) {
+    v = group_sum<kWave>(v);
+    if constexpr (TPR > kWave) {
+        constexpr int kWaves = TPR / kWave;
+        const int     wave   = static_cast<int>(threadIdx.x) / kWave;
+        if (threadIdx.x % kWave == 0) {
+            part[wave] = v;
+        }
+        __syncthreads();
+        const int first = wave / kWaves * kWaves;
+        v               = part[first];
+#pragma unroll
+        for (int k = 1; k < kWaves; ++k) {
+            v += part[first + k];
+        }
     }
-    const float * xr  = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, row));
-    float *       yr  = reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, row));
-    double        acc = 0.0;
-    for (int i = lane; i < a.ne0; i += kWave) {
-        acc += static_cast<double>(xr[i]);
+    return v;
+}
+
+// ggml_norm (LayerNorm without the affine part): the mean from a double sum,
+// the variance from a double sum of the squared f32 centred values v = x -
+// mean, scale = 1/sqrtf(variance + eps), y = v*scale (ggml-CPU's order of
+// roundings; the sums' order differs, within the tolerance). Sites:
+// qwen3-tts/codec.cpp:216 (ConvNeXt, rows of 1024 channels),
+// kokoro/operations.cpp:12,93 (AdaIN: 64-512 rows of a whole utterance's
+// samples, of any length).
+//
+// HBM-bound: x read once and y written once. A row stays in the registers of
+// the TPR lanes that share it between the two reductions and the store, VPL
+// float4 each (the last ne0 % 4 values one per lane), so both reductions and
+// the store run from one pass over memory. Rows of odd length start on any
+// 4-byte boundary: the 16-byte accesses are the unaligned form. Measured on
+// MI355X (cold) against one wave per row reading the row three times with
+// 4-byte accesses: 128 rows of 24001 253 -> 8.3 us, 256 of 4001 43 -> 4.5,
+// 1000 of 1024 13.2 -> 4.0, 8192 of 1024 28.2 -> 13.5, 300 of 8192 87.6 -> 5.7,
+// 64 of 65536 646 -> 12.5.
+template <int TPR, int VPL> __global__ __launch_bounds__(TPR > 256 ? TPR : 256) void k_layer_norm(const NormArgs a) {
+    constexpr int     kBlock = TPR > 256 ? TPR : 256;
+    __shared__ double s_mean[kBlock / kWave], s_var[kBlock / kWave];
+    const int         l    = static_cast<int>(threadIdx.x) % TPR;
+    const int64_t     row  = static_cast<int64_t>(blockIdx.x) * (kBlock / TPR) + row_in_block<TPR>();
+    const bool        live = row < a.nrows;
+    const int64_t     rr   = live ? row : 0;
+    const int         n4   = live ? a.ne0 / 4 : 0;
+    const int         tail = live ? a.ne0 % 4 : 0;
+    const float *     xr = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, rr));
+    float *           yr = reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, rr));
+    f32x4             v[VPL];
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        const int c = l + TPR * k;
+        v[k]        = c < n4 ? ld_stream4u(xr + c * 4) : splat4(0.0f);
     }
-    const float mean = static_cast<float>(group_sum<kWave>(acc) / static_cast<double>(a.ne0));
-    double      acc2 = 0.0;
-    for (int i = lane; i < a.ne0; i += kWave) {
-        const float v = xr[i] - mean;
-        acc2 += static_cast<double>(v * v);
+    float  last = l < tail ? xr[n4 * 4 + l] : 0.0f;
+    double acc  = static_cast<double>(last);
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        acc += (static_cast<double>(v[k].x) + static_cast<double>(v[k].y)) +
+               (static_cast<double>(v[k].z) + static_cast<double>(v[k].w));
     }
-    const float variance = static_cast<float>(group_sum<kWave>(acc2) / static_cast<double>(a.ne0));
+    const float mean = static_cast<float>(row_sum<TPR>(acc, s_mean) / static_cast<double>(a.ne0));
+    last             = last - mean;
+    acc              = l < tail ? static_cast<double>(last * last) : 0.0;
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        v[k]            = f32x4{ v[k].x - mean, v[k].y - mean, v[k].z - mean, v[k].w - mean };
+        const double sq = sq4v(v[k]);
+        acc += l + TPR * k < n4 ? sq : 0.0;
+    }
+    const float variance = static_cast<float>(row_sum<TPR>(acc, s_var) / static_cast<double>(a.ne0));
     const float scale    = 1.0f / __builtin_sqrtf(variance + a.eps);
-    for (int i = lane; i < a.ne0; i += kWave) {
-        yr[i] = (xr[i] - mean) * scale;
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        const int c = l + TPR * k;
+        if (c < n4) {
+            st_stream4u(yr + c * 4,
+                      f32x4{ v[k].x * scale, v[k].y * scale, v[k].z * scale, v[k].w * scale });
+        }
     }
+    if (l < tail) {
+        yr[n4 * 4 + l] = last * scale;
+    }
+}
+
+// Rows too long for the registers of one block (kLayerNormMax values): one
+// 1024-thread block per row and three passes, the later ones from cache.
+// 128 rows of 131072: 1988 -> 43 us.
+constexpr int kLayerNormMax  = 1024 * 16 * 4;
+constexpr int kLayerNormWide = 1024;
+
+__global__ __launch_bounds__(kLayerNormWide) void k_layer_norm_wide(const NormArgs a) {
+    __shared__ double s_mean[kLayerNormWide / kWave], s_var[kLayerNormWide / kWave];
+    const int         l    = static_cast<int>(threadIdx.x);
+    const int64_t     row  = blockIdx.x;
+    const int         n4   = a.ne0 / 4;
+    const int         tail = a.ne0 % 4;
+    const float *     xr = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, row));
+    float *           yr = reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, row));
+    const float       last = l < tail ? xr[n4 * 4 + l] : 0.0f;
+    double            acc  = static_cast<double>(last);
+#pragma unroll 4
+    for (int c = l; c < n4; c += kLayerNormWide) {
+        const f32x4 v = ld4u(xr + c * 4);
+        acc += (static_cast<double>(v.x) + static_cast<double>(v.y)) + (static_cast<double>(v.z) + static_cast<double>(v.w));
+    }
+    const float mean = static_cast<float>(row_sum<kLayerNormWide>(acc, s_mean) / static_cast<double>(a.ne0));
+    acc              = l < tail ? static_cast<double>((last - mean) * (last - mean)) : 0.0;
+#pragma unroll 4
+    for (int c = l; c < n4; c += kLayerNormWide) {
+        const f32x4 v = ld4u(xr + c * 4);
+        acc += sq4v(f32x4{ v.x - mean, v.y - mean, v.z - mean, v.w - mean });
+    }
+    const float variance = static_cast<float>(row_sum<kLayerNormWide>(acc, s_var) / static_cast<double>(a.ne0));
+    const float scale    = 1.0f / __builtin_sqrtf(variance + a.eps);
+#pragma unroll 4
+    for (int c = l; c < n4; c += kLayerNormWide) {
+        const f32x4 v = ld4u(xr + c * 4);
+        st_stream4u(yr + c * 4, f32x4{ (v.x - mean) * scale, (v.y - mean) * scale,
+                                                             (v.z - mean) * scale, (v.w - mean) * scale });
+    }
+    if (l < tail) {
+        yr[n4 * 4 + l] = (last - mean) * scale;
+    }
+}
+
+// Lanes per row: enough that a lane holds one float4 where the rows are many
+// (the RMSNorm rule), and 1024 where they are too few to fill the chip with
+// 256-thread blocks (kLayerNormFewRows: one block per CU) or too long for one.
+// From kLayerNormManyRows rows of up to 2048 values the chip is full either way
+// and fewer lanes per row, with more loads in flight each, are ahead, as for
+// the RMSNorm (8192 rows of 1024: 256 lanes 15.7 us, 64 lanes 13.5).
+constexpr int64_t kLayerNormFewRows  = 256;
+constexpr int64_t kLayerNormManyRows = 2048;
+
+shp_status_t launch_layer_norm(const NormArgs & a, hipStream_t stream) {
+    auto go = [&](auto kernel, int tpr) {
+        const int     block  = tpr > 256 ? tpr : 256;
+        const int64_t blocks = (a.nrows + block / tpr - 1) / (block / tpr);
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(block), 0, stream, a);
+        return launch_status();
+    };
+    const int n4 = a.ne0 / 4;
+    if (a.ne0 > kLayerNormMax) {
+        hipLaunchKernelGGL(k_layer_norm_wide, dim3(static_cast<unsigned>(a.nrows)), dim3(kLayerNormWide), 0, stream, a);
+        return launch_status();
+    }
+    if (n4 <= 64) {
+        return go(k_layer_norm<64, 1>, 64);
+    }
+    if (n4 <= 128) {
+        return go(k_layer_norm<128, 1>, 128);
+    }
+    if (n4 <= 256) {
+        return a.nrows <= kLayerNormManyRows     ? go(k_layer_norm<256, 1>, 256) :
+               a.nrows <= 3 * kLayerNormManyRows ? go(k_layer_norm<128, 2>, 128) : go(k_layer_norm<64, 4>, 64);
+    }
+    if (n4 <= 512 && a.nrows > kLayerNormManyRows) {
+        return go(k_layer_norm<128, 4>, 128);
+    }
+    if (a.nrows > kLayerNormFewRows && n4 <= 2048) {
+        return n4 <= 512 ? go(k_layer_norm<256, 2>, 256) :
+               n4 <= 1024 ? go(k_layer_norm<256, 4>, 256) : go(k_layer_norm<256, 8>, 256);
+    }
+    return n4 <= 1024 ? go(k_layer_norm<1024, 1>, 1024) :
+           n4 <= 2048 ? go(k_layer_norm<1024, 2>, 1024) :
+           n4 <= 4096 ? go(k_layer_norm<1024, 4>, 1024) :
+           n4 <= 8192 ? go(k_layer_norm<1024, 8>, 1024) : go(k_layer_norm<1024, 16>, 1024);
 }
 
 // ggml_sum_rows / ggml_mean, and the product-sum of ggml_mul then
 // ggml_sum_rows (the speaker encoder's attention-weighted statistics,
-// qwen3-tts/speaker-encoder.cpp:292-293,374): one wave per row, each lane
-// accumulating its f32 values (or f32 products) into a double in element
-// order, the lanes' doubles summed by DPP moves and rounded to f32 once; the
-// mean divides that f32 by ne0 in f32. ggml-CPU accumulates the row in double
-// in element order: the f32 results agree unless the two double sums fall on
-// opposite sides of an f32 rounding boundary.
+// qwen3-tts/speaker-encoder.cpp:292-293,374): TPR lanes per row, each
+// accumulating its f32 values (or f32 products) into a double, the lanes'
+// doubles summed by DPP moves, the waves' through LDS, and rounded to f32
+// once; the mean divides that f32 by ne0 in f32. ggml-CPU accumulates the row
+// in double in element order: the f32 results agree unless the two double
+// sums fall on opposite sides of an f32 rounding boundary. 16-byte loads from
+// any 4-byte boundary (the pooled frames of a clip are rows of any length).
+// Measured on MI355X (cold) against one wave per row with 4-byte loads: 1536
+// rows of 937 9.2 -> 3.4 us (products 10.1 -> 4.6), 128 of 24001 164 -> 5.3;
+// 4096 of 1024, one wave per row in both, 5.2 -> 4.7.
 enum SumRowsMode { kSumRows = 0, kMeanRows = 1, kMulSumRows = 2 };
 
 struct SumRowsArgs {
@@ -304,44 +450,59 @@ struct SumRowsArgs {
     int32_t       pad;
 };
 
-template <int MODE, bool VEC> __global__ __launch_bounds__(256) void k_sum_rows(const SumRowsArgs a) {
-    const int     lane = threadIdx.x % kWave;
-    const int64_t row  = static_cast<int64_t>(blockIdx.x) * (256 / kWave) + threadIdx.x / kWave;
-    if (row >= a.nrows) {
-        return;
-    }
-    const float * xr  = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, row));
-    const float * wr  = MODE == kMulSumRows ?
-                            reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.w) + row_offset(a.wm, row)) :
-                            nullptr;
-    double        acc = 0.0;
-    if constexpr (VEC) {
-        const int nvec = a.ne0 / 4;
-        for (int i = lane; i < nvec; i += kWave) {
-            f32x4 v = ld_stream(reinterpret_cast<const f32x4 *>(xr) + i);
-            if constexpr (MODE == kMulSumRows) {
-                const f32x4 u = ld_stream(reinterpret_cast<const f32x4 *>(wr) + i);
-                v             = f32x4{ v.x * u.x, v.y * u.y, v.z * u.z, v.w * u.w };
-            }
-            acc += static_cast<double>(v.x);
-            acc += static_cast<double>(v.y);
-            acc += static_cast<double>(v.z);
-            acc += static_cast<double>(v.w);
+template <int MODE, int TPR> __global__ __launch_bounds__(TPR > 256 ? TPR : 256) void k_sum_rows(const SumRowsArgs a) {
+    constexpr int     kBlock = TPR > 256 ? TPR : 256;
+    __shared__ double s_part[kBlock / kWave];
+    const int         l    = static_cast<int>(threadIdx.x) % TPR;
+    const int64_t     row  = static_cast<int64_t>(blockIdx.x) * (kBlock / TPR) + row_in_block<TPR>();
+    const bool        live = row < a.nrows;
+    const int64_t     rr   = live ? row : 0;
+    const int         n4   = live ? a.ne0 / 4 : 0;
+    const int         tail = live ? a.ne0 % 4 : 0;
+    const float *     xr = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, rr));
+    const float *     wr = MODE == kMulSumRows ?
+                               reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.w) + row_offset(a.wm, rr)) :
+                               nullptr;
+    double            acc = 0.0;
+#pragma unroll 4
+    for (int c = l; c < n4; c += TPR) {
+        f32x4 v = ld_stream4u(xr + c * 4);
+        if constexpr (MODE == kMulSumRows) {
+            const f32x4 u = ld_stream4u(wr + c * 4);
+            v             = f32x4{ v.x * u.x, v.y * u.y, v.z * u.z, v.w * u.w };
         }
-    } else {
-        for (int i = lane; i < a.ne0; i += kWave) {
-            const float v = MODE == kMulSumRows ? xr[i] * wr[i] : xr[i];
-            acc += static_cast<double>(v);
-        }
+        acc += static_cast<double>(v.x);
+        acc += static_cast<double>(v.y);
+        acc += static_cast<double>(v.z);
+        acc += static_cast<double>(v.w);
     }
-    acc = group_sum<kWave>(acc);
-    if (lane == 0) {
+    if (l < tail) {
+        const int   i = n4 * 4 + l;
+        const float v = MODE == kMulSumRows ? xr[i] * wr[i] : xr[i];
+        acc += static_cast<double>(v);
+    }
+    acc = row_sum<TPR>(acc, s_part);
+    if (live && l == 0) {
         float v = static_cast<float>(acc);
         if constexpr (MODE == kMeanRows) {
             v = v / static_cast<float>(a.ne0);
         }
         *reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, row)) = v;
     }
+}
+
+// One wave per row fills the chip from 2048 rows (8 waves per CU); fewer rows
+// take 256 lanes each, and up to one row per CU 1024.
+template <int MODE> shp_status_t launch_sum_rows(const SumRowsArgs & a, hipStream_t stream) {
+    const int n4 = a.ne0 / 4;
+    if (n4 <= 64 || a.nrows >= 2048) {
+        hipLaunchKernelGGL((k_sum_rows<MODE, 64>), dim3(static_cast<unsigned>((a.nrows + 3) / 4)), dim3(256), 0, stream, a);
+    } else if (n4 <= 512 || a.nrows > kLayerNormFewRows) {
+        hipLaunchKernelGGL((k_sum_rows<MODE, 256>), dim3(static_cast<unsigned>(a.nrows)), dim3(256), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL((k_sum_rows<MODE, 1024>), dim3(static_cast<unsigned>(a.nrows)), dim3(1024), 0, stream, a);
+    }
+    return launch_status();
 }
 
 template <int MODE> shp_status_t sum_rows_entry(const shp_tensor * x, const shp_tensor * w, shp_tensor * y,
@@ -369,19 +530,11 @@ template <int MODE> shp_status_t sum_rows_entry(const shp_tensor * x, const shp_
     a.ym    = make_rowmap(*y);
     a.nrows = nrows(*x);
     a.ne0   = static_cast<int32_t>(x->ne[0]);
-    bool vec = x->ne[0] % 4 == 0 && rows_aligned(*x, 16);
     if constexpr (MODE == kMulSumRows) {
         a.w  = static_cast<const float *>(w->data);
         a.wm = make_rowmap(*w);
-        vec  = vec && rows_aligned(*w, 16);
     }
-    const dim3 grid(static_cast<unsigned>((a.nrows + 3) / 4)), block(256);
-    if (vec) {
-        hipLaunchKernelGGL((k_sum_rows<MODE, true>), grid, block, 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((k_sum_rows<MODE, false>), grid, block, 0, stream, a);
-    }
-    return launch_status();
+    return launch_sum_rows<MODE>(a, stream);
 }
 
 template <int WT, int MODE> shp_status_t launch_norm(const NormArgs & a, bool vec, hipStream_t stream) {
@@ -1251,9 +1404,7 @@ extern "C" shp_status_t shp_norm(const shp_tensor * x, float eps, shp_tensor * y
     a.nrows              = nrows(*x);
     a.ne0                = static_cast<int32_t>(x->ne[0]);
     a.eps                = eps;
-    const int64_t blocks = (a.nrows + 3) / 4;
-    hipLaunchKernelGGL(k_layer_norm, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream), a);
-    return launch_status();
+    return launch_layer_norm(a, as_stream(stream));
 }
 
 extern "C" shp_status_t shp_sum_rows(const shp_tensor * x, shp_tensor * y, shp_stream_t stream) {

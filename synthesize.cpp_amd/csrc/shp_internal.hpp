@@ -30,6 +30,24 @@ __device__ __forceinline__ void st_stream(f32x4 * p, f32x4 v) {
     __builtin_nontemporal_store(v, p);
 }
 
+// Four consecutive f32 at any 4-byte boundary: global_load/store_dwordx4 needs
+// dword alignment only on gfx950, so a row that starts off a 16-byte boundary
+// still moves 16 bytes per lane (its lines are shared between two lanes'
+// accesses where it crosses them).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ f32x4 ld_stream4u(const float * p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const f32x4u *>(p));
+}
+
+__device__ __forceinline__ f32x4 ld4u(const float * p) {
+    return *reinterpret_cast<const f32x4u *>(p);
+}
+
+__device__ __forceinline__ void st_stream4u(float * p, f32x4 v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<f32x4u *>(p));
+}
+
 __device__ __forceinline__ float ld_stream(const float * p) {
     return __builtin_nontemporal_load(p);
 }
