@@ -10,6 +10,7 @@ energies are held within 1e-5 and > 99 % identical."""
 import numpy as np
 import pytest
 
+import ggml_ref as R
 from test_gpu_parity import _np, _t
 from test_oracle_goldens import MEL, oracle_log_mel
 
@@ -63,3 +64,50 @@ def test_log_mel_refusals(gpu):
         gpu.log_mel(pcm, fb, 1024, 256, 1100)
     with pytest.raises(gpu.ShpError):       # a filterbank of another transform
         gpu.log_mel(pcm, fb, 512, 128, 512)
+
+
+@pytest.mark.parametrize("n_fft,hop,win,bins,dense", [(2, 1, 2, 3, True), (4, 2, 3, 5, True), (8, 3, 8, 4, True),
+                                                      (16, 16, 16, 7, True), (32, 5, 20, 6, True), (64, 16, 64, 513, True),
+                                                      (128, 31, 100, 20, False), (256, 64, 256, 1025, True),
+                                                      (512, 512, 512, 512, False), (1024, 300, 1000, 40, True),
+                                                      (2048, 700, 1500, 128, False)])
+def test_log_mel_transform_sizes_and_filterbanks(gpu, n_fft, hop, win, bins, dense):
+    """Every pass length of the transform, windows of any width, more bins than
+    one span table holds, frame counts that leave a block part empty; filter
+    rows of any weights, and rows with zeros inside, at the ends or throughout.
+    (Held by the energies, as the production cases: 1e-5 absolute on the log.)"""
+    rng = np.random.default_rng([SEED, n_fft, bins])
+    nf = n_fft // 2 + 1
+    pcm = (rng.standard_normal(5 * n_fft + 3 * hop + 7) * 0.3).astype(np.float32)
+    fb = rng.uniform(0.1, 1.0, (bins, nf)).astype(np.float32)
+    if not dense:
+        fb[rng.random((bins, nf)) < 0.7] = 0.0
+        fb[1] = 0.0
+        fb[2] = -0.0
+        fb[0, -1] = 0.5
+    got = _np(gpu.log_mel(_t(gpu, pcm), _t(gpu, fb), n_fft, hop, win))
+    ref = R.run(lambda g: g.log_mel(pcm, fb, n_fft, hop, win))
+    _close(got, ref)
+
+
+def test_log_mel_one_sample_frames(gpu):
+    """n_fft 1: the periodic window's only value is 0, so every bin is the floor of sqrt(1e-9) times its weight."""
+    fb = np.float32([[1.0], [3.0]])
+    got = _np(gpu.log_mel(_t(gpu, np.ones(5, np.float32)), _t(gpu, fb), 1, 1, 1))
+    amp = np.float32(np.sqrt(1e-9))
+    assert np.abs(got - np.log(fb.T.astype(np.float64) * amp)).max() <= 1e-6
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan, 3e38])
+def test_log_mel_infinite_amplitudes(gpu, value):
+    """A sample that is not finite, or whose transform overflows: its frames'
+    zero weights multiply an infinity, which the host code's dense sum turns
+    into NaN; the other frames are untouched."""
+    rng = np.random.default_rng(SEED + 9)
+    pcm = (rng.standard_normal(24000) * 0.2).astype(np.float32)
+    pcm[9000:9003] = value
+    ref, got = oracle_log_mel(pcm, MEL), _gpu_mel(gpu, pcm, MEL)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.isnan(ref).any()
+    assert np.array_equal(np.isinf(got), np.isinf(ref))
+    ok = np.isfinite(ref)
+    _close(got[ok], ref[ok])
