@@ -82,10 +82,6 @@ struct EwArgs {
     int32_t       tail;   // flat path: elements past the last float4
 };
 
-__device__ __forceinline__ float silu(float x) {
-    return x / (1.0f + expf(-x));
-}
-
 // ggml's leaky: (x > 0 ? x : 0) + slope * (x < 0 ? x : 0), so -0 and NaN give +0.
 __device__ __forceinline__ float leaky(float x, float slope) {
     const float pos = x > 0.0f ? x : 0.0f;

@@ -1234,25 +1234,33 @@ bool part_aligned(const shp_tensor & t) {
     return reinterpret_cast<uintptr_t>(t.data) % 16 == 0 && t.nb[1] % 16 == 0 && t.nb[2] % 16 == 0;
 }
 
-shp_status_t rope_entry(const shp_tensor * q,
-                        const shp_tensor * k,
-                        const shp_tensor * v,
-                        const shp_tensor * wq,
-                        const shp_tensor * wk,
-                        bool               norm,
-                        float              eps,
-                        const shp_tensor * pos,
-                        int32_t            n_dims,
-                        float              freq_base,
-                        float              freq_scale,
-                        float              attn_factor,
-                        shp_tensor *       q_out,
-                        shp_tensor *       k_out,
-                        shp_tensor *       v_out,
-                        shp_stream_t       stream,
-                        const int32_t *    slot   = nullptr,
-                        int32_t *          status = nullptr,
-                        int64_t            cap    = 0) {
+// A checked rope launch: its arguments, gain kind and whether the 128-wide
+// kernels take it.
+struct RopePlan {
+    RopeArgs args{};
+    int      wkind = kWNone;
+    bool     fast  = false;
+};
+
+shp_status_t plan_rope(const shp_tensor * q,
+                       const shp_tensor * k,
+                       const shp_tensor * v,
+                       const shp_tensor * wq,
+                       const shp_tensor * wk,
+                       bool               norm,
+                       float              eps,
+                       const shp_tensor * pos,
+                       int32_t            n_dims,
+                       float              freq_base,
+                       float              freq_scale,
+                       float              attn_factor,
+                       shp_tensor *       q_out,
+                       shp_tensor *       k_out,
+                       shp_tensor *       v_out,
+                       const int32_t *    slot,
+                       int32_t *          status,
+                       int64_t            cap,
+                       RopePlan &         plan) {
     if (!rope_part_ok(q, q_out) || !well_formed(pos) || pos->type != SHP_TYPE_I32) {
         return SHP_ERR_INVALID_ARG;
     }
@@ -1306,8 +1314,8 @@ shp_status_t rope_entry(const shp_tensor * q,
         return SHP_ERR_UNSUPPORTED;
     }
 
-    RopeArgs a{};
-    auto     fill = [](RopePart & P, const shp_tensor * x, shp_tensor * y, const shp_tensor * w) {
+    RopeArgs & a    = plan.args;
+    auto       fill = [](RopePart & P, const shp_tensor * x, shp_tensor * y, const shp_tensor * w) {
         P.x     = static_cast<const float *>(x->data);
         P.y     = static_cast<float *>(y->data);
         P.w     = w != nullptr ? w->data : nullptr;
@@ -1358,11 +1366,44 @@ shp_status_t rope_entry(const shp_tensor * q,
     if (a.npos > INT32_MAX) {
         return SHP_ERR_UNSUPPORTED;
     }
-    const hipStream_t st = as_stream(stream);
-    if (v != nullptr) {
-        return norm ? dispatch_rope_w<true, true>(a, wkind, fast, st) : dispatch_rope_w<false, true>(a, kWNone, fast, st);
+    plan.wkind = wkind;
+    plan.fast  = fast;
+    return SHP_OK;
+}
+
+shp_status_t rope_entry(const shp_tensor * q,
+                        const shp_tensor * k,
+                        const shp_tensor * v,
+                        const shp_tensor * wq,
+                        const shp_tensor * wk,
+                        bool               norm,
+                        float              eps,
+                        const shp_tensor * pos,
+                        int32_t            n_dims,
+                        float              freq_base,
+                        float              freq_scale,
+                        float              attn_factor,
+                        shp_tensor *       q_out,
+                        shp_tensor *       k_out,
+                        shp_tensor *       v_out,
+                        shp_stream_t       stream,
+                        const int32_t *    slot   = nullptr,
+                        int32_t *          status = nullptr,
+                        int64_t            cap    = 0) {
+    RopePlan           plan;
+    const shp_status_t st = plan_rope(q, k, v, wq, wk, norm, eps, pos, n_dims, freq_base, freq_scale, attn_factor, q_out,
+                                      k_out, v_out, slot, status, cap, plan);
+    if (st != SHP_OK) {
+        return st;
     }
-    return norm ? dispatch_rope_w<true, false>(a, wkind, fast, st) : dispatch_rope_w<false, false>(a, kWNone, fast, st);
+    const RopeArgs &  a  = plan.args;
+    const hipStream_t hs = as_stream(stream);
+    if (v != nullptr) {
+        return norm ? dispatch_rope_w<true, true>(a, plan.wkind, plan.fast, hs) :
+                      dispatch_rope_w<false, true>(a, kWNone, plan.fast, hs);
+    }
+    return norm ? dispatch_rope_w<true, false>(a, plan.wkind, plan.fast, hs) :
+                  dispatch_rope_w<false, false>(a, kWNone, plan.fast, hs);
 }
 
 // The rows [filled, filled + T) of a KV cache [head_dim, kv_heads, capacity, 1]
@@ -1379,7 +1420,317 @@ bool cache_view(const shp_tensor * cache, const shp_tensor * src, int64_t filled
     return true;
 }
 
+// ---------------------------------------------------------------------------
+// A decoder layer's non-GEMM runs in one launch
+// ---------------------------------------------------------------------------
+
+// shp_layer_nongemm_step's five node runs (qwen3-tts/operations.cpp:84-147)
+// have the GEMM and attention outputs as inputs, so none of them waits for
+// another but the adds, which work row by row: one launch takes them all. Its
+// blocks have one of three jobs:
+//   - a row each: x, the attention output and the MLP output read once;
+//     rms(x)*w_in, x + attn, rms(x + attn)*w_post and (x + attn) + mlp written.
+//     The single launches read x twice and the sum once more (134 MB of 1.41 GB
+//     at [2048,8192]);
+//   - a position's (DEC: kLayerDecRows) q and k head rows through the QK-norm
+//     and rope, as k_rope128 and k_rope128_dec do;
+//   - 256 consecutive float4 of SwiGLU (512, two per lane: 205 us against 198 at
+//     [2048,8192], 10.4 against 9.8 at [1024,509]).
+// The arithmetic is the single kernels' (the double row sums in another order).
+// HBM-bound for a prefill, one kernel's latency for a decode step. Measured on
+// MI355X (cold) against the five launches: one token at 1024 8.7 -> 2.2 us, 64
+// 11.5 -> 3.3, 509 17.1 -> 9.8, 4000 70.7 -> 58.8; 8192 at 2048 219.9 -> 198 (6.45
+// TB/s, the copy 6.69).
+struct LayerArgs {
+    const float * x;
+    const float * attn;
+    const float * mlp;
+    float *       normed;
+    float *       resid;
+    float *       mlp_in;
+    float *       out;
+    int64_t       xs;  // row strides in bytes
+    int64_t       attns;
+    int64_t       mlps;
+    int64_t       normeds;
+    int64_t       resids;
+    int64_t       mlp_ins;
+    int64_t       outs;
+    const void *  w_in;
+    const void *  w_post;
+    const float * gate;
+    const float * up;
+    float *       act;
+    int64_t       act4;         // float4 of SwiGLU
+    RopeArgs      rope;
+    uint32_t      rope_first;   // first block of the rope job
+    uint32_t      swiglu_first;
+    int32_t       ne0;
+    int32_t       chunks;       // DEC: blocks per position
+    float         eps;
+    int32_t       pad;
+};
+
+constexpr int kLayerBlock   = 256;
+constexpr int kLayerDecRows = (kLayerBlock - kWave) / kRopeLanes;  // head rows per block beside the theta wave
+constexpr int kLayerPasses  = 2;                                   // head rows per 16-lane group otherwise
+constexpr int kLayerMaxRows = kLayerPasses * kLayerBlock / kRopeLanes;
+
+template <int WT, int VPL> __device__ __forceinline__ void layer_row(const LayerArgs & a, int64_t row, double (&part)[2][4]) {
+    args_in_sgprs(a.x, a.attn, a.mlp, a.w_in, a.w_post, a.xs, a.attns, a.mlps, a.ne0);
+    const int     l    = static_cast<int>(threadIdx.x);
+    const int     nvec = a.ne0 / 4;
+    const f32x4 * xp   = reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(a.x) + row * a.xs);
+    const f32x4 * ap   = reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(a.attn) + row * a.attns);
+    const f32x4 * mp   = reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(a.mlp) + row * a.mlps);
+    f32x4         v[VPL], r[VPL], m[VPL];
+    WRaw<WT>      wi[VPL], wp[VPL];
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        const int c = k * kLayerBlock + l;
+        v[k]        = c < nvec ? ld_stream(xp + c) : splat4(0.0f);
+        r[k]        = c < nvec ? ld_stream(ap + c) : splat4(0.0f);
+        m[k]        = c < nvec ? ld_stream(mp + c) : splat4(0.0f);
+    }
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        const int c = k * kLayerBlock + l;
+        wi[k]       = WRaw<WT>{};
+        wp[k]       = WRaw<WT>{};
+        if (c < nvec) {
+            wi[k] = load_wraw<WT>(a.w_in, static_cast<int64_t>(c) * 4);
+            wp[k] = load_wraw<WT>(a.w_post, static_cast<int64_t>(c) * 4);
+        }
+    }
+    f32x4 * rp = reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(a.resid) + row * a.resids);
+    f32x4 * op = reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(a.out) + row * a.outs);
+    double  accx = 0.0, accr = 0.0;
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        const int c = k * kLayerBlock + l;
+        r[k]        = add4v(v[k], r[k]);
+        accx += sq4v(v[k]);
+        accr += sq4v(r[k]);
+        if (c < nvec) {
+            st_stream(rp + c, r[k]);
+            st_stream(op + c, add4v(r[k], m[k]));
+        }
+    }
+    accx           = group_sum<kWave>(accx);
+    accr           = group_sum<kWave>(accr);
+    const int wave = l / kWave;
+    if (l % kWave == 0) {
+        part[0][wave] = accx;
+        part[1][wave] = accr;
+    }
+    __syncthreads();
+    accx            = part[0][0] + part[0][1] + part[0][2] + part[0][3];
+    accr            = part[1][0] + part[1][1] + part[1][2] + part[1][3];
+    const float sx  = norm_scale(accx, a.ne0, a.eps);
+    const float sr  = norm_scale(accr, a.ne0, a.eps);
+    f32x4 *     np  = reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(a.normed) + row * a.normeds);
+    f32x4 *     ip  = reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(a.mlp_in) + row * a.mlp_ins);
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+        const int c = k * kLayerBlock + l;
+        if (c < nvec) {
+            const f32x4 w0 = cvt_wraw<WT>(wi[k]), w1 = cvt_wraw<WT>(wp[k]);
+            st_stream(np + c, f32x4{ v[k].x * sx * w0.x, v[k].y * sx * w0.y, v[k].z * sx * w0.z, v[k].w * sx * w0.w });
+            st_stream(ip + c, f32x4{ r[k].x * sr * w1.x, r[k].y * sr * w1.y, r[k].z * sr * w1.z, r[k].w * sr * w1.w });
+        }
+    }
+}
+
+// Head rows r0 + g, r0 + g + groups, ... (PASSES of them) of position pi in
+// the block's 16-lane groups; wave 0 builds the position's cos/sin cache
+// (THETA: and holds no rows).
+template <int WT, int PASSES, bool THETA>
+__device__ __forceinline__ void layer_rope(const RopeArgs & a, int64_t pi, int r0, f32x4 (&s_cos)[16], f32x4 (&s_sin)[16]) {
+    const int32_t    p      = a.pos[pi];
+    const RopeFields f      = rope_fields<false>(a);
+    const int        total  = rope_rows<false>(f);
+    const int        tid    = static_cast<int>(threadIdx.x) - (THETA ? kWave : 0);
+    constexpr int    groups = (kLayerBlock - (THETA ? kWave : 0)) / kRopeLanes;
+    const int        l      = static_cast<int>(threadIdx.x) % kRopeLanes;
+    const int        g      = r0 + (tid < 0 ? 0 : tid / kRopeLanes);
+    float *          y[PASSES];
+    bool             live[PASSES];
+    f32x4            lo[PASSES], hi[PASSES];
+    WRaw<WT>         wlo[PASSES], whi[PASSES];
+#pragma unroll
+    for (int k = 0; k < PASSES; ++k) {
+        live[k]        = (tid >= 0) & (g + k * groups < total);
+        const RowRef r = rope_row<false>(f, live[k] ? g + k * groups : 0, pi);
+        y[k]           = r.y;
+        lo[k]          = splat4(0.0f);
+        hi[k]          = splat4(0.0f);
+        wlo[k]         = WRaw<WT>{};
+        whi[k]         = WRaw<WT>{};
+        if (live[k]) {
+            lo[k]  = ld_stream(to_global(reinterpret_cast<const f32x4 *>(r.x)) + l);
+            hi[k]  = ld_stream(to_global(reinterpret_cast<const f32x4 *>(r.x + 64)) + l);
+            wlo[k] = load_wraw<WT>(r.w, 4 * l);
+            whi[k] = load_wraw<WT>(r.w, 64 + 4 * l);
+        }
+    }
+    if (threadIdx.x < kWave) {
+        const float mth = theta_chain64(static_cast<float>(p), a.theta_scale);
+        float       sv, cv;
+        rope_sincos(a.freq_scale * mth, sv, cv);
+        reinterpret_cast<float *>(s_cos)[threadIdx.x] = cv * a.attn_factor;
+        reinterpret_cast<float *>(s_sin)[threadIdx.x] = sv * a.attn_factor;
+    }
+    if constexpr (!THETA) {
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < PASSES; ++k) {
+        const double acc   = group_sum<kRopeLanes>(sq4v(lo[k]) + sq4v(hi[k]));
+        const float  scale = norm_scale(acc, 128, a.eps);
+        const f32x4  w0 = cvt_wraw<WT>(wlo[k]), w1 = cvt_wraw<WT>(whi[k]);
+        lo[k] = f32x4{ lo[k].x * scale * w0.x, lo[k].y * scale * w0.y, lo[k].z * scale * w0.z, lo[k].w * scale * w0.w };
+        hi[k] = f32x4{ hi[k].x * scale * w1.x, hi[k].y * scale * w1.y, hi[k].z * scale * w1.z, hi[k].w * scale * w1.w };
+    }
+    if constexpr (THETA) {
+        __syncthreads();
+    }
+    const f32x4 cs = s_cos[l], sn = s_sin[l];
+#pragma unroll
+    for (int k = 0; k < PASSES; ++k) {
+        if (live[k]) {
+            st_stream(to_global(reinterpret_cast<f32x4 *>(y[k])) + l,
+                      f32x4{ lo[k].x * cs.x - hi[k].x * sn.x, lo[k].y * cs.y - hi[k].y * sn.y,
+                             lo[k].z * cs.z - hi[k].z * sn.z, lo[k].w * cs.w - hi[k].w * sn.w });
+            st_stream(to_global(reinterpret_cast<f32x4 *>(y[k] + 64)) + l,
+                      f32x4{ lo[k].x * sn.x + hi[k].x * cs.x, lo[k].y * sn.y + hi[k].y * cs.y,
+                             lo[k].z * sn.z + hi[k].z * cs.z, lo[k].w * sn.w + hi[k].w * cs.w });
+        }
+    }
+}
+
+template <int WT, int VPL, bool DEC> __global__ __launch_bounds__(kLayerBlock) void k_layer_step(const LayerArgs a) {
+    __shared__ double s_part[2][4];
+    __shared__ f32x4  s_cos[16], s_sin[16];
+    const uint32_t    b = blockIdx.x;
+    if (b < a.rope_first) {
+        layer_row<WT, VPL>(a, b, s_part);
+    } else if (b < a.swiglu_first) {
+        const uint32_t j = b - a.rope_first;
+        if constexpr (DEC) {
+            const uint32_t pi = j / static_cast<uint32_t>(a.chunks);
+            layer_rope<WT, 1, true>(a.rope, pi, static_cast<int>(j - pi * a.chunks) * kLayerDecRows, s_cos, s_sin);
+        } else {
+            layer_rope<WT, kLayerPasses, false>(a.rope, j, 0, s_cos, s_sin);
+        }
+    } else {
+        args_in_sgprs(a.gate, a.up, a.act, a.act4);
+        const int64_t i = static_cast<int64_t>(b - a.swiglu_first) * kLayerBlock + threadIdx.x;
+        if (i < a.act4) {
+            const f32x4 g = ld_stream4u(a.gate + i * 4), u = ld_stream4u(a.up + i * 4);
+            st_stream4u(a.act + i * 4, f32x4{ silu(g.x) * u.x, silu(g.y) * u.y, silu(g.z) * u.z, silu(g.w) * u.w });
+        }
+    }
+}
+
+template <int WT> shp_status_t launch_layer(const LayerArgs & a, bool dec, int64_t blocks, hipStream_t stream) {
+    const int nvec = a.ne0 / 4;
+    auto      go   = [&](auto dk, auto bk) {
+        hipLaunchKernelGGL(dec ? dk : bk, dim3(static_cast<unsigned>(blocks)), dim3(kLayerBlock), 0, stream, a);
+        return launch_status();
+    };
+    if (nvec <= kLayerBlock) {
+        return go(k_layer_step<WT, 1, true>, k_layer_step<WT, 1, false>);
+    }
+    if (nvec <= 2 * kLayerBlock) {
+        return go(k_layer_step<WT, 2, true>, k_layer_step<WT, 2, false>);
+    }
+    return go(k_layer_step<WT, 4, true>, k_layer_step<WT, 4, false>);
+}
+
 }  // namespace
+
+// The one launch takes F32 steps of the 128-wide rope with up to 32 head rows
+// a position, rows of up to 4096 whole, aligned float4-wise values, one gain
+// type, and outputs that overlap nothing: the five launches allow an output
+// over an input that a later one no longer reads, or over another's output.
+shp_status_t layer_step_launch(const shp_layer_step & s, hipStream_t stream, bool & taken) {
+    taken = false;
+    if (dry_run()) {
+        return SHP_OK;
+    }
+    RopePlan plan;
+    if (plan_rope(s.q, s.k, nullptr, s.wq, s.wk, true, s.eps, s.pos, s.n_dims, s.freq_base, 1.0f, 1.0f, s.q_out, s.k_out,
+                  nullptr, nullptr, nullptr, 0, plan) != SHP_OK || !plan.fast) {
+        return SHP_OK;
+    }
+    const int64_t t = s.x->ne[1], rows = s.q->ne[1] + s.k->ne[1], ne0 = s.x->ne[0];
+    if (rows > kLayerMaxRows || ne0 % 4 != 0 || ne0 > 4 * 4 * kLayerBlock || s.gate->ne[0] % 4 != 0 ||
+        s.w_in->type != s.wq->type || s.w_post->type != s.wq->type || !gain_aligned(s.w_in) || !gain_aligned(s.w_post) ||
+        !contiguous(*s.gate) || !contiguous(*s.up) || !contiguous(*s.act)) {
+        return SHP_OK;
+    }
+    const shp_tensor * const ins[]  = { s.x, s.attn_out, s.mlp_out, s.q, s.k, s.gate, s.up, s.w_in, s.w_post, s.wq, s.wk, s.pos };
+    const shp_tensor * const outs[] = { s.normed, s.resid, s.mlp_in, s.out, s.q_out, s.k_out, s.act };
+    for (const shp_tensor * r : { s.x, s.attn_out, s.mlp_out, outs[0], outs[1], outs[2], outs[3] }) {
+        if (!rows_aligned(*r, 16)) {
+            return SHP_OK;
+        }
+    }
+    for (size_t i = 0; i < sizeof(outs) / sizeof(outs[0]); ++i) {
+        for (const shp_tensor * in : ins) {
+            if (spans_overlap(*outs[i], *in)) {
+                return SHP_OK;
+            }
+        }
+        for (size_t j = 0; j < i; ++j) {
+            if (spans_overlap(*outs[i], *outs[j])) {
+                return SHP_OK;
+            }
+        }
+    }
+    LayerArgs a{};
+    a.x            = static_cast<const float *>(s.x->data);
+    a.attn         = static_cast<const float *>(s.attn_out->data);
+    a.mlp          = static_cast<const float *>(s.mlp_out->data);
+    a.normed       = static_cast<float *>(s.normed->data);
+    a.resid        = static_cast<float *>(s.resid->data);
+    a.mlp_in       = static_cast<float *>(s.mlp_in->data);
+    a.out          = static_cast<float *>(s.out->data);
+    a.xs           = static_cast<int64_t>(s.x->nb[1]);
+    a.attns        = static_cast<int64_t>(s.attn_out->nb[1]);
+    a.mlps         = static_cast<int64_t>(s.mlp_out->nb[1]);
+    a.normeds      = static_cast<int64_t>(s.normed->nb[1]);
+    a.resids       = static_cast<int64_t>(s.resid->nb[1]);
+    a.mlp_ins      = static_cast<int64_t>(s.mlp_in->nb[1]);
+    a.outs         = static_cast<int64_t>(s.out->nb[1]);
+    a.w_in         = s.w_in->data;
+    a.w_post       = s.w_post->data;
+    a.gate         = static_cast<const float *>(s.gate->data);
+    a.up           = static_cast<const float *>(s.up->data);
+    a.act          = static_cast<float *>(s.act->data);
+    a.act4         = nelements(*s.act) / 4;
+    a.rope         = plan.args;
+    a.ne0          = static_cast<int32_t>(ne0);
+    a.eps          = s.eps;
+    const bool dec = t <= kRopeDecMaxPos;
+    a.chunks       = static_cast<int32_t>((rows + kLayerDecRows - 1) / kLayerDecRows);
+    const int64_t rope = dec ? t * a.chunks : t, act = (a.act4 + kLayerBlock - 1) / kLayerBlock;
+    if (t + rope + act > INT32_MAX) {
+        return SHP_OK;
+    }
+    a.rope_first   = static_cast<uint32_t>(t);
+    a.swiglu_first = static_cast<uint32_t>(t + rope);
+    taken          = true;
+    switch (plan.wkind) {
+        case kWBF16:
+            return launch_layer<kWBF16>(a, dec, t + rope + act, stream);
+        case kWF16:
+            return launch_layer<kWF16>(a, dec, t + rope + act, stream);
+        default:
+            return launch_layer<kWF32>(a, dec, t + rope + act, stream);
+    }
+}
+
 }  // namespace shp
 
 extern "C" shp_status_t shp_norm(const shp_tensor * x, float eps, shp_tensor * y, shp_stream_t stream) {

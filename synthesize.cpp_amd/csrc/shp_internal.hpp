@@ -241,6 +241,11 @@ template <int WT> __device__ __forceinline__ float2 load_w2(const void * w, int6
     }
 }
 
+// ggml_silu.
+__device__ __forceinline__ float silu(float x) {
+    return x / (1.0f + expf(-x));
+}
+
 // Cross-lane moves inside a row of 16 lanes (DPP), no LDS round trip. Each
 // pattern pairs lanes symmetrically, so `v op move(v)` gives both lanes of a
 // pair the same two operands in swapped order: with a commutative op every
@@ -551,5 +556,9 @@ inline hipStream_t as_stream(shp_stream_t s) {
 inline shp_status_t launch_status() {
     return hipGetLastError() == hipSuccess ? SHP_OK : SHP_ERR_BACKEND;
 }
+
+// A checked layer step in one launch (k_norm.hip). `taken` is false when the
+// step's layouts are not that launch's: nothing was enqueued then.
+shp_status_t layer_step_launch(const shp_layer_step & s, hipStream_t stream, bool & taken);
 
 }  // namespace shp

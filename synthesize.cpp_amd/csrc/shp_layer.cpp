@@ -2,10 +2,9 @@
 // (src/arch/qwen3-tts/operations.cpp:84-147) enqueued in the layer's order on
 // one stream, after every tensor of the step has been checked.
 //
-// The five launches are the ones the single entry points make; the value of
-// this entry point is the contract (one call per layer, with the GEMM and
-// attention outputs as inputs, and no partial enqueue on a malformed step),
-// not a different kernel.
+// With the GEMM and attention outputs as inputs, the step is one launch where
+// its layouts allow (layer_step_launch, k_norm.hip); otherwise the five launches
+// of the single entry points, in the layer's order.
 #include <cstdint>
 
 #include "shp_internal.hpp"
@@ -89,6 +88,11 @@ extern "C" shp_status_t shp_layer_nongemm_step(const shp_layer_step * step, shp_
     const shp_layer_step & s  = *step;
     shp_status_t           st = shp::check_step(s);
     if (st != SHP_OK) {
+        return st;
+    }
+    bool taken = false;
+    st         = shp::layer_step_launch(s, shp::as_stream(stream), taken);
+    if (taken) {
         return st;
     }
     // operations.cpp:85-86, the input norm.
