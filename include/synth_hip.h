@@ -609,9 +609,11 @@ shp_status_t shp_cont_add_leaky_relu(const shp_tensor * x,
  *   mlp_in       = rms_norm(resid)*w_post                  (:145)
  *   act          = silu(gate)*up                           (:39-41 via :146)
  *   out          = resid + mlp_out                         (:147)
- * Five launches on `stream`, each the launch of shp_rms_norm_mul,
- * shp_qk_norm_rope, shp_add_rms_norm_mul, shp_swiglu and shp_add, with the
- * same results. Every tensor's presence, type and shape is checked first:
+ * One launch on `stream` where no output overlaps an input or another output
+ * and the layouts are the 128-wide rope's and whole aligned float4 rows of up
+ * to 4096 values; otherwise five, each the launch of shp_rms_norm_mul,
+ * shp_qk_norm_rope, shp_add_rms_norm_mul, shp_swiglu and shp_add, in this
+ * order. The same results either way. Every tensor's presence, type and shape is checked first:
  * a malformed step returns SHP_ERR_INVALID_ARG with nothing enqueued.
  * x, normed, attn_out, resid, mlp_in, mlp_out, out: F32 [hidden, T];
  * q, q_out: F32 [head_dim, q_heads, T]; k, k_out: F32 [head_dim, kv_heads, T];

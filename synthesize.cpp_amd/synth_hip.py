@@ -13,11 +13,15 @@ libamdhip64.so.7 and one process must run one HIP runtime.
 There is no CPU fallback: without the built library every call raises.
 """
 import ctypes
+import functools
+import importlib.machinery
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 # SHP_LIB selects another build of the library (the sanitized one of `make asan`).
 LIB_PATH = os.environ.get("SHP_LIB") or os.path.join(HERE, "libsynth_hip.so")
+BIND_PATH = os.path.join(HERE, "shp_bind.so")
 
 OK, ERR_INVALID_ARG, ERR_UNSUPPORTED, ERR_BACKEND = 0, 1, 2, 17
 TYPE_F32, TYPE_F16, TYPE_Q8_0, TYPE_Q5_K, TYPE_I32, TYPE_BF16 = 0, 1, 8, 13, 26, 30
@@ -191,52 +195,47 @@ class Q5KTensor(BlockTensor):
     TYPE, ELEMS, BYTES = TYPE_Q5_K, Q5_K_BLOCK_ELEMS, Q5_K_BLOCK_BYTES
 
 
-def _torch_type(t):
-    import torch
-    return {torch.float32: TYPE_F32, torch.float16: TYPE_F16, torch.bfloat16: TYPE_BF16,
-            torch.int32: TYPE_I32}[t.dtype]
+_bind = None
+
+
+def _binding():
+    """The native half of this binding (csrc/shp_bind.cpp), loaded once."""
+    global _bind
+    if _bind is None:
+        import torch  # noqa: F401  -- its libraries resolve the module's symbols
+        if not os.path.exists(BIND_PATH):
+            raise RuntimeError("shp_bind.so is not built (%s); run __graft_entry__.build() or make -C "
+                               "synthesize.cpp_amd" % BIND_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("shp_bind", BIND_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("shp_bind", BIND_PATH,
+                                                                                    loader=loader))
+        loader.exec_module(mod)
+        _bind = mod
+    return _bind
 
 
 def desc(t):
     """shp_tensor for a torch tensor (or BlockTensor); None stays None."""
-    if t is None:
-        return None
-    d = ShpTensor()
-    if isinstance(t, BlockTensor):
-        raw = t.data
-        shape = list(raw.shape[::-1])
-        strides = list(raw.stride()[::-1])
-        d.type = t.TYPE
-        shape[0] = t.ne0
-        strides[0] = t.BYTES
-        item = 1
-    else:
-        shape = list(t.shape[::-1]) or [1]
-        strides = list(t.stride()[::-1]) or [1]
-        d.type = _torch_type(t)
-        item = t.element_size()
-        strides = [s * item for s in strides]
-        raw = t
-    if len(shape) > 4:
-        raise ValueError("at most 4 dimensions")
-    while len(shape) < 4:
-        strides.append(strides[-1] * shape[-1] if item else 0)
-        shape.append(1)
-    d.reserved = 0
-    for k in range(4):
-        d.ne[k] = int(shape[k])
-        d.nb[k] = int(strides[k])
-    d.data = raw.data_ptr()
-    return d
+    return None if t is None else ShpTensor.from_buffer_copy(_binding().describe(t))
 
 
-def _ref(d):
-    return ctypes.byref(d) if d is not None else None
+_fns = {}
+
+
+def _fn(name):
+    """The entry point `name` as a callable over torch tensors (csrc/shp_bind.cpp)."""
+    f = _fns.get(name)
+    if f is None:
+        f = _fns[name] = _binding().bind(load()._handle, name)
+    return f
 
 
 def _stream():
+    """The address of torch's current stream on the current device."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _check(status, what):
@@ -260,7 +259,7 @@ def get_rows(src, ids, out=None):
     ne0 = src.ne0 if isinstance(src, BlockTensor) else src.shape[-1]
     if out is None:
         out = _empty_like_f32(tuple(ids.shape) + (ne0,), raw.device)
-    _check(load().shp_get_rows(_ref(desc(src)), _ref(desc(ids)), _ref(desc(out)), _stream()), "get_rows")
+    _check(_fn("shp_get_rows")(src, ids, out, _stream()), "get_rows")
     return out
 
 
@@ -268,20 +267,19 @@ def get_rows_sum(tables, codes, out=None):
     """sum_code_embeddings: codes int32 (groups, frames) (ggml [frames, groups]); tables
     one per group; returns f32 (frames, ne0) = ordered sum of the gathered rows."""
     n = len(tables)
-    arr = (ShpTensor * n)(*[desc(t) for t in tables])
     first = tables[0]
     ne0 = first.ne0 if isinstance(first, BlockTensor) else first.shape[-1]
     raw = first.data if isinstance(first, BlockTensor) else first
     if out is None:
         out = _empty_like_f32((codes.shape[-1], ne0), raw.device)
-    _check(load().shp_get_rows_sum(arr, n, _ref(desc(codes)), _ref(desc(out)), _stream()), "get_rows_sum")
+    _check(_fn("shp_get_rows_sum")(list(tables), n, codes, out, _stream()), "get_rows_sum")
     return out
 
 
 def rms_norm_mul(x, w, eps, out=None):
     """rms_norm() of src/arch/qwen3-tts/operations.cpp:27-32 (w None: bare ggml_rms_norm)."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_rms_norm_mul(_ref(desc(x)), _ref(desc(w)), float(eps), _ref(desc(out)), _stream()),
+    _check(_fn("shp_rms_norm_mul")(x, w, float(eps), out, _stream()),
            "rms_norm_mul")
     return out
 
@@ -291,16 +289,16 @@ def add_rms_norm_mul(a, b, w, eps, out=None, sum_out=None, want_sum=True):
     out = a.new_empty(a.shape) if out is None else out
     if sum_out is None and want_sum:
         sum_out = a.new_empty(a.shape)
-    _check(load().shp_add_rms_norm_mul(_ref(desc(a)), _ref(desc(b)), _ref(desc(w)), float(eps), _ref(desc(sum_out)),
-                                       _ref(desc(out)), _stream()), "add_rms_norm_mul")
+    _check(_fn("shp_add_rms_norm_mul")(a, b, w, float(eps), sum_out,
+                                       out, _stream()), "add_rms_norm_mul")
     return sum_out, out
 
 
 def rope_ext(x, pos, n_dims, mode, freq_base, freq_scale=1.0, ext_factor=0.0, attn_factor=1.0, out=None):
     """ggml_rope_ext on x (T, heads, head_dim) with I32 positions (T,)."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_rope_ext(_ref(desc(x)), _ref(desc(pos)), int(n_dims), int(mode), float(freq_base),
-                               float(freq_scale), float(ext_factor), float(attn_factor), _ref(desc(out)), _stream()),
+    _check(_fn("shp_rope_ext")(x, pos, int(n_dims), int(mode), float(freq_base),
+                               float(freq_scale), float(ext_factor), float(attn_factor), out, _stream()),
            "rope_ext")
     return out
 
@@ -310,9 +308,9 @@ def qk_norm_rope(q, k, wq, wk, eps, pos, n_dims, freq_base, freq_scale=1.0, q_ou
     q_out = q.new_empty(q.shape) if q_out is None else q_out
     if k is not None and k_out is None:
         k_out = k.new_empty(k.shape)
-    _check(load().shp_qk_norm_rope(_ref(desc(q)), _ref(desc(k)), _ref(desc(wq)), _ref(desc(wk)), float(eps),
-                                   _ref(desc(pos)), int(n_dims), float(freq_base), float(freq_scale),
-                                   _ref(desc(q_out)), _ref(desc(k_out)), _stream()), "qk_norm_rope")
+    _check(_fn("shp_qk_norm_rope")(q, k, wq, wk, float(eps),
+                                   pos, int(n_dims), float(freq_base), float(freq_scale),
+                                   q_out, k_out, _stream()), "qk_norm_rope")
     return q_out, k_out
 
 
@@ -322,9 +320,9 @@ def qk_norm_rope_kv(q, k, v, wq, wk, eps, pos, n_dims, freq_base, k_cache, v_cac
     [filled, filled + T) of k_cache / v_cache (T, ...) = torch (capacity, kv_heads,
     head_dim); returns q_out."""
     q_out = q.new_empty(q.shape) if q_out is None else q_out
-    _check(load().shp_qk_norm_rope_kv(_ref(desc(q)), _ref(desc(k)), _ref(desc(v)), _ref(desc(wq)), _ref(desc(wk)),
-                                      float(eps), _ref(desc(pos)), int(n_dims), float(freq_base), float(freq_scale),
-                                      _ref(desc(q_out)), _ref(desc(k_cache)), _ref(desc(v_cache)), int(filled),
+    _check(_fn("shp_qk_norm_rope_kv")(q, k, v, wq, wk,
+                                      float(eps), pos, int(n_dims), float(freq_base), float(freq_scale),
+                                      q_out, k_cache, v_cache, int(filled),
                                       _stream()), "qk_norm_rope_kv")
     return q_out
 
@@ -335,45 +333,45 @@ def qk_norm_rope_kv_at(q, k, v, wq, wk, eps, pos, n_dims, freq_base, k_cache, v_
     `slot` when the kernel runs (graph-replayable); `status` (int32, one element)
     is set to 1 when the rows do not fit the cache."""
     q_out = q.new_empty(q.shape) if q_out is None else q_out
-    _check(load().shp_qk_norm_rope_kv_at(_ref(desc(q)), _ref(desc(k)), _ref(desc(v)), _ref(desc(wq)), _ref(desc(wk)),
-                                         float(eps), _ref(desc(pos)), int(n_dims), float(freq_base), float(freq_scale),
-                                         _ref(desc(q_out)), _ref(desc(k_cache)), _ref(desc(v_cache)), _ref(desc(slot)),
-                                         _ref(desc(status)), _stream()), "qk_norm_rope_kv_at")
+    _check(_fn("shp_qk_norm_rope_kv_at")(q, k, v, wq, wk,
+                                         float(eps), pos, int(n_dims), float(freq_base), float(freq_scale),
+                                         q_out, k_cache, v_cache, slot,
+                                         status, _stream()), "qk_norm_rope_kv_at")
     return q_out
 
 
 def swiglu(g, u=None, out=None):
     """ggml_silu(g) then ggml_mul(., u) (u None: bare silu)."""
     out = g.new_empty(g.shape) if out is None else out
-    _check(load().shp_swiglu(_ref(desc(g)), _ref(desc(u)), _ref(desc(out)), _stream()), "swiglu")
+    _check(_fn("shp_swiglu")(g, u, out, _stream()), "swiglu")
     return out
 
 
 def glu_swiglu(a, swapped=False, out=None):
     """ggml_swiglu(a) / ggml_swiglu_swapped(a) on a (..., 2n) -> (..., n)."""
     out = a.new_empty(tuple(a.shape[:-1]) + (a.shape[-1] // 2,)) if out is None else out
-    _check(load().shp_glu_swiglu(_ref(desc(a)), 1 if swapped else 0, _ref(desc(out)), _stream()), "glu_swiglu")
+    _check(_fn("shp_glu_swiglu")(a, 1 if swapped else 0, out, _stream()), "glu_swiglu")
     return out
 
 
 def snake(x, alpha, out=None):
     """Kokoro Snake on x (T, C) (ggml [C, T], channels fastest), alpha (C,)."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_snake(_ref(desc(x)), _ref(desc(alpha)), _ref(desc(out)), _stream()), "snake")
+    _check(_fn("shp_snake")(x, alpha, out, _stream()), "snake")
     return out
 
 
 def snake_guarded(x, alpha, out=None):
     """codec_snake (omnivoice): x + sin(x*alpha)^2 / (alpha + 1e-9), x (T, C), alpha C values."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_snake_guarded(_ref(desc(x)), _ref(desc(alpha)), _ref(desc(out)), _stream()), "snake_guarded")
+    _check(_fn("shp_snake_guarded")(x, alpha, out, _stream()), "snake_guarded")
     return out
 
 
 def snake_beta(x, log_alpha, log_beta, out=None):
     """codec_snake_beta (qwen3-tts): x + sin(x*exp(la))^2 / (exp(lb) + 1e-9), x (T, C)."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_snake_beta(_ref(desc(x)), _ref(desc(log_alpha)), _ref(desc(log_beta)), _ref(desc(out)),
+    _check(_fn("shp_snake_beta")(x, log_alpha, log_beta, out,
                                  _stream()), "snake_beta")
     return out
 
@@ -382,7 +380,7 @@ def soft_max_ext(a, mask, scale, max_bias=0.0, out=None):
     """ggml_soft_max_ext over the last axis of a (..., ne1, ne0); mask None or
     (ne1', ne0) / (heads', ne1', ne0) broadcast as ggml does."""
     out = a.new_empty(a.shape) if out is None else out
-    _check(load().shp_soft_max_ext(_ref(desc(a)), _ref(desc(mask)), float(scale), float(max_bias), _ref(desc(out)),
+    _check(_fn("shp_soft_max_ext")(a, mask, float(scale), float(max_bias), out,
                                    _stream()), "soft_max_ext")
     return out
 
@@ -390,26 +388,25 @@ def soft_max_ext(a, mask, scale, max_bias=0.0, out=None):
 def exp(x, out=None):
     """ggml_exp."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_exp(_ref(desc(x)), _ref(desc(out)), _stream()), "exp")
+    _check(_fn("shp_exp")(x, out, _stream()), "exp")
     return out
 
 
 def scale_bias(x, s, b=0.0, out=None):
     """ggml_scale_bias(x, s, b); b == 0 is ggml_scale(x, s)."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_scale_bias(_ref(desc(x)), float(s), float(b), _ref(desc(out)), _stream()), "scale_bias")
+    _check(_fn("shp_scale_bias")(x, float(s), float(b), out, _stream()), "scale_bias")
     return out
 
 
 def sum_scale_leaky_relu(terms, scale, slope, out=None, mean_out=None, want_mean=False):
     """Branch average: leaky_relu((t0 + t1 + ...) * scale, slope); returns (mean or None, y)."""
     n = len(terms)
-    arr = (ShpTensor * n)(*[desc(t) for t in terms])
     out = terms[0].new_empty(terms[0].shape) if out is None else out
     if mean_out is None and want_mean:
         mean_out = terms[0].new_empty(terms[0].shape)
-    _check(load().shp_sum_scale_leaky_relu(arr, n, float(scale), float(slope), _ref(desc(mean_out)),
-                                           _ref(desc(out)), _stream()), "sum_scale_leaky_relu")
+    _check(_fn("shp_sum_scale_leaky_relu")(list(terms), n, float(scale), float(slope), mean_out,
+                                           out, _stream()), "sum_scale_leaky_relu")
     return mean_out, out
 
 
@@ -418,8 +415,8 @@ def add_leaky_relu(a, b, slope, out=None, sum_out=None, want_sum=False):
     out = a.new_empty(a.shape) if out is None else out
     if sum_out is None and want_sum:
         sum_out = a.new_empty(a.shape)
-    _check(load().shp_add_leaky_relu(_ref(desc(a)), _ref(desc(b)), float(slope), _ref(desc(sum_out)),
-                                     _ref(desc(out)), _stream()), "add_leaky_relu")
+    _check(_fn("shp_add_leaky_relu")(a, b, float(slope), sum_out,
+                                     out, _stream()), "add_leaky_relu")
     return sum_out, out
 
 
@@ -431,7 +428,7 @@ def add(a, b, out=None):
     """ggml_add(a, b), b of a's shape or any shape that repeats to it
     (ggml_can_repeat: each ggml extent of b divides a's)."""
     out = a.new_empty(a.shape) if out is None else out
-    _check(load().shp_add(_ref(desc(a)), _ref(desc(b)), _ref(desc(out)), _stream()), "add")
+    _check(_fn("shp_add")(a, b, out, _stream()), "add")
     return out
 
 
@@ -450,42 +447,39 @@ def layer_nongemm_step(x, w_in, q, k, wq, wk, pos, attn_out, w_post, gate, up, m
     for name in LAYER_OUTPUTS:
         if outs.get(name) is None:
             outs[name] = like[name].new_empty(like[name].shape)
-    ins = dict(x=x, w_in=w_in, q=q, k=k, wq=wq, wk=wk, pos=pos, attn_out=attn_out, w_post=w_post, gate=gate, up=up,
-               mlp_out=mlp_out)
-    descs = {n: desc(t) for n, t in list(ins.items()) + list(outs.items())}
-    step = ShpLayerStep()
-    for n, d in descs.items():
-        setattr(step, n, ctypes.pointer(d) if d is not None else None)
-    step.eps, step.freq_base, step.n_dims, step.reserved = float(eps), float(freq_base), int(n_dims), 0
-    _check(load().shp_layer_nongemm_step(ctypes.byref(step), _stream()), "layer_nongemm_step")
+    _check(_fn("shp_layer_nongemm_step")(x, w_in, outs["normed"], q, k, wq, wk, pos, outs["q_out"], outs["k_out"],
+                                         attn_out, w_post, outs["resid"], outs["mlp_in"], gate, up, outs["act"],
+                                         mlp_out, outs["out"], float(eps), float(freq_base), int(n_dims),
+                                         _stream()),
+           "layer_nongemm_step")
     return outs
 
 
 def mul(a, b, out=None):
     """ggml_mul(a, b), b as in add."""
     out = a.new_empty(a.shape) if out is None else out
-    _check(load().shp_mul(_ref(desc(a)), _ref(desc(b)), _ref(desc(out)), _stream()), "mul")
+    _check(_fn("shp_mul")(a, b, out, _stream()), "mul")
     return out
 
 
 def div(a, b, out=None):
     """ggml_div(a, b), b as in add."""
     out = a.new_empty(a.shape) if out is None else out
-    _check(load().shp_div(_ref(desc(a)), _ref(desc(b)), _ref(desc(out)), _stream()), "div")
+    _check(_fn("shp_div")(a, b, out, _stream()), "div")
     return out
 
 
 def sin(x, out=None):
     """ggml_sin."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_sin(_ref(desc(x)), _ref(desc(out)), _stream()), "sin")
+    _check(_fn("shp_sin")(x, out, _stream()), "sin")
     return out
 
 
 def sqr(x, out=None):
     """ggml_sqr."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_sqr(_ref(desc(x)), _ref(desc(out)), _stream()), "sqr")
+    _check(_fn("shp_sqr")(x, out, _stream()), "sqr")
     return out
 
 
@@ -496,8 +490,8 @@ def cont_add_leaky_relu(x, b, r=None, slope=None, out=None, sum_out=None):
     import torch
     out = torch.empty(x.shape, dtype=torch.float32, device=x.device) if out is None else out
     leaky = slope is not None
-    _check(load().shp_cont_add_leaky_relu(_ref(desc(x)), _ref(desc(b)), _ref(desc(r)), int(leaky),
-                                          float(slope if leaky else 0.0), _ref(desc(sum_out)), _ref(desc(out)),
+    _check(_fn("shp_cont_add_leaky_relu")(x, b, r, int(leaky),
+                                          float(slope if leaky else 0.0), sum_out, out,
                                           _stream()), "cont_add_leaky_relu")
     return out
 
@@ -505,13 +499,13 @@ def cont_add_leaky_relu(x, b, r=None, slope=None, out=None, sum_out=None):
 def sub(a, b, out=None):
     """ggml_sub(a, b), b as in add."""
     out = a.new_empty(a.shape) if out is None else out
-    _check(load().shp_sub(_ref(desc(a)), _ref(desc(b)), _ref(desc(out)), _stream()), "sub")
+    _check(_fn("shp_sub")(a, b, out, _stream()), "sub")
     return out
 
 
 def _unary_call(name, x, out):
     out = x.new_empty(x.shape) if out is None else out
-    _check(getattr(load(), "shp_" + name)(_ref(desc(x)), _ref(desc(out)), _stream()), name)
+    _check(_fn("shp_" + name)(x, out, _stream()), name)
     return out
 
 
@@ -558,8 +552,8 @@ def sqrt(x, out=None):
 def _row_sums(name, x, w, out):
     import torch
     out = torch.empty(tuple(x.shape[:-1]) + (1,), dtype=torch.float32, device=x.device) if out is None else out
-    args = [_ref(desc(x))] + ([_ref(desc(w))] if w is not None else []) + [_ref(desc(out)), _stream()]
-    _check(getattr(load(), "shp_" + name)(*args), name)
+    args = (x, out, _stream()) if w is None else (x, w, out, _stream())
+    _check(_fn("shp_" + name)(*args), name)
     return out
 
 
@@ -581,14 +575,14 @@ def mul_sum_rows(x, w, out=None):
 def diag_mask_inf(x, n_past, out=None):
     """ggml_diag_mask_inf(x, n_past); out=x for the inplace form."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_diag_mask_inf(_ref(desc(x)), int(n_past), _ref(desc(out)), _stream()), "diag_mask_inf")
+    _check(_fn("shp_diag_mask_inf")(x, int(n_past), out, _stream()), "diag_mask_inf")
     return out
 
 
 def soft_max_causal(x, n_past, scale, out=None):
     """ggml_diag_mask_inf(x, n_past) then ggml_soft_max_ext(., NULL, scale, 0), one launch."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_soft_max_causal(_ref(desc(x)), int(n_past), float(scale), _ref(desc(out)), _stream()),
+    _check(_fn("shp_soft_max_causal")(x, int(n_past), float(scale), out, _stream()),
            "soft_max_causal")
     return out
 
@@ -598,7 +592,7 @@ def inverse_stft(spectrum, n_fft, hop, out=None):
     import torch
     frames = spectrum.shape[0]
     out = torch.empty(((frames - 1) * hop,), dtype=torch.float32, device=spectrum.device) if out is None else out
-    _check(load().shp_inverse_stft(_ref(desc(spectrum)), int(n_fft), int(hop), _ref(desc(out)), _stream()),
+    _check(_fn("shp_inverse_stft")(spectrum, int(n_fft), int(hop), out, _stream()),
            "inverse_stft")
     return out
 
@@ -614,9 +608,9 @@ def harmonic_source(f0, merge_weight, merge_bias, rand_ini, noise, *, rate, scal
         out = (torch.empty((U,), dtype=torch.float32, device=f0.device),
                torch.empty((frames, n_fft + 2), dtype=torch.float32, device=f0.device))
     exc, har = out
-    _check(load().shp_harmonic_source(_ref(desc(f0)), _ref(desc(merge_weight)), float(merge_bias), _ref(desc(rand_ini)),
-                                      _ref(desc(noise)), int(rate), int(scale), float(sine_amp), float(noise_std),
-                                      float(voiced_threshold), int(n_fft), int(hop), _ref(desc(exc)), _ref(desc(har)),
+    _check(_fn("shp_harmonic_source")(f0, merge_weight, float(merge_bias), rand_ini,
+                                      noise, int(rate), int(scale), float(sine_amp), float(noise_std),
+                                      float(voiced_threshold), int(n_fft), int(hop), exc, har,
                                       _stream()), "harmonic_source")
     return exc, har
 
@@ -638,22 +632,22 @@ def log_mel(pcm, filterbank, n_fft, hop, win_length, out=None):
     frames = 1 + (pcm.numel() + 2 * pad - n_fft) // hop
     out = torch.empty((max(frames, 1), filterbank.shape[0]), dtype=torch.float32, device=pcm.device) if out is None \
         else out
-    _check(load().shp_log_mel(_ref(desc(pcm)), _ref(desc(filterbank)), int(n_fft), int(hop), int(win_length),
-                              _ref(desc(out)), _stream()), "log_mel")
+    _check(_fn("shp_log_mel")(pcm, filterbank, int(n_fft), int(hop), int(win_length),
+                              out, _stream()), "log_mel")
     return out
 
 
 def clamp(x, lo, hi, out=None):
     """ggml_clamp(x, lo, hi)."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_clamp(_ref(desc(x)), float(lo), float(hi), _ref(desc(out)), _stream()), "clamp")
+    _check(_fn("shp_clamp")(x, float(lo), float(hi), out, _stream()), "clamp")
     return out
 
 
 def norm(x, eps, out=None):
     """ggml_norm(x, eps)."""
     out = x.new_empty(x.shape) if out is None else out
-    _check(load().shp_norm(_ref(desc(x)), float(eps), _ref(desc(out)), _stream()), "norm")
+    _check(_fn("shp_norm")(x, float(eps), out, _stream()), "norm")
     return out
 
 
@@ -664,7 +658,7 @@ def concat(a, b, dim, out=None):
     shape = list(a.shape)
     shape[ax] += b.shape[ax]
     out = torch.empty(shape, dtype=torch.float32, device=a.device) if out is None else out
-    _check(load().shp_concat(_ref(desc(a)), _ref(desc(b)), int(dim), _ref(desc(out)), _stream()), "concat")
+    _check(_fn("shp_concat")(a, b, int(dim), out, _stream()), "concat")
     return out
 
 
@@ -687,6 +681,9 @@ def kernel_shape(k, ic, oc=1):
     return d
 
 
+_kernel_shape = functools.lru_cache(maxsize=64)(kernel_shape)
+
+
 def im2col(x, k, s0=1, p0=0, d0=1, dtype=None, out=None):
     """ggml_im2col(kernel [k, IC], x, s0, 0, p0, 0, d0, 0, false, dtype): x a
     torch F32 tensor (N, IC, IW) or (IC, IW) = ggml [IW, IC, N], any strides;
@@ -697,8 +694,8 @@ def im2col(x, k, s0=1, p0=0, d0=1, dtype=None, out=None):
         ow = conv_out_len(iw, k, s0, p0, d0)
         out = torch.empty((n_, max(ow, 1), ic * k), dtype=dtype or torch.float32, device=x.device)
     ic = x.shape[-2]
-    _check(load().shp_im2col(ctypes.byref(kernel_shape(k, ic)), _ref(desc(x)), int(s0), int(p0), int(d0),
-                             _ref(desc(out)), _stream()), "im2col")
+    _check(_fn("shp_im2col")(_kernel_shape(int(k), int(ic)), x, int(s0), int(p0), int(d0),
+                             out, _stream()), "im2col")
     return out
 
 
@@ -709,7 +706,7 @@ def col2im_1d(cols, stride, out_channels, padding=0, out=None):
     L, ko = cols.shape
     t = (L - 1) * stride + ko // out_channels - 2 * padding
     out = torch.empty((out_channels, max(t, 1)), dtype=torch.float32, device=cols.device) if out is None else out
-    _check(load().shp_col2im_1d(_ref(desc(cols)), int(stride), int(out_channels), int(padding), _ref(desc(out)),
+    _check(_fn("shp_col2im_1d")(cols, int(stride), int(out_channels), int(padding), out,
                                 _stream()), "col2im_1d")
     return out
 
@@ -723,7 +720,7 @@ def pad_ext(x, lp, rp, out=None):
         ne = list(x.shape[::-1]) + [1] * (4 - x.dim())
         nd = max(x.dim(), max([d + 1 for d in range(4) if lp[d] or rp[d]] + [1]))
         out = torch.empty([ne[d] + lp[d] + rp[d] for d in range(nd)][::-1], dtype=torch.float32, device=x.device)
-    _check(load().shp_pad(_ref(desc(x)), (ctypes.c_int32 * 4)(*lp), _ref(desc(out)), _stream()), "pad")
+    _check(_fn("shp_pad")(x, lp, out, _stream()), "pad")
     return out
 
 
@@ -732,7 +729,7 @@ def pad_reflect_1d(x, p0, p1, out=None):
     import torch
     out = torch.empty(tuple(x.shape[:-1]) + (x.shape[-1] + p0 + p1,), dtype=torch.float32,
                       device=x.device) if out is None else out
-    _check(load().shp_pad_reflect_1d(_ref(desc(x)), int(p0), int(p1), _ref(desc(out)), _stream()), "pad_reflect_1d")
+    _check(_fn("shp_pad_reflect_1d")(x, int(p0), int(p1), out, _stream()), "pad_reflect_1d")
     return out
 
 
@@ -740,7 +737,7 @@ def repeat(x, shape, out=None):
     """ggml_repeat(x, a tensor of torch shape `shape`)."""
     import torch
     out = torch.empty(tuple(shape), dtype=torch.float32, device=x.device) if out is None else out
-    _check(load().shp_repeat(_ref(desc(x)), _ref(desc(out)), _stream()), "repeat")
+    _check(_fn("shp_repeat")(x, out, _stream()), "repeat")
     return out
 
 
@@ -753,7 +750,7 @@ def acc(a, b, nb1, nb2, nb3, offset, out=None, inplace=False):
         out = a
     elif out is None:
         out = torch.empty(a.shape, dtype=torch.float32, device=a.device)
-    _check(load().shp_acc(_ref(desc(a)), _ref(desc(b)), int(nb1), int(nb2), int(nb3), int(offset), _ref(desc(out)),
+    _check(_fn("shp_acc")(a, b, int(nb1), int(nb2), int(nb3), int(offset), out,
                           _stream()), "acc")
     return out
 
@@ -762,7 +759,7 @@ def cpy(x, out=None):
     """ggml_cpy / ggml_cast into F32 of x's shape (x F32, F16 or BF16)."""
     import torch
     out = torch.empty(x.shape, dtype=torch.float32, device=x.device) if out is None else out
-    _check(load().shp_cpy(_ref(desc(x)), _ref(desc(out)), _stream()), "cpy")
+    _check(_fn("shp_cpy")(x, out, _stream()), "cpy")
     return out
 
 

@@ -1,0 +1,77 @@
+"""The binding's native half (csrc/shp_bind.cpp) on host tensors: descriptors
+of every type, rank and stride against the rule written out here, what it
+refuses, and the conversion of call arguments through entry points that refuse
+their arguments before touching a device."""
+import ctypes
+
+import pytest
+import torch
+
+import synth_hip as S
+
+
+def _rule(t):
+    """ne, nb of a tensor: its extents and byte strides innermost first, a
+    scalar one element, then extents of 1 at the stride of all below."""
+    item = t.element_size()
+    ne, nb = list(t.shape[::-1]) or [1], [s * item for s in t.stride()[::-1]] or [item]
+    while len(ne) < 4:
+        nb.append(nb[-1] * ne[-1])
+        ne.append(1)
+    return ne, nb
+
+
+@pytest.mark.parametrize("dtype,type_", [(torch.float32, S.TYPE_F32), (torch.float16, S.TYPE_F16),
+                                         (torch.bfloat16, S.TYPE_BF16), (torch.int32, S.TYPE_I32)])
+def test_descriptors(dtype, type_):
+    base = torch.zeros(2, 3, 5, 8).to(dtype)
+    for t in (base, base[0], base[1, 2], base[1, 2, 3], base[1, 2, 3, 4], base.transpose(1, 3), base[:, :, 1:4, 2:7],
+              base[0].t() if base[0].dim() == 2 else base[0].permute(2, 0, 1), base[:, :1], base.expand(2, 3, 5, 8)[:, :, :, ::2]):
+        d = S.desc(t)
+        ne, nb = _rule(t)
+        assert (d.type, d.reserved, d.data) == (type_, 0, t.data_ptr())
+        assert list(d.ne) == ne and list(d.nb) == nb
+
+
+@pytest.mark.parametrize("cls", [S.Q8Tensor, S.Q5KTensor])
+def test_block_descriptors(cls):
+    raw = torch.zeros(4, 7, 3 * cls.BYTES, dtype=torch.uint8)
+    for r in (raw, raw[1], raw[:, 2:5], raw[0, :, :cls.BYTES]):
+        n = r.shape[-1] // cls.BYTES * cls.ELEMS
+        d = S.desc(cls(r, n))
+        ne, nb = _rule(r)
+        ne[0], nb[0] = n, cls.BYTES
+        assert d.type == cls.TYPE and d.data == r.data_ptr()
+        assert list(d.ne) == ne and list(d.nb)[:r.dim()] == nb[:r.dim()]
+
+
+def test_refused_tensors():
+    assert S.desc(None) is None
+    with pytest.raises(KeyError):
+        S.desc(torch.zeros(3, dtype=torch.float64))
+    with pytest.raises(KeyError):
+        S.desc(torch.zeros(3, dtype=torch.uint8))       # raw blocks come in a BlockTensor
+    with pytest.raises(ValueError):
+        S.desc(torch.zeros(1, 1, 1, 1, 2))
+    with pytest.raises((AttributeError, TypeError)):
+        S.desc(3.0)
+
+
+def test_calls():
+    a, b = torch.zeros(2, 8), torch.zeros(2, 4)
+    f = S._fn("shp_swiglu")
+    assert f(a, None, b, 0) == S.ERR_INVALID_ARG        # shapes differ
+    assert f(None, a, a, None) == S.ERR_INVALID_ARG
+    with pytest.raises(TypeError):
+        f(a, a, a)                                      # no stream
+    with pytest.raises(TypeError):
+        S._fn("shp_norm")(a, "eps", a, 0)
+    with pytest.raises(AttributeError):
+        S._binding().bind(S.load()._handle, "shp_no_such_entry")
+    assert S._fn("shp_get_rows_sum")([a, a], 2, b, a, 0) == S.ERR_INVALID_ARG      # ids are not I32
+    assert S._fn("shp_pad")(a, [0, 0, 0, 0], b, 0) == S.ERR_INVALID_ARG
+    with pytest.raises(TypeError):
+        S._fn("shp_pad")(a, [0, 0], b, 0)
+    d = S.kernel_shape(3, 2)                            # a ctypes descriptor without data
+    assert S._fn("shp_im2col")(d, a, 1, 0, 1, b, 0) != S.OK
+    assert ctypes.sizeof(S.ShpTensor) == len(S._binding().describe(a))
