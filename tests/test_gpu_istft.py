@@ -41,6 +41,28 @@ def test_istft_matches_restatement(gpu, n_fft, hop, frames):
     _close(_np(gpu.inverse_stft(_t(gpu, spec), n_fft, hop)), R.run(lambda g: g.inverse_stft(spec, n_fft, hop)))
 
 
+@pytest.mark.parametrize("n_fft,hop,frames", [(2, 1, 9), (2, 1, 2000), (4, 7, 40), (20, 5, 43), (20, 5, 44), (20, 20, 700),
+                                              (20, 1, 300), (22, 3, 400), (254, 64, 30), (300, 30, 40), (30, 200, 30)])
+def test_istft_block_shapes(gpu, n_fft, hop, frames):
+    """Blocks of the rule's whole hops and of 256, 128 and 64 samples, the last
+    one sample long or full; windows of one bin pair, hops without overlap and
+    with gaps, and (n_fft 300, hop 30) the form without windowed samples."""
+    rng = np.random.default_rng([SEED, n_fft, hop, frames])
+    spec = rng.uniform(-3, 2, (frames, n_fft + 2)).astype(np.float32)
+    _close(_np(gpu.inverse_stft(_t(gpu, spec), n_fft, hop)), R.run(lambda g: g.inverse_stft(spec, n_fft, hop)))
+
+
+def test_istft_infinite_magnitude(gpu):
+    """A log-magnitude past exp's range makes its own frames' samples infinite or NaN and no others."""
+    rng = np.random.default_rng(SEED + 5)
+    spec = rng.uniform(-3, 2, (200, 22)).astype(np.float32)
+    spec[100, 4] = 1e5
+    got, ref = _np(gpu.inverse_stft(_t(gpu, spec), 20, 5)), R.run(lambda g: g.inverse_stft(spec, 20, 5))
+    assert np.array_equal(np.isfinite(got), np.isfinite(ref)) and not np.isfinite(ref).all()
+    ok = np.isfinite(ref)
+    _close(got[ok], ref[ok])
+
+
 def test_istft_strided_frames(gpu):
     """Frames at a row stride past n_fft + 2 values (a view of a wider
     tensor)."""
