@@ -1,26 +1,32 @@
 // Kokoro's harmonic-plus-noise source and its short-time spectrum for gfx950
 // (kokoro/source.cpp:60-184, build_harmonic_source; the host runs it between
-// the prosody and generator graphs). Four launches on one stream:
+// the prosody and generator graphs). Three launches on one stream:
 //
-//   k_source_coarse (a lane per frame and harmonic): the phase increments
-//     frac(f0 * (h+1) / rate) of the upsampled grid, resampled linearly to the
-//     f0 grid (PyTorch's align_corners=false mapping, in double, the weight
-//     rounded to f32), staged in the spectrum output's own memory until the
-//     excitation launch has read them;
-//   k_source_phase (one block): each harmonic's running f32 sum in frame
-//     order -- one lane per harmonic, the order the host code adds in, so the
-//     sums are bit for bit its own -- over LDS chunks, and the phase
-//     running * 2 pi * scale (double, rounded) in place of the increment;
+//   k_source_phase (one block): the phase increments frac(f0 * (h+1) / rate) of
+//     the upsampled grid, resampled linearly to the f0 grid (PyTorch's
+//     align_corners=false mapping, in double, the weight rounded to f32), into
+//     LDS, a harmonic's frames in a row; each harmonic's running f32 sum in
+//     frame order -- one lane per harmonic, the order the host code adds in, so
+//     the sums are bit for bit its own; and the phase running * 2 pi * scale
+//     (double, rounded), staged in the spectrum output's own memory until the
+//     excitation launch has read it;
 //   k_source_excite (a lane per upsampled sample): the phase resampled back,
 //     sin(phase) * amp for voiced samples plus the noise at its gain, merged
 //     with the weights in harmonic order from the bias, tanh;
-//   k_source_stft (a lane per frame and bin): torch.stft's centred framing --
+//   k_source_stft (blocks of whole frames): torch.stft's centred framing --
 //     reflect padding by n_fft/2, the periodic Hann window rounded to f32 --
-//     and the DFT in double with the host code's twiddles (the angle
-//     -2 pi b k / n_fft as it computes it), the magnitude by hypot and the
-//     phase by atan2, each rounded to f32.
+//     each windowed sample formed once into LDS, then a lane per frame and bin
+//     for the DFT in double with the host code's twiddles (the angle
+//     -2 pi b k / n_fft as it computes it), the magnitude by hypot and the phase
+//     by atan2, each rounded to f32.
 // The f32 sine and tanh are the device's, within an ulp or two of the host
 // library's; everything else is the host code's arithmetic in its order.
+//
+// Latency-bound: 5 seconds of speech are 400 serial sums, 120,000 samples and
+// 24,001 frames. Measured on MI355X at Kokoro's 9 harmonics, x300, n_fft 20, hop
+// 5: 1 second 16.2 -> 13.8 us, 5 seconds 28.4 -> 20.3, 20 seconds 76.6 -> 52.8, against
+// four launches with the increments in one of their own, the sums read one value
+// at a time and the twiddles of a 256-lane block made for 23 frames.
 
 #include <cmath>
 
@@ -54,16 +60,25 @@ struct SourceArgs {
     int32_t       nfft;
     int32_t       hop;
     int32_t       bins;
+    int32_t       fpb;    // frames per spectrum block
+    int32_t       pad;
+    FastDiv       fH;
+    FastDiv       fscale;
+    FastDiv       fnfft;
+    FastDiv       fbins;
 };
 
-// The increment of harmonic h at upsampled sample u.
-__device__ __forceinline__ float increment(const SourceArgs & a, int64_t u, int h) {
-    const float v = a.f0[u / a.scale] * static_cast<float>(h + 1) / a.rate;
-    float       r = v - floorf(v);
-    if (u == 0) {
-        r += a.ri[h];
-    }
-    return r;
+// The increment of harmonic h at a sample of frequency f0 (the initial phase
+// apart).
+__device__ __forceinline__ float increment(float f0, int h, float rate) {
+    const float v = f0 * static_cast<float>(h + 1) / rate;
+    return v - floorf(v);
+}
+
+// LDS floats per harmonic of a phase chunk: whole kSrcAhead runs of frames and
+// four of padding, kSrcChunk values in all at most.
+__host__ __device__ __forceinline__ int source_stride(int H) {
+    return kSrcChunk / H / 16 * 16 + 4;
 }
 
 // PyTorch's align_corners=false source position for output o, clamped at 0:
@@ -77,80 +92,86 @@ __device__ __forceinline__ void linear_at(int64_t o, double ratio, int64_t in_le
     w               = static_cast<float>(position - static_cast<double>(lo));
 }
 
-// The coarse increments, one lane per (frame, harmonic), staged in har.
-__global__ __launch_bounds__(256) void k_source_coarse(const SourceArgs a) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= a.L * a.H) {
-        return;
-    }
-    const int64_t j = i / a.H;
-    const int     h = static_cast<int>(i - j * a.H);
-    int64_t       lo, hi;
-    float         w;
-    linear_at(j, static_cast<double>(a.U) / static_cast<double>(a.L), a.U, lo, hi, w);
-    a.har[i] = increment(a, lo, h) * (1.0f - w) + increment(a, hi, h) * w;
-}
+// The increments, their running sums (one lane per harmonic in frame order) and
+// the phases, over LDS chunks of whole frames. A harmonic's frames lie in a row
+// of LDS, so its lane reads and writes four at a time, 16 ahead of their adds.
+constexpr int kSrcPhaseBlock = 1024;
+constexpr int kSrcAhead      = 16;
 
-// The running sums, one lane per harmonic in frame order, over LDS chunks of
-// the staged increments (each chunk read and written back in one coalesced
-// pass); the phase replaces the increment in place.
-__global__ __launch_bounds__(256) void k_source_phase(const SourceArgs a) {
-    extern __shared__ float s_run[];  // [chunk][H]
-    const int     tid   = static_cast<int>(threadIdx.x);
-    const int     H     = a.H;
-    const int64_t chunk = kSrcChunk / H;
-    float         run   = 0.0f;  // lane h < H: harmonic h's running sum
+__global__ __launch_bounds__(kSrcPhaseBlock) void k_source_phase(const SourceArgs a) {
+    extern __shared__ f32x4 s_run4[];  // [H][stride]
+    float *       s_run  = reinterpret_cast<float *>(s_run4);
+    const int     tid    = static_cast<int>(threadIdx.x);
+    const int     H      = a.H;
+    const int     stride = source_stride(H);
+    const int     chunk  = stride - 4;  // frames per chunk, a multiple of kSrcAhead
+    float         run    = 0.0f;        // lane h < H: harmonic h's running sum
     for (int64_t j0 = 0; j0 < a.L; j0 += chunk) {
-        const int64_t nj = a.L - j0 < chunk ? a.L - j0 : chunk;
-        const int64_t n = nj * H;
-        for (int64_t i0 = tid; i0 < n; i0 += 256 * 8) {  // eight loads in flight per lane
-            float v[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int64_t i = i0 + q * 256;
-                v[q]            = i < n ? a.har[j0 * H + i] : 0.0f;
+        const int nj = static_cast<int>(a.L - j0 < chunk ? a.L - j0 : chunk);
+        const int up = (nj + kSrcAhead - 1) / kSrcAhead * kSrcAhead;  // zeros past the last frame: x + 0 is x
+        // a lane per frame, whose position and f0 serve all its harmonics: the
+        // one block's lanes are few, and the increments' arithmetic is not
+        for (int j = tid; j < up; j += kSrcPhaseBlock) {
+            int64_t lo = 0, hi = 0;
+            float   w = 0.0f, flo = 0.0f, fhi = 0.0f;
+            if (j < nj) {
+                linear_at(j0 + j, static_cast<double>(a.U) / static_cast<double>(a.L), a.U, lo, hi, w);
+                flo = a.f0[fastdiv(static_cast<uint32_t>(lo), a.fscale)];
+                fhi = a.f0[fastdiv(static_cast<uint32_t>(hi), a.fscale)];
             }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int64_t i = i0 + q * 256;
-                if (i < n) {
-                    s_run[i] = v[q];
+            const bool apart = j < nj && (lo == 0 || __float_as_uint(flo) != __float_as_uint(fhi));
+            for (int h = 0; h < H; ++h) {
+                float r0 = increment(flo, h, a.rate), r1 = r0;
+                if (apart) {
+                    r1 = increment(fhi, h, a.rate);
+                    r0 = lo == 0 ? r0 + a.ri[h] : r0;
+                    r1 = hi == 0 ? r1 + a.ri[h] : r1;
                 }
+                s_run[h * stride + j] = j < nj ? r0 * (1.0f - w) + r1 * w : 0.0f;
             }
         }
         __syncthreads();
         if (tid < H) {
-            constexpr int kAhead = 16;  // reads ahead of their adds; the sums stay in frame order
-            int64_t       j      = 0;
-            for (; j + kAhead <= nj; j += kAhead) {
-                float v[kAhead];
+            f32x4 * row = reinterpret_cast<f32x4 *>(s_run + tid * stride);
+            f32x4   next[kSrcAhead / 4];
 #pragma unroll
-                for (int q = 0; q < kAhead; ++q) {
-                    v[q] = s_run[(j + q) * H + tid];
-                }
-#pragma unroll
-                for (int q = 0; q < kAhead; ++q) {
-                    run = run + v[q];
-                    v[q] = run;
-                }
-#pragma unroll
-                for (int q = 0; q < kAhead; ++q) {
-                    s_run[(j + q) * H + tid] = v[q];
-                }
+            for (int q = 0; q < kSrcAhead / 4; ++q) {
+                next[q] = row[q];
             }
-            for (; j < nj; ++j) {
-                run                = run + s_run[j * H + tid];
-                s_run[j * H + tid] = run;
+            for (int j = 0; j < up; j += kSrcAhead) {
+                f32x4 v[kSrcAhead / 4];
+#pragma unroll
+                for (int q = 0; q < kSrcAhead / 4; ++q) {
+                    v[q]    = next[q];
+                    next[q] = row[(j + kSrcAhead < up ? j + kSrcAhead : j) / 4 + q];
+                }
+#pragma unroll
+                for (int q = 0; q < kSrcAhead / 4; ++q) {
+                    v[q].x = run + v[q].x;
+                    v[q].y = v[q].x + v[q].y;
+                    v[q].z = v[q].y + v[q].z;
+                    v[q].w = v[q].z + v[q].w;
+                    run    = v[q].w;
+                }
+#pragma unroll
+                for (int q = 0; q < kSrcAhead / 4; ++q) {
+                    row[j / 4 + q] = v[q];
+                }
             }
         }
         __syncthreads();
-        for (int64_t i = tid; i < nj * H; i += 256) {
-            a.har[j0 * H + i] = static_cast<float>(static_cast<double>(s_run[i]) * 2.0 * kSrcPi *
+        for (int t = tid; t < nj * H; t += kSrcPhaseBlock) {
+            const int j       = static_cast<int>(fastdiv(static_cast<uint32_t>(t), a.fH));
+            const int h       = t - j * H;
+            a.har[j0 * H + t] = static_cast<float>(static_cast<double>(s_run[h * stride + j]) * 2.0 * kSrcPi *
                                                    static_cast<double>(a.scale));
         }
         __syncthreads();
     }
 }
+
+// Harmonics whose loads go out before the first one's sine.
+constexpr int kSrcBatch = 5;
 
 __global__ __launch_bounds__(256) void k_source_excite(const SourceArgs a) {
     const int64_t u = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -160,58 +181,87 @@ __global__ __launch_bounds__(256) void k_source_excite(const SourceArgs a) {
     int64_t lo, hi;
     float   w;
     linear_at(u, static_cast<double>(a.L) / static_cast<double>(a.U), a.L, lo, hi, w);
-    const float   f0u    = a.f0[u / a.scale];
+    const float   f0u    = a.f0[fastdiv(static_cast<uint32_t>(u), a.fscale)];
     const float   uv     = f0u > a.threshold ? 1.0f : 0.0f;
     const float   gain   = uv * a.noise_std + (1.0f - uv) * a.amp / 3.0f;
     const float * plo    = a.har + lo * a.H;
     const float * phi    = a.har + hi * a.H;
     const float * nz     = a.noise + u * a.H;
     float         merged = a.bias;
-    for (int h = 0; h < a.H; ++h) {
-        const float fine  = plo[h] * (1.0f - w) + phi[h] * w;
-        const float sine  = sinf(fine) * a.amp;
-        const float value = sine * uv + gain * nz[h];
-        merged            = merged + a.mw[h] * value;
+    for (int h0 = 0; h0 < a.H; h0 += kSrcBatch) {
+        float p0[kSrcBatch], p1[kSrcBatch], n[kSrcBatch], mw[kSrcBatch];
+#pragma unroll
+        for (int q = 0; q < kSrcBatch; ++q) {
+            const int h = h0 + q < a.H ? h0 + q : a.H - 1;
+            p0[q]       = plo[h];
+            p1[q]       = phi[h];
+            n[q]        = nz[h];
+            mw[q]       = a.mw[h];
+        }
+#pragma unroll
+        for (int q = 0; q < kSrcBatch; ++q) {
+            if (h0 + q < a.H) {
+                const float fine  = p0[q] * (1.0f - w) + p1[q] * w;
+                const float sine  = sinf(fine) * a.amp;
+                const float value = sine * uv + gain * n[q];
+                merged            = merged + mw[q] * value;
+            }
+        }
     }
     a.exc[u] = tanhf(merged);
 }
 
-__global__ __launch_bounds__(256) void k_source_stft(const SourceArgs a) {
-    __shared__ double2 s_tw[(kSrcMaxNfft / 2 + 1) * kSrcMaxNfft];
-    __shared__ float   s_win[kSrcMaxNfft];
-    const int tid = static_cast<int>(threadIdx.x);
-    for (int i = tid; i < a.bins * a.nfft; i += 256) {
-        const int    b     = i / a.nfft;
-        const int    k     = i - b * a.nfft;
-        const double angle = -2.0 * kSrcPi * static_cast<double>(b) * static_cast<double>(k) / static_cast<double>(a.nfft);
-        s_tw[i]            = double2{ cos(angle), sin(angle) };
-    }
-    for (int k = tid; k < a.nfft; k += 256) {
-        s_win[k] = static_cast<float>(0.5 * (1.0 - cos(2.0 * kSrcPi * static_cast<double>(k) / static_cast<double>(a.nfft))));
-    }
-    __syncthreads();
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + tid;
-    if (i >= a.frames * a.bins) {
-        return;
-    }
-    const int64_t f    = i / a.bins;
-    const int     b    = static_cast<int>(i - f * a.bins);
-    const int     half = a.nfft / 2;
-    const int64_t last = a.U - 1;
-    double        re = 0.0, im = 0.0;
-    for (int k = 0; k < a.nfft; ++k) {
-        int64_t src = f * a.hop + k - half;
+// Frames per spectrum block: an item (frame, bin) per lane. (256 lanes with two
+// items each: the f64 hypot and atan2 chains then run one after the other.)
+constexpr int kSrcStftBlock = 512;
+
+__global__ __launch_bounds__(kSrcStftBlock) void k_source_stft(const SourceArgs a) {
+    extern __shared__ double2 s_tw[];  // [nfft][bins] twiddles, then [fpb][nfft] windowed samples, then the window
+    float *       s_seg = reinterpret_cast<float *>(s_tw + a.bins * a.nfft);
+    float *       s_win = s_seg + a.fpb * a.nfft;
+    const int     tid   = static_cast<int>(threadIdx.x);
+    const int64_t f0    = static_cast<int64_t>(blockIdx.x) * a.fpb;
+    const int     nf    = static_cast<int>(a.frames - f0 < a.fpb ? a.frames - f0 : a.fpb);
+    const int     half  = a.nfft / 2;
+    const int64_t last  = a.U - 1;
+    for (int i = tid; i < nf * a.nfft; i += kSrcStftBlock) {
+        const int f   = static_cast<int>(fastdiv(static_cast<uint32_t>(i), a.fnfft));
+        int64_t   src = (f0 + f) * a.hop + (i - f * a.nfft) - half;
         while (src < 0 || src > last) {  // reflection without repeating the edge sample
             src = src < 0 ? -src : 2 * last - src;
         }
-        const float   seg = a.exc[src] * s_win[k];
-        const double2 t   = s_tw[b * a.nfft + k];
-        re += static_cast<double>(seg) * t.x;
-        im += static_cast<double>(seg) * t.y;
+        s_seg[i] = a.exc[src];
     }
-    float * row       = a.har + f * 2 * a.bins;
-    row[b]            = static_cast<float>(hypot(re, im));
-    row[a.bins + b]   = static_cast<float>(atan2(im, re));
+    for (int i = tid; i < (a.bins + 1) * a.nfft; i += kSrcStftBlock) {
+        const int k = static_cast<int>(fastdiv(static_cast<uint32_t>(i), a.fbins));  // by bins, one past the twiddles' rows
+        if (i < a.bins * a.nfft) {
+            const int    b     = i - k * a.bins;
+            const double angle = -2.0 * kSrcPi * static_cast<double>(b) * static_cast<double>(k) / static_cast<double>(a.nfft);
+            double       sn, cs;
+            sincos(angle, &sn, &cs);
+            s_tw[i] = double2{ cs, sn };
+        } else {
+            const int j = i - a.bins * a.nfft;
+            s_win[j] = static_cast<float>(0.5 * (1.0 - cos(2.0 * kSrcPi * static_cast<double>(j) / static_cast<double>(a.nfft))));
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < nf * a.bins; i += kSrcStftBlock) {
+        const int     f   = static_cast<int>(fastdiv(static_cast<uint32_t>(i), a.fbins));
+        const int     b   = i - f * a.bins;
+        const float * x   = s_seg + f * a.nfft;
+        double        re = 0.0, im = 0.0;
+#pragma unroll 4
+        for (int k = 0; k < a.nfft; ++k) {
+            const float   seg = x[k] * s_win[k];
+            const double2 t   = s_tw[k * a.bins + b];
+            re += static_cast<double>(seg) * t.x;
+            im += static_cast<double>(seg) * t.y;
+        }
+        float * row     = a.har + (f0 + f) * 2 * a.bins;
+        row[b]          = static_cast<float>(hypot(re, im));
+        row[a.bins + b] = static_cast<float>(atan2(im, re));
+    }
 }
 
 bool contiguous_f32(const shp_tensor * t) {
@@ -290,15 +340,15 @@ extern "C" shp_status_t shp_harmonic_source(const shp_tensor * f0,
     a.nfft      = n_fft;
     a.hop       = hop;
     a.bins      = static_cast<int32_t>(bins);
-    const hipStream_t st    = as_stream(stream);
-    const int64_t     chunk = kSrcChunk / H;
-    hipLaunchKernelGGL(k_source_coarse, dim3(static_cast<unsigned>((L * H + 255) / 256)), dim3(256), 0, st, a);
+    a.fpb       = static_cast<int32_t>(kSrcStftBlock / bins);
+    a.fH        = make_fastdiv(static_cast<uint32_t>(H));
+    a.fscale    = make_fastdiv(static_cast<uint32_t>(upsample_scale));
+    a.fnfft     = make_fastdiv(static_cast<uint32_t>(n_fft));
+    a.fbins     = make_fastdiv(static_cast<uint32_t>(bins));
+    const hipStream_t st = as_stream(stream);
+    hipLaunchKernelGGL(k_source_phase, dim3(1), dim3(kSrcPhaseBlock),
+                       static_cast<size_t>(H * source_stride(static_cast<int>(H))) * sizeof(float), st, a);
     shp_status_t s = launch_status();
-    if (s != SHP_OK) {
-        return s;
-    }
-    hipLaunchKernelGGL(k_source_phase, dim3(1), dim3(256), static_cast<size_t>(chunk * H) * sizeof(float), st, a);
-    s = launch_status();
     if (s != SHP_OK) {
         return s;
     }
@@ -307,6 +357,7 @@ extern "C" shp_status_t shp_harmonic_source(const shp_tensor * f0,
     if (s != SHP_OK) {
         return s;
     }
-    hipLaunchKernelGGL(k_source_stft, dim3(static_cast<unsigned>((frames * bins + 255) / 256)), dim3(256), 0, st, a);
+    const size_t lds = static_cast<size_t>(bins * n_fft) * sizeof(double2) + static_cast<size_t>((a.fpb + 1) * n_fft) * sizeof(float);
+    hipLaunchKernelGGL(k_source_stft, dim3(static_cast<unsigned>((frames + a.fpb - 1) / a.fpb)), dim3(kSrcStftBlock), lds, st, a);
     return launch_status();
 }

@@ -59,6 +59,17 @@ def test_source_matches_restatement(gpu, L, H, scale, n_fft, hop):
     _close(_run_gpu(gpu, args, kw), _run_ref(args, kw), n_fft // 2 + 1)
 
 
+@pytest.mark.parametrize("L,H,scale,n_fft,hop", [(2, 1, 1, 2, 1), (50, 2, 1, 4, 1), (15, 9, 300, 20, 5), (16, 4, 30, 20, 5),
+                                                 (17, 64, 40, 64, 16), (129, 64, 64, 64, 16), (896, 9, 24, 20, 5),
+                                                 (897, 9, 24, 20, 5), (33, 3, 50, 20, 37), (100, 5, 2, 62, 1)])
+def test_source_block_shapes(gpu, L, H, scale, n_fft, hop):
+    """Frames around the runs of 16 the serial sums read ahead and around a
+    chunk (896 frames of 9 harmonics, 128 of 64), one sample per frame, every
+    window up to 64, hops that skip samples, spectrum blocks of one frame."""
+    args, kw = random_source_case(SEED + 31 * L + H, L, H, scale, n_fft, hop)
+    _close(_run_gpu(gpu, args, kw), _run_ref(args, kw), n_fft // 2 + 1)
+
+
 def test_source_refusals(gpu):
     import torch
     d = _load("kokoro_source.json")
