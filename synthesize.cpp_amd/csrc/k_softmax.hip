@@ -16,12 +16,13 @@
 // or +inf (or only -inf) comes out NaN, as on the CPU: the max is then NaN or
 // inf, or the NaN reaches the sum.
 //
-// Launch shapes: rows up to 2048 wide are held in registers. With float4
-// rows, a row takes one wave (wave-level reductions only: no LDS, no barrier)
-// when there are enough rows to fill the chip, else 2 or 4 waves (the decode
-// step's 16 rows of ~512, a short prefill's 1024 rows of 2048); other rows
-// take one wave each with scalar accesses. Wider rows take one 256-thread
-// block per row and three passes over the row.
+// Launch shapes: rows of up to 16384 scores are held in the registers of 1 to
+// 16 waves, a float4 from any 4-byte boundary at a time (a prompt of an odd
+// length has odd rows): one wave per row (wave-level reductions only: no LDS,
+// no barrier) where the rows fill the chip, more where they are few or long
+// (the decode step's 16 rows, a short prefill). Longer rows take one block and
+// three passes over the row; rows of up to 128 scores a wave and an element per
+// lane at a time.
 
 #include <cmath>
 
@@ -64,13 +65,8 @@ struct SoftMaxArgs {
 // +inf or NaN score drops out instead of turning the row into NaN).
 enum MaskKind { kMaskNone = 0, kMaskTensor = 1, kMaskCausal = 2 };
 
-constexpr int kSoftMaxWaveMax = 2048;  // widest row of the one-wave kernel
-constexpr int kSoftMaxBlock   = 256;
-
-// exp with the table read from memory (divergent loops).
-__device__ __forceinline__ float exp_f32(float x) {
-    return exp_f32_rn(x, [](int j) { return kExpTable[j]; });
-}
+constexpr int kSoftMaxRegs  = 16384;  // widest row held in registers
+constexpr int kSoftMaxBlock = 1024;   // threads per longer row
 
 // Mask row of score row r = (i1, i2, i3): ggml's i11 = i1, i12 = i2 % ne12,
 // i13 = i3 % ne13.
@@ -108,7 +104,9 @@ template <int MK> __device__ __forceinline__ void softmax_args_in_sgprs(const So
     }
 }
 
-// One wave per row, element lane + 64k in register k (k < K, 64K >= ne0).
+// One wave per row of up to 64 K scores (K at most 2), element lane + 64k in
+// register k: a lane then has one or two exps in its chain, not a float4's four
+// (a decode step's 16 rows of 38: 1.71 us, 2.04 by float4).
 template <int K, int MK> __global__ __launch_bounds__(256) void k_soft_max_wave(const SoftMaxArgs a) {
     constexpr bool MASK = MK == kMaskTensor;
     __shared__ double s_tab[256 / kWave][64];
@@ -175,16 +173,27 @@ template <int K, int MK> __global__ __launch_bounds__(256) void k_soft_max_wave(
     }
 }
 
-// float4 rows (16-byte aligned rows, ne0 % 4 == 0), WPR waves per row: lane q
-// of the row's 64*WPR lanes holds chunks q + 64*WPR*k in registers k (k < K4).
+// Rows of at least four scores, WPR waves per row: lane q of the row's 64*WPR
+// lanes holds chunks q + 64*WPR*k in registers k (k < K4). Chunk c is the four
+// scores from 4c on; the row's last chunk, where fewer are left, the row's last
+// four, whose first ones belong to the chunk before (left out of the sum here,
+// and stored twice with the same value).
 // The scores are read and the probabilities written once per launch, so both
 // stream with the nontemporal hint (the mask, shared by heads, stays
 // cacheable): 21 % faster than plain loads and stores at [512,512,16] on
-// MI355X (9.65 -> 7.58 us).
+// MI355X (9.65 -> 7.58 us). The causal form does not read a chunk that the mask
+// hides, nor take its exps. Measured on MI355X (cold) against a wave per row with
+// 4-byte accesses for odd rows and a 256-thread block of three passes past 2048:
+// 16 heads of 1021 x 1021 31.0 -> 27.0 us, with a mask 35.4 -> 31.7, causal 30.2 ->
+// 23.8; 16 rows of 4000 9.6 -> 3.3, 16 x 16 rows of 4096 15.8 -> 4.7, 8 x 64 of
+// 12000 66 -> 14; 1024 x 1024 with aligned rows unchanged (26.2). Slower for 1021:
+// two or four waves a row (30.1, 33.8). With a mask, blocks of one position's
+// four heads, to share its row: 30.8, but 28.1 against 26.8 at 1024.
 // WPR > 1 spreads the few long rows of a decode or short prefill over more
 // waves; the row's waves then combine their max and sum through LDS, in wave
 // order.
-template <int WPR, int K4, int MK, int BLOCK = 256>
+// ODD: the row is no whole number of chunks.
+template <int WPR, int K4, int MK, bool ODD, int BLOCK = (WPR > 4 ? WPR * kWave : 256)>
 __global__ __launch_bounds__(BLOCK) void k_soft_max_rows4(const SoftMaxArgs a) {
     constexpr bool MASK   = MK == kMaskTensor;
     constexpr int  kLanes = kWave * WPR;
@@ -202,12 +211,13 @@ __global__ __launch_bounds__(BLOCK) void k_soft_max_rows4(const SoftMaxArgs a) {
         return;  // whole wave; the one-wave form has no barrier
     }
     const int64_t rr = live ? r : 0;
-    const f32x4 * xr =
-        reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, rr));
-    f32x4 *       yr    = reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, rr));
-    const f32x4 * mr    = MASK ? reinterpret_cast<const f32x4 *>(mask_row(a, rr)) : nullptr;
-    const int64_t lim   = MK == kMaskCausal ? causal_lim(a, rr) : 0;
-    const int     n4 = live ? a.ne0 / 4 : 0;
+    const float * xr = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, rr));
+    float *       yr = reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, rr));
+    const float * mr = MASK ? mask_row(a, rr) : nullptr;
+    const int64_t lim  = MK == kMaskCausal ? causal_lim(a, rr) : 0;
+    const int     nc   = live ? (a.ne0 + 3) / 4 : 0;
+    const int     last = a.ne0 - 4;  // the last chunk's first score
+    auto          first = [last](int c) { return ODD && c * 4 > last ? last : c * 4; };  // of chunk c
     f32x4         w[K4];
     f32x4         mk[K4];
     // The exp table's entry is loaded with the row, so it is not a round trip
@@ -218,12 +228,20 @@ __global__ __launch_bounds__(BLOCK) void k_soft_max_rows4(const SoftMaxArgs a) {
 #pragma unroll
     for (int k = 0; k < K4; ++k) {
         const int c = q + kLanes * k;
-        w[k]        = ld_stream(xr + (c < n4 ? c : 0));
-        mk[k]       = MASK ? mr[c < n4 ? c : 0] : splat4(0.0f);
+        const int i = c < nc ? first(c) : 0;
+        if constexpr (MK == kMaskCausal) {
+            w[k] = splat4(-INFINITY);
+            if (i <= lim) {
+                w[k] = ld_stream4u(xr + i);
+            }
+        } else {
+            w[k] = ld_stream4u(xr + i);
+        }
+        mk[k] = MASK ? ld4u(mr + i) : splat4(0.0f);
     }
 #pragma unroll
     for (int k = 0; k < K4; ++k) {
-        const bool in = q + kLanes * k < n4;
+        const bool in = q + kLanes * k < nc;
         w[k]          = in ? w[k] : splat4(0.0f);
         mk[k]         = in ? mk[k] : splat4(0.0f);
     }
@@ -237,12 +255,12 @@ __global__ __launch_bounds__(BLOCK) void k_soft_max_rows4(const SoftMaxArgs a) {
             w[k] = f32x4{ w[k].x + mk[k].x, w[k].y + mk[k].y, w[k].z + mk[k].z, w[k].w + mk[k].w };
         }
         if constexpr (MK == kMaskCausal) {
-            const int64_t i = static_cast<int64_t>(c) * 4;
+            const int64_t i = first(c);
             w[k]            = f32x4{ i > lim ? -INFINITY : w[k].x, i + 1 > lim ? -INFINITY : w[k].y,
                                      i + 2 > lim ? -INFINITY : w[k].z, i + 3 > lim ? -INFINITY : w[k].w };
         }
         const float m4 = fmaxf(fmaxf(w[k].x, w[k].y), fmaxf(w[k].z, w[k].w));
-        mx             = c < n4 ? fmaxf(mx, m4) : mx;
+        mx             = c < nc ? fmaxf(mx, m4) : mx;
     }
     mx = wave_max(mx);
     if constexpr (WPR > 1) {
@@ -260,11 +278,20 @@ __global__ __launch_bounds__(BLOCK) void k_soft_max_rows4(const SoftMaxArgs a) {
 #pragma unroll
     for (int k = 0; k < K4; ++k) {
         const int c = q + kLanes * k;
+        if (MK == kMaskCausal && WPR == 1 && kLanes * k * 4 > lim + 3 && mx > -INFINITY) {
+            // the wave's chunks are all hidden, the scores a last chunk shares
+            // with the one before it included: e^-inf (an infinite or NaN
+            // maximum takes the exps)
+            w[k] = splat4(0.0f);
+            continue;
+        }
         w[k] = f32x4{ exp_f32_lds(w[k].x - mx, tab), exp_f32_lds(w[k].y - mx, tab), exp_f32_lds(w[k].z - mx, tab),
                       exp_f32_lds(w[k].w - mx, tab) };
-        const double s4 = (static_cast<double>(w[k].x) + static_cast<double>(w[k].y)) +
-                          (static_cast<double>(w[k].z) + static_cast<double>(w[k].w));
-        sum += c < n4 ? s4 : 0.0;
+        // the last chunk's scores that are the chunk before's
+        const int    twice = ODD ? c * 4 - last : 0;
+        const double s4    = (static_cast<double>(twice > 0 ? 0.0f : w[k].x) + static_cast<double>(twice > 1 ? 0.0f : w[k].y)) +
+                          (static_cast<double>(twice > 2 ? 0.0f : w[k].z) + static_cast<double>(w[k].w));
+        sum += c < nc ? s4 : 0.0;
     }
     sum = group_sum<kWave>(sum);
     if constexpr (WPR > 1) {
@@ -282,40 +309,56 @@ __global__ __launch_bounds__(BLOCK) void k_soft_max_rows4(const SoftMaxArgs a) {
 #pragma unroll
     for (int k = 0; k < K4; ++k) {
         const int c = q + kLanes * k;
-        if (c < n4) {
-            st_stream(yr + c, f32x4{ w[k].x * inv, w[k].y * inv, w[k].z * inv, w[k].w * inv });
+        if (c < nc) {
+            st_stream4u(yr + first(c),
+                        f32x4{ w[k].x * inv, w[k].y * inv, w[k].z * inv, w[k].w * inv });
         }
     }
 }
 
-// One block per row, three passes: the max, the sum, the scaled exps.
+// One block per row too long for registers, three passes: the max, the sum,
+// the scaled exps; chunks as above.
 template <int MK>
-__device__ __forceinline__ float sm_w(const SoftMaxArgs & a, const float * xr, const float * mr, int64_t lim, int i) {
-    float w = xr[i] * a.scale;
+__device__ __forceinline__ f32x4 sm_w4(const SoftMaxArgs & a, const float * xr, const float * mr, int64_t lim, int i) {
+    f32x4 w;
+    if constexpr (MK == kMaskCausal) {
+        w = i <= lim ? ld4u(xr + i) : splat4(-INFINITY);
+    } else {
+        w = ld4u(xr + i);
+    }
+    w = f32x4{ w.x * a.scale, w.y * a.scale, w.z * a.scale, w.w * a.scale };
     if constexpr (MK == kMaskTensor) {
-        w = w + mr[i];
+        const f32x4 m = ld4u(mr + i);
+        w             = f32x4{ w.x + m.x, w.y + m.y, w.z + m.z, w.w + m.w };
     }
     if constexpr (MK == kMaskCausal) {
-        w = i > lim ? -INFINITY : w;
+        w = f32x4{ i > lim ? -INFINITY : w.x, i + 1 > lim ? -INFINITY : w.y, i + 2 > lim ? -INFINITY : w.z,
+                   i + 3 > lim ? -INFINITY : w.w };
     }
     return w;
 }
 
 template <int MK> __global__ __launch_bounds__(kSoftMaxBlock) void k_soft_max_block(const SoftMaxArgs a) {
-    constexpr bool MASK = MK == kMaskTensor;
-    __shared__ float  s_max[kSoftMaxBlock / kWave];
-    __shared__ double s_sum[kSoftMaxBlock / kWave];
-    const int64_t r    = blockIdx.x;
-    const int     lane = threadIdx.x % kWave;
-    const int     wv   = threadIdx.x / kWave;
-    const float * xr   = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, r));
-    float *       yr   = reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, r));
-    const float * mr   = MASK ? mask_row(a, r) : nullptr;
-    const int64_t lim  = MK == kMaskCausal ? causal_lim(a, r) : 0;
+    constexpr bool MASK   = MK == kMaskTensor;
+    constexpr int  kWaves = kSoftMaxBlock / kWave;
+    __shared__ float  s_max[kWaves];
+    __shared__ double s_sum[kWaves];
+    __shared__ double s_tab[kWaves][64];
+    const int64_t  r    = blockIdx.x;
+    const int      lane = threadIdx.x % kWave;
+    const int      wv   = threadIdx.x / kWave;
+    const float *  xr   = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, r));
+    float *        yr   = reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, r));
+    const float *  mr   = MASK ? mask_row(a, r) : nullptr;
+    const int64_t  lim  = MK == kMaskCausal ? causal_lim(a, r) : 0;
+    const int      nc   = (a.ne0 + 3) / 4, last = a.ne0 - 4;
+    const double * tab  = wave_exp_table(s_tab, lane, exp_table_entry(lane));
 
     float mx = -INFINITY;
-    for (int i = threadIdx.x; i < a.ne0; i += kSoftMaxBlock) {
-        mx = fmaxf(mx, sm_w<MK>(a, xr, mr, lim, i));
+#pragma unroll 2
+    for (int c = threadIdx.x; c < nc; c += kSoftMaxBlock) {
+        const f32x4 w = sm_w4<MK>(a, xr, mr, lim, c * 4 < last ? c * 4 : last);
+        mx            = fmaxf(mx, fmaxf(fmaxf(w.x, w.y), fmaxf(w.z, w.w)));
     }
     mx = wave_max(mx);
     if (lane == 0) {
@@ -324,13 +367,18 @@ template <int MK> __global__ __launch_bounds__(kSoftMaxBlock) void k_soft_max_bl
     __syncthreads();
     mx = s_max[0];
 #pragma unroll
-    for (int j = 1; j < kSoftMaxBlock / kWave; ++j) {
+    for (int j = 1; j < kWaves; ++j) {
         mx = fmaxf(mx, s_max[j]);
     }
 
     double sum = 0.0;
-    for (int i = threadIdx.x; i < a.ne0; i += kSoftMaxBlock) {
-        sum += static_cast<double>(exp_f32(sm_w<MK>(a, xr, mr, lim, i) - mx));
+#pragma unroll 2
+    for (int c = threadIdx.x; c < nc; c += kSoftMaxBlock) {
+        const f32x4 w     = sm_w4<MK>(a, xr, mr, lim, c * 4 < last ? c * 4 : last);
+        const int   twice = c * 4 - last;
+        const float e0 = exp_f32_lds(w.x - mx, tab), e1 = exp_f32_lds(w.y - mx, tab), e2 = exp_f32_lds(w.z - mx, tab);
+        sum += (static_cast<double>(twice > 0 ? 0.0f : e0) + static_cast<double>(twice > 1 ? 0.0f : e1)) +
+               (static_cast<double>(twice > 2 ? 0.0f : e2) + static_cast<double>(exp_f32_lds(w.w - mx, tab)));
     }
     sum = group_sum<kWave>(sum);
     if (lane == 0) {
@@ -339,79 +387,88 @@ template <int MK> __global__ __launch_bounds__(kSoftMaxBlock) void k_soft_max_bl
     __syncthreads();
     sum = s_sum[0];
 #pragma unroll
-    for (int j = 1; j < kSoftMaxBlock / kWave; ++j) {
+    for (int j = 1; j < kWaves; ++j) {
         sum += s_sum[j];
     }
     const float inv = static_cast<float>(1.0 / sum);
-    for (int i = threadIdx.x; i < a.ne0; i += kSoftMaxBlock) {
-        yr[i] = exp_f32(sm_w<MK>(a, xr, mr, lim, i) - mx) * inv;
+    // Each score is written by the chunk that owns it (the last chunk's shared
+    // ones by the chunk before), which has read it: in place, nothing reads a
+    // written score but the last chunk, read ahead of the barrier.
+    const int   tail  = nc - 1;
+    const bool  owner = static_cast<int>(threadIdx.x) == tail % kSoftMaxBlock;
+    const f32x4 wt    = owner ? sm_w4<MK>(a, xr, mr, lim, last) : splat4(0.0f);
+    __syncthreads();
+#pragma unroll 2
+    for (int c = threadIdx.x; c < tail; c += kSoftMaxBlock) {
+        const f32x4 w = sm_w4<MK>(a, xr, mr, lim, c * 4);
+        st_stream4u(yr + c * 4, f32x4{ exp_f32_lds(w.x - mx, tab) * inv, exp_f32_lds(w.y - mx, tab) * inv,
+                                       exp_f32_lds(w.z - mx, tab) * inv, exp_f32_lds(w.w - mx, tab) * inv });
+    }
+    if (owner) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (last + e >= tail * 4) {
+                yr[last + e] = exp_f32_lds(wt[e] - mx, tab) * inv;
+            }
+        }
     }
 }
 
-template <int MK> shp_status_t launch_soft_max(const SoftMaxArgs & a, bool vec, hipStream_t stream) {
+template <int MK, bool ODD, class Go> shp_status_t launch_rows4(const SoftMaxArgs & a, const Go & go) {
+    const int nc = (a.ne0 + 3) / 4;
+    if (nc <= 64) {
+        return go(k_soft_max_rows4<1, 1, MK, ODD>, 4, 256);
+    }
+    // Few rows (under 8 waves per CU at one wave per row): 2, 4 or 16 waves per
+    // row. The decode step's 16 rows of 512 take one wave each (2.30 us
+    // against 2.36 us with two waves and their LDS combine, MI355X), in
+    // one-wave blocks: each row on its own CU (2.12 -> 1.99 us warm; the
+    // 28-layer decode graph's layer with the softmax 9.62 -> 9.45 us).
+    if (a.nrows < 2048 && nc >= 128) {
+        if (nc >= 256) {
+            if (a.nrows <= 256 && nc > 512) {
+                return nc <= 1024 ? go(k_soft_max_rows4<16, 1, MK, ODD>, 1, 1024) :
+                       nc <= 2048 ? go(k_soft_max_rows4<16, 2, MK, ODD>, 1, 1024) :
+                                    go(k_soft_max_rows4<16, 4, MK, ODD>, 1, 1024);
+            }
+            return nc <= 256  ? go(k_soft_max_rows4<4, 1, MK, ODD>, 1, 256) :
+                   nc <= 512  ? go(k_soft_max_rows4<4, 2, MK, ODD>, 1, 256) :
+                   nc <= 1024 ? go(k_soft_max_rows4<4, 4, MK, ODD>, 1, 256) :
+                   nc <= 2048 ? go(k_soft_max_rows4<4, 8, MK, ODD>, 1, 256) :
+                                go(k_soft_max_rows4<16, 4, MK, ODD>, 1, 1024);
+        }
+        if (a.nrows > 64) {
+            return nc <= 128 ? go(k_soft_max_rows4<2, 1, MK, ODD>, 2, 256) : go(k_soft_max_rows4<2, 2, MK, ODD>, 2, 256);
+        }
+    }
+    if (nc <= 128) {
+        // a decode step's few rows: one one-wave block per row
+        return a.nrows <= 64 ? go(k_soft_max_rows4<1, 2, MK, ODD, kWave>, 1, kWave) :
+                               go(k_soft_max_rows4<1, 2, MK, ODD>, 4, 256);
+    }
+    return nc <= 256  ? go(k_soft_max_rows4<1, 4, MK, ODD>, 4, 256) :
+           nc <= 512  ? (MK == kMaskCausal ? go(k_soft_max_rows4<1, 8, MK, ODD>, 4, 256) :
+                                             go(k_soft_max_rows4<2, 4, MK, ODD>, 2, 256)) :
+           nc <= 1024 ? go(k_soft_max_rows4<4, 4, MK, ODD>, 1, 256) :
+           nc <= 2048 ? go(k_soft_max_rows4<4, 8, MK, ODD>, 1, 256) : go(k_soft_max_rows4<16, 4, MK, ODD>, 1, 1024);
+}
+
+template <int MK> shp_status_t launch_soft_max(const SoftMaxArgs & a, hipStream_t stream) {
     if (dry_run()) {
         return SHP_OK;
     }
-    if (a.ne0 > kSoftMaxWaveMax) {
-        hipLaunchKernelGGL((k_soft_max_block<MK>), dim3(static_cast<unsigned>(a.nrows)), dim3(kSoftMaxBlock), 0,
-                           stream, a);
+    auto go = [&](auto kernel, int rows_per_block, int block) {
+        const int64_t blocks = (a.nrows + rows_per_block - 1) / rows_per_block;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(block), 0, stream, a);
         return launch_status();
+    };
+    if (a.ne0 <= 2 * kWave) {
+        return a.ne0 <= kWave ? go(k_soft_max_wave<1, MK>, 4, 256) : go(k_soft_max_wave<2, MK>, 4, 256);
     }
-    const dim3 grid(static_cast<unsigned>((a.nrows + 3) / 4));
-    if (vec) {
-        // Few rows (under 8 waves per CU at one wave per row): 2 or 4 waves per
-        // row. The decode step's 16 rows of 512 take one wave each (2.30 us
-        // against 2.36 us with two waves and their LDS combine, MI355X), in
-        // one-wave blocks: each row on its own CU (2.12 -> 1.99 us warm; the
-        // 28-layer decode graph's layer with the softmax 9.62 -> 9.45 us).
-        const int n4  = a.ne0 / 4;
-        const int wpr = a.nrows >= 2048 ? 1 : (n4 >= 256 ? 4 : (n4 >= 128 && a.nrows > 64 ? 2 : 1));
-        const int k4  = (n4 + kWave * wpr - 1) / (kWave * wpr);
-        const dim3 g4(static_cast<unsigned>((a.nrows * wpr + 3) / 4));
-        if (wpr == 4) {
-            if (k4 <= 1) {
-                hipLaunchKernelGGL((k_soft_max_rows4<4, 1, MK>), g4, dim3(256), 0, stream, a);
-            } else {
-                hipLaunchKernelGGL((k_soft_max_rows4<4, 2, MK>), g4, dim3(256), 0, stream, a);
-            }
-        } else if (wpr == 2) {
-            if (k4 <= 1) {
-                hipLaunchKernelGGL((k_soft_max_rows4<2, 1, MK>), g4, dim3(256), 0, stream, a);
-            } else if (k4 <= 2) {
-                hipLaunchKernelGGL((k_soft_max_rows4<2, 2, MK>), g4, dim3(256), 0, stream, a);
-            } else {
-                hipLaunchKernelGGL((k_soft_max_rows4<2, 4, MK>), g4, dim3(256), 0, stream, a);
-            }
-        } else if (k4 <= 1) {
-            hipLaunchKernelGGL((k_soft_max_rows4<1, 1, MK>), g4, dim3(256), 0, stream, a);
-        } else if (k4 <= 2 && a.nrows <= 64) {
-            // a decode step's few rows: one one-wave block per row
-            hipLaunchKernelGGL((k_soft_max_rows4<1, 2, MK, kWave>), dim3(static_cast<unsigned>(a.nrows)), dim3(kWave),
-                               0, stream, a);
-        } else if (k4 <= 2) {
-            hipLaunchKernelGGL((k_soft_max_rows4<1, 2, MK>), g4, dim3(256), 0, stream, a);
-        } else if (k4 <= 4) {
-            hipLaunchKernelGGL((k_soft_max_rows4<1, 4, MK>), g4, dim3(256), 0, stream, a);
-        } else {
-            hipLaunchKernelGGL((k_soft_max_rows4<1, 8, MK>), g4, dim3(256), 0, stream, a);
-        }
-        return launch_status();
+    if (a.ne0 > kSoftMaxRegs) {
+        return go(k_soft_max_block<MK>, 1, kSoftMaxBlock);
     }
-    const int k = (a.ne0 + kWave - 1) / kWave;
-    if (k <= 1) {
-        hipLaunchKernelGGL((k_soft_max_wave<1, MK>), grid, dim3(256), 0, stream, a);
-    } else if (k <= 2) {
-        hipLaunchKernelGGL((k_soft_max_wave<2, MK>), grid, dim3(256), 0, stream, a);
-    } else if (k <= 4) {
-        hipLaunchKernelGGL((k_soft_max_wave<4, MK>), grid, dim3(256), 0, stream, a);
-    } else if (k <= 8) {
-        hipLaunchKernelGGL((k_soft_max_wave<8, MK>), grid, dim3(256), 0, stream, a);
-    } else if (k <= 16) {
-        hipLaunchKernelGGL((k_soft_max_wave<16, MK>), grid, dim3(256), 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((k_soft_max_wave<32, MK>), grid, dim3(256), 0, stream, a);
-    }
-    return launch_status();
+    return a.ne0 % 4 == 0 ? launch_rows4<MK, false>(a, go) : launch_rows4<MK, true>(a, go);
 }
 
 }  // namespace
@@ -469,12 +526,8 @@ extern "C" shp_status_t shp_soft_max_ext(const shp_tensor * a,
             g.fmne3 = make_fastdiv(static_cast<uint32_t>(g.mne3));
         }
     }
-    // float4 rows: every row start of the scores, the output and the mask
-    // 16-byte aligned and whole float4s per row
-    const bool vec = a->ne[0] % 4 == 0 && rows_aligned(*a, 16) && rows_aligned(*y, 16) &&
-                     (mask == nullptr || rows_aligned(*mask, 16));
-    return mask != nullptr ? launch_soft_max<kMaskTensor>(g, vec, as_stream(stream))
-                           : launch_soft_max<kMaskNone>(g, vec, as_stream(stream));
+    return mask != nullptr ? launch_soft_max<kMaskTensor>(g, as_stream(stream))
+                           : launch_soft_max<kMaskNone>(g, as_stream(stream));
 }
 
 // ggml_diag_mask_inf(x, n_past): every element past n_past + its row's index
@@ -567,6 +620,5 @@ extern "C" shp_status_t shp_soft_max_causal(const shp_tensor * a,
     g.n_past = n_past;
     g.mfast  = 1;  // rows below 2^31
     g.fne1   = make_fastdiv(static_cast<uint32_t>(g.ne1));
-    const bool vec = a->ne[0] % 4 == 0 && rows_aligned(*a, 16) && rows_aligned(*y, 16);
-    return launch_soft_max<kMaskCausal>(g, vec, as_stream(stream));
+    return launch_soft_max<kMaskCausal>(g, as_stream(stream));
 }
