@@ -16,10 +16,13 @@
 // entry (no loop: a block's stores never wait at a barrier):
 //   1. the tile's input window (ICT channel rows of (OWT-1)*s0 + (K-1)*d0 + 1
 //      samples, zeros past the input's ends) goes to LDS, consecutive lanes on
-//      consecutive addresses: along time for a time-contiguous x, along
-//      channels for a channel-contiguous x (the transposed view of a
-//      channel-major activation, so the ggml_cont the reference puts in front
-//      of im2col is not needed);
+//      consecutive addresses, four values a lane: along time for a
+//      time-contiguous x, along channels for a channel-contiguous x (the
+//      transposed view of a channel-major activation, so the ggml_cont the
+//      reference puts in front of im2col is not needed). Value by value, behind
+//      a leaky-ReLU that has just written x (MI355X, both launches): K = 3
+//      [128,131072] 75.3 -> 72.5 us, [256,4136] 10.4 -> 9.1; K = 7 d = 3 F16
+//      [128,131072] 101 -> 89.7;
 //   2. the tile's outputs are written in y's order, V values (16 bytes) per
 //      store. The LDS offsets of the values a store takes repeat with a short
 //      period -- one position's run of ICT*K values, or for a tile of every
@@ -28,7 +31,10 @@
 //      read, V window reads and running sums, with no division.
 // Both phases step their indices by running sums: the kernel is bound by its
 // stores, not by address arithmetic (per-value divisions held an earlier form
-// to ~65 % of HBM peak at [128,131072], K = 3).
+// to ~65 % of HBM peak at [128,131072], K = 3). A replay over inputs that no
+// kernel rewrites reads them from the Infinity Cache (the stores bypass it):
+// the figures below are such replays' and compare tiles, but an input fresh
+// from its producer comes from HBM, at 5.4 TB/s with the writes.
 
 #include "shp_internal.hpp"
 
@@ -38,6 +44,7 @@ namespace {
 constexpr int kIm2colBlock = 256;
 constexpr int kIm2colLds   = 4480;   // floats of LDS window per block at most (17.5 KB; with the table, 8 blocks per CU)
 constexpr int kIm2colBatch = 8;      // window loads a lane issues before its LDS writes
+constexpr int kIm2colQuads = 4;      // the same for float4 loads
 constexpr int kIm2colTab   = 1024;   // int16 LDS offsets of the store table (one period)
 
 // Tile shape: ict channels; at least owt positions, or enough for `elems`
@@ -71,6 +78,11 @@ inline TileRule tile_rule(bool chfast, bool f16, int64_t ic, int64_t k) {
     }
     return f16 ? TileRule{ 32, 128, 8192 } : TileRule{ 32, 64, 8192 };
 }
+
+// How a block reads its window: value by value (any strides), or four samples of
+// a channel (time-contiguous x) or four channels of a sample (channel-contiguous)
+// per load.
+enum Im2colWalk { kWalkValues = 0, kWalkTime = 1, kWalkChannels = 2 };
 
 struct Im2colArgs {
     const char * x;
@@ -153,10 +165,11 @@ __device__ __forceinline__ int tap_offset(const Im2colArgs & a, uint32_t f, cons
 // values). Otherwise each position has a run of ICT*K values, a multiple of V,
 // starting V-aligned (table period: one run). V == 1: no table, one value per
 // lane and step, located by division (layouts the others cannot take).
-template <bool FLAT, int V, bool F16, bool CHFAST>
+template <bool FLAT, int V, bool F16, int WALK>
 __global__ __launch_bounds__(kIm2colBlock) void k_im2col(const Im2colArgs a) {
     typedef int16_t         tv __attribute__((ext_vector_type(V > 1 ? V : 2)));  // one store's offsets
-    extern __shared__ float lds[];
+    extern __shared__ f32x4 lds4[];
+    float *                 lds = reinterpret_cast<float *>(lds4);
     __shared__ tv           tabv[V > 1 ? kIm2colTab / V : 1];
     int16_t *               tab = reinterpret_cast<int16_t *>(tabv);
     const int               tid = static_cast<int>(threadIdx.x);
@@ -173,42 +186,87 @@ __global__ __launch_bounds__(kIm2colBlock) void k_im2col(const Im2colArgs a) {
     const int               wlo = static_cast<int>(iw0 < 0 ? -iw0 : 0);                      // first sample in x
     const int               whi = static_cast<int>(a.iw - iw0 < a.wt ? a.iw - iw0 : a.wt);  // past the last
     // 1. the window, by running sums; zeros outside [wlo, whi) and for
-    //    channels past IC (never read)
-    {
-        const int nf = static_cast<int>(a.fdiv.d);
-        int       s  = static_cast<int>(fastdiv(static_cast<uint32_t>(tid), a.fdiv));
-        int       f  = tid - s * nf;
-        int       ox = s * a.nbs + f * a.nbf;
-        int       ol = s * a.ls + f * a.lf;
-        const int sx = a.ds * a.nbs + a.df * a.nbf, cx = a.nbs - nf * a.nbf;
-        const int sl = a.ds * a.ls + a.df * a.lf, cl = a.ls - nf * a.lf;
+    //    channels past IC (never read). (Offsets past the walk's end wrap,
+    //    unused.)
+    const int nf = static_cast<int>(a.fdiv.d);
+    int       s  = static_cast<int>(fastdiv(static_cast<uint32_t>(tid), a.fdiv));
+    int       f  = tid - s * nf;
+    uint32_t  ox = static_cast<uint32_t>(s) * a.nbs + static_cast<uint32_t>(f) * a.nbf;
+    int       ol = s * a.ls + f * a.lf;
+    const uint32_t sx = static_cast<uint32_t>(a.ds) * a.nbs + static_cast<uint32_t>(a.df) * a.nbf;
+    const uint32_t cx = static_cast<uint32_t>(a.nbs) - static_cast<uint32_t>(nf) * a.nbf;
+    const int      sl = a.ds * a.ls + a.df * a.lf, cl = a.ls - nf * a.lf;
+    auto           step = [&]() {
+        s += a.ds;
+        f += a.df;
+        ox += sx;
+        ol += sl;
+        if (f >= nf) {
+            f -= nf;
+            ++s;
+            ox += cx;
+            ol += cl;
+        }
+    };
+    if constexpr (WALK == kWalkValues) {
         while (s < a.ns) {
             float v[kIm2colBatch];
             int   at[kIm2colBatch];
 #pragma unroll
             for (int u = 0; u < kIm2colBatch; ++u) {
-                const int icl = CHFAST ? f : s;
-                const int w   = CHFAST ? s : f;
-                at[u]         = s < a.ns ? ol : -1;
-                v[u]          = 0.0f;
-                if (s < a.ns && icl < nic && w >= wlo && w < whi) {
+                at[u] = s < a.ns ? ol : -1;
+                v[u]  = 0.0f;
+                if (s < a.ns && s < nic && f >= wlo && f < whi) {
                     v[u] = *reinterpret_cast<const float *>(xw + ox);
                 }
-                s += a.ds;
-                f += a.df;
-                ox += sx;
-                ol += sl;
-                if (f >= nf) {
-                    f -= nf;
-                    ++s;
-                    ox += cx;
-                    ol += cl;
-                }
+                step();
             }
 #pragma unroll
             for (int u = 0; u < kIm2colBatch; ++u) {
                 if (at[u] >= 0) {
                     lds[at[u]] = v[u];
+                }
+            }
+        }
+    } else {
+        // four at a time from any 4-byte boundary: whole where the row goes on
+        // in memory (past the window's last sample too: its row of LDS has room)
+        const int most = WALK == kWalkTime ? static_cast<int>(a.iw - iw0 < a.wt + 4 ? a.iw - iw0 : a.wt + 4) : nic;
+        const int from = WALK == kWalkTime ? wlo : 0;
+        while (s < a.ns) {
+            f32x4 v[kIm2colQuads];
+            int   at[kIm2colQuads], ch[kIm2colQuads];
+#pragma unroll
+            for (int u = 0; u < kIm2colQuads; ++u) {
+                at[u]         = s < a.ns ? ol : -1;
+                ch[u]         = f * 4;
+                v[u]          = splat4(0.0f);
+                const bool in = s < a.ns && (WALK == kWalkTime ? s < nic : (s >= wlo && s < whi));
+                if (in && f * 4 >= from && f * 4 + 4 <= most) {
+                    v[u] = ld4u(reinterpret_cast<const float *>(xw + ox));
+                } else if (in) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (f * 4 + e >= from && f * 4 + e < most) {
+                            v[u][e] = reinterpret_cast<const float *>(xw + ox)[e];
+                        }
+                    }
+                }
+                step();
+            }
+#pragma unroll
+            for (int u = 0; u < kIm2colQuads; ++u) {
+                if (at[u] >= 0) {
+                    if constexpr (WALK == kWalkTime) {
+                        *reinterpret_cast<f32x4 *>(lds + at[u]) = v[u];
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if (ch[u] + e < a.ict) {
+                                lds[at[u] + e * a.wtp] = v[u][e];
+                            }
+                        }
+                    }
                 }
             }
         }
@@ -303,20 +361,21 @@ __global__ __launch_bounds__(kIm2colBlock) void k_im2col(const Im2colArgs a) {
 }
 
 template <bool FLAT, int V, bool F16>
-void launch_form(const Im2colArgs & a, bool chfast, unsigned grid, size_t shmem, hipStream_t s) {
-    if (chfast) {
-        hipLaunchKernelGGL((k_im2col<FLAT, V, F16, true>), dim3(grid), dim3(kIm2colBlock), shmem, s, a);
-    } else {
-        hipLaunchKernelGGL((k_im2col<FLAT, V, F16, false>), dim3(grid), dim3(kIm2colBlock), shmem, s, a);
-    }
+void launch_form(const Im2colArgs & a, int walk, unsigned grid, size_t shmem, hipStream_t s) {
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(kIm2colBlock), shmem, s, a); };
+    walk == kWalkTime     ? go(k_im2col<FLAT, V, F16, kWalkTime>) :
+    walk == kWalkChannels ? go(k_im2col<FLAT, V, F16, kWalkChannels>) : go(k_im2col<FLAT, V, F16, kWalkValues>);
 }
 
 inline int64_t window(int64_t owt, int64_t s0, int64_t k, int64_t d0) {
     return (owt - 1) * s0 + (k - 1) * d0 + 1;
 }
 
-inline int64_t padded(int64_t w) {
-    return w | 1;  // an odd row stride spreads a column of the window over the banks
+// LDS row stride of a window of w samples: odd, which spreads a column of the
+// window over the banks; for rows written 16 bytes at a time, an odd number of
+// float4, which spreads 16 channels' taps over all of them.
+inline int64_t padded(int64_t w, bool quads) {
+    return quads ? ((w + 3) / 4 | 1) * 4 : w | 1;
 }
 
 inline int64_t gcd64(int64_t a, int64_t b) {
@@ -343,6 +402,7 @@ struct Im2colPlan {
     int        v      = 1;   // values per store: 1, 4 (F32 or F16) or 8 (F16)
     bool       f16    = false;
     bool       chfast = false;
+    int        walk   = kWalkValues;
     unsigned   grid   = 0;   // one block per tile
     size_t     shmem  = 0;
 };
@@ -441,22 +501,24 @@ shp_status_t plan_im2col(const shp_tensor * kernel, const shp_tensor * x, int32_
     a.ict              = static_cast<int32_t>(ict);
     a.owt              = static_cast<int32_t>(owt);
     a.wt               = static_cast<int32_t>(wt);
-    a.wtp              = static_cast<int32_t>(padded(wt));
+    pl.walk            = pl.chfast ? kWalkChannels : (nb0 == 4 ? kWalkTime : kWalkValues);
+    a.wtp              = static_cast<int32_t>(padded(wt, pl.walk == kWalkTime));
     a.tic              = make_fastdiv(static_cast<uint32_t>(tic));
     a.tow              = make_fastdiv(static_cast<uint32_t>(tow));
     a.kdiv             = make_fastdiv(static_cast<uint32_t>(K));
     a.rdiv             = make_fastdiv(static_cast<uint32_t>(IC * K));
     a.segf             = make_fastdiv(static_cast<uint32_t>(ict * K));
     a.segl             = make_fastdiv(static_cast<uint32_t>(last * K));
-    const int64_t nf   = pl.chfast ? ict : wt;
+    const int64_t per  = pl.walk == kWalkValues ? 1 : 4;  // values per load
+    const int64_t nf   = ((pl.chfast ? ict : wt) + per - 1) / per;
     a.fdiv             = make_fastdiv(static_cast<uint32_t>(nf));
     a.ns               = static_cast<int32_t>(pl.chfast ? wt : ict);
     a.ds               = static_cast<int32_t>(kIm2colBlock / nf);
     a.df               = static_cast<int32_t>(kIm2colBlock % nf);
     a.nbs              = static_cast<int32_t>(pl.chfast ? nb0 : nb1);
-    a.nbf              = static_cast<int32_t>(pl.chfast ? nb1 : nb0);
+    a.nbf              = static_cast<int32_t>((pl.chfast ? nb1 : nb0) * per);
     a.ls               = pl.chfast ? 1 : a.wtp;
-    a.lf               = pl.chfast ? a.wtp : 1;
+    a.lf               = static_cast<int32_t>((pl.chfast ? a.wtp : 1) * per);
     // Stores of 16 bytes where the layout allows (8 values of F16, 4 of F32),
     // else 8 bytes of F16, else one value. One table period must fit.
     const size_t    esz   = pl.f16 ? 2 : 4;
@@ -479,7 +541,7 @@ shp_status_t plan_im2col(const shp_tensor * kernel, const shp_tensor * x, int32_
 
 shp_status_t launch_im2col(const Im2colPlan & pl, hipStream_t s) {
     const Im2colArgs & a = pl.args;
-    const bool         c = pl.chfast;
+    const int          c = pl.walk;
     if (pl.f16) {
         if (pl.flat) {
             pl.v == 8 ? launch_form<true, 8, true>(a, c, pl.grid, pl.shmem, s) :

@@ -197,3 +197,22 @@ def test_cont_im2col_run_equals_its_nodes(gpu, C, T, K, d0, f16):
     assert np.array_equal(outs[0].view(np.uint16 if f16 else np.uint32), outs[1].view(np.uint16 if f16 else np.uint32))
     ref = _cols_ref(np.ascontiguousarray(x.T), K, 1, (K - 1) * d0, d0, R.F16 if f16 else R.F32)
     _check(torch.from_numpy(outs[0]), ref, R.F16 if f16 else R.F32)
+
+
+@pytest.mark.parametrize("layout", ["time", "channels", "neither"])
+@pytest.mark.parametrize("IC,IW,K,s0,p0,d0", [(3, 1, 1, 1, 0, 1), (2, 2, 3, 1, 1, 1), (6, 3, 2, 1, 0, 1), (17, 4, 3, 1, 1, 1),
+                                              (33, 63, 3, 1, 1, 1), (34, 65, 5, 1, 2, 1), (35, 67, 3, 2, 1, 1),
+                                              (5, 257, 7, 1, 9, 3), (131, 130, 3, 1, 200, 1), (16, 1025, 4, 3, 2, 7)])
+def test_im2col_window_walks(gpu, IC, IW, K, s0, p0, d0, layout):
+    """The window read four samples of a channel, four channels of a sample or
+    one value at a time: rows and channel counts of every remainder of four,
+    inside a wider tensor whose neighbours (7) must not show."""
+    import torch
+    rng = np.random.default_rng([SEED + 7, IC, IW, K])
+    x = rng.standard_normal((IC, IW)).astype(np.float32)
+    shape, pick = {"time": ((IC + 2, IW + 3), lambda b: b[1:1 + IC, 1:1 + IW]),
+                   "channels": ((IW + 3, IC + 2), lambda b: b[1:1 + IW, 1:1 + IC].t()),
+                   "neither": ((IC + 2, 2 * IW + 3), lambda b: b[1:1 + IC, 1:1 + 2 * IW:2])}[layout]
+    view = pick(torch.full(shape, 7.0, device="cuda"))
+    view.copy_(_t(gpu, x))
+    _check(gpu.im2col(view, K, s0, p0, d0), _cols_ref(x, K, s0, p0, d0, R.F32), R.F32)
