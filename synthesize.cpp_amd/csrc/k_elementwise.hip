@@ -1194,8 +1194,10 @@ template <int TYPE> __global__ __launch_bounds__(256) void k_cast_rows(const Cas
 // LDS: the loads read 512-byte source lines along dim k, the stores write
 // 256-byte destination lines along dim 0. Consecutive blocks take the tiles of
 // one dim-0 range along dim k first; the other two dimensions (a, b) number
-// the tiles last. V = 4: 16-byte accesses (every stride and both extents
-// allow it); V = 1 otherwise.
+// the tiles last. 16-byte accesses from any 4-byte boundary (an utterance's
+// samples are rows of any length). 24001 x 128 8.3 -> 6.9 us, 1536 x 937 5.1 -> 4.2,
+// 31999 x 256 24.2 -> 16.4, the tail with residual and sum at 256 x 31999 53.8 ->
+// 32.9, against 4-byte accesses for such rows and tiles in order.
 // Measured on MI355X (cold inputs, the vocoder shapes [C,T] = [128,131072],
 // [256,32768], [512,8192]): 25.2 / 13.6 / 6.4 us, against 29.6 / 13.7 / 7.5 us
 // for 64 x 64 tiles with dim 0 first, 27.3 / 14.3 / 6.7 us with tiles spread
@@ -1216,7 +1218,9 @@ struct TransposeArgs {
     FastDiv      t0;    // tiles along dim 0
     FastDiv      na;    // extent of dim a
     uint32_t     ntiles;
-    uint32_t     pad;
+    uint32_t     nblocks;
+    uint32_t     perxcd;  // tiles per XCD where neighbouring tiles share cache lines, else 0: tiles in order
+    uint32_t     pad3;
     // epilogue (shp_cont_add_leaky_relu)
     const char * bias;   // one value per destination row, at row number * brs
     int64_t      brs;
@@ -1231,6 +1235,9 @@ struct TransposeArgs {
 
 constexpr int kTile0 = 64;
 constexpr int kTileK = 128;
+// Elements from which partly written lines are kept in L2: 128 x 24001 (12 MB)
+// 6.9 us streamed, 7.3 kept; 256 x 31999 (33 MB) 18.8 and 16.2 (MI355X, cold).
+constexpr int64_t kTransposeKeep = int64_t{ 1 } << 22;
 
 // Epilogue bits: add the bias -- the destination row's value (kEpiBias) or
 // one value per destination column, a row of ne0 repeated over the rows
@@ -1238,29 +1245,58 @@ constexpr int kTileK = 128;
 // write that sum, apply leaky-ReLU.
 enum TransposeEpi { kEpiBias = 1, kEpiResid = 2, kEpiLeaky = 4, kEpiSum = 8, kEpiBias0 = 16 };
 
-// One tile: loads into registers, LDS, stores. FULL = the tile lies wholly
-// inside the tensor: no guards, so each load's data goes to LDS as it arrives
-// and the LDS reads of two passes issue before their stores. The epilogue's
-// bias values and residual rows are requested with the tile's loads, before
-// the barrier.
-template <int V, bool FULL, int EPI>
+// One tile: loads into registers, LDS, stores, 16 bytes a lane from any 4-byte
+// boundary. FULL = the tile lies wholly inside the tensor: no guards, so each
+// load's data goes to LDS as it arrives and the LDS reads of two passes issue
+// before their stores. The epilogue's bias values and residual rows are
+// requested with the tile's loads, before the barrier.
+template <bool WHOLE> __device__ __forceinline__ f32x4 tile_load(const char * p, int left) {
+    const float * x = reinterpret_cast<const float *>(p);
+    if (WHOLE || left >= 4) {
+        return ld_stream4u(x);
+    }
+    f32x4 v = splat4(0.0f);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        if (e < left) {
+            v[e] = x[e];
+        }
+    }
+    return v;
+}
+
+template <bool WHOLE, bool KEEP> __device__ __forceinline__ void tile_store(char * p, f32x4 v, int left) {
+    float * y = reinterpret_cast<float *>(p);
+    if (WHOLE || left >= 4) {
+        if constexpr (KEEP) {
+            *reinterpret_cast<f32x4u *>(y) = v;
+        } else {
+            st_stream4u(y, v);
+        }
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        if (e < left) {
+            y[e] = v[e];
+        }
+    }
+}
+
+template <bool FULL, bool ODD, bool KEEP, int EPI>
 __device__ __forceinline__ void transpose_tile(float (&tile)[kTile0][kTileK + 1], float (&s_bias)[kTileK],
                                                const TransposeArgs & a, const char * xb, char * yb, int64_t i0,
                                                int64_t row0, int n0, int nk) {
-    typedef float vec __attribute__((ext_vector_type(V)));
-    constexpr int RL = kTileK / V, RLINES = 256 / RL, RPASS = kTile0 / RLINES;  // loads: lines along dim k
-    constexpr int WL = kTile0 / V, WLINES = 256 / WL, WPASS = kTileK / WLINES;  // stores: lines along dim 0
-    const int     rc = (static_cast<int>(threadIdx.x) % RL) * V, rl = static_cast<int>(threadIdx.x) / RL;
-    const int     wc = (static_cast<int>(threadIdx.x) % WL) * V, wl = static_cast<int>(threadIdx.x) / WL;
-    vec           v[RPASS];
+    constexpr int RL = kTileK / 4, RLINES = 256 / RL, RPASS = kTile0 / RLINES;  // loads: lines along dim k
+    constexpr int WL = kTile0 / 4, WLINES = 256 / WL, WPASS = kTileK / WLINES;  // stores: lines along dim 0
+    const int     rc = (static_cast<int>(threadIdx.x) % RL) * 4, rl = static_cast<int>(threadIdx.x) / RL;
+    const int     wc = (static_cast<int>(threadIdx.x) % WL) * 4, wl = static_cast<int>(threadIdx.x) / WL;
+    f32x4         v[RPASS];
 #pragma unroll
     for (int p = 0; p < RPASS; ++p) {
         const int r = rl + p * RLINES;
-        if (FULL || (r < n0 && rc < nk)) {
-            v[p] = __builtin_nontemporal_load(reinterpret_cast<const vec *>(xb + static_cast<int64_t>(r) * a.xnb0 + rc * 4));
-        } else {
-            v[p] = vec{};
-        }
+        v[p] = FULL || (r < n0 && rc < nk) ? tile_load<FULL || !ODD>(xb + static_cast<int64_t>(r) * a.xnb0 + rc * 4, nk - rc) :
+                                             splat4(0.0f);
     }
     // The tile's 128 destination lines take one bias value each: one load per
     // line into LDS (8 loads per lane otherwise: measured 3-9 % slower).
@@ -1271,29 +1307,27 @@ __device__ __forceinline__ void transpose_tile(float (&tile)[kTile0][kTileK + 1]
             s_bias[r]    = *reinterpret_cast<const float *>(a.bias + (row0 + rr * a.rowk) * a.brs);
         }
     }
-    // kEpiBias0: the lane's V columns are the same in every pass: one load
+    // kEpiBias0: the lane's four columns are the same in every pass: one load
     // (b is one contiguous row of ne0 values).
-    vec b0{};
+    f32x4 b0 = splat4(0.0f);
     if constexpr ((EPI & kEpiBias0) != 0) {
         if (FULL || wc < n0) {
-            b0 = *reinterpret_cast<const vec *>(a.bias + (i0 + wc) * 4);
+            b0 = tile_load<FULL || !ODD>(a.bias + (i0 + wc) * 4, n0 - wc);
         }
     }
-    vec rv[WPASS];
+    f32x4 rv[WPASS];
 #pragma unroll
     for (int p = 0; p < WPASS; ++p) {
         const int  r  = wl + p * WLINES;  // ik local
         const bool in = FULL || (r < nk && wc < n0);
         if constexpr ((EPI & kEpiResid) != 0) {
-            rv[p] = in ? __builtin_nontemporal_load(
-                             reinterpret_cast<const vec *>(yb + a.rdelta + static_cast<int64_t>(r) * a.ynbk + wc * 4)) :
-                         vec{};
+            rv[p] = in ? tile_load<FULL || !ODD>(yb + a.rdelta + static_cast<int64_t>(r) * a.ynbk + wc * 4, n0 - wc) : splat4(0.0f);
         }
     }
 #pragma unroll
     for (int p = 0; p < RPASS; ++p) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
+        for (int e = 0; e < 4; ++e) {
             tile[rl + p * RLINES][rc + e] = v[p][e];
         }
     }
@@ -1302,9 +1336,9 @@ __device__ __forceinline__ void transpose_tile(float (&tile)[kTile0][kTileK + 1]
     for (int p = 0; p < WPASS; ++p) {
         const int   r  = wl + p * WLINES;  // ik local
         const float bv = (EPI & kEpiBias) != 0 ? s_bias[r] : 0.0f;
-        vec         w;
+        f32x4       w;
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
+        for (int e = 0; e < 4; ++e) {
             w[e] = tile[wc + e][r];
             if constexpr ((EPI & kEpiBias) != 0) {
                 w[e] = w[e] + bv;
@@ -1319,24 +1353,28 @@ __device__ __forceinline__ void transpose_tile(float (&tile)[kTile0][kTileK + 1]
         if (FULL || (r < nk && wc < n0)) {
             char * yo = yb + static_cast<int64_t>(r) * a.ynbk + wc * 4;
             if constexpr ((EPI & kEpiSum) != 0) {
-                __builtin_nontemporal_store(w, reinterpret_cast<vec *>(yo + a.sdelta));
+                tile_store<FULL || !ODD, KEEP>(yo + a.sdelta, w, n0 - wc);
             }
             if constexpr ((EPI & kEpiLeaky) != 0) {
 #pragma unroll
-                for (int e = 0; e < V; ++e) {
+                for (int e = 0; e < 4; ++e) {
                     w[e] = leaky(w[e], a.slope);
                 }
             }
-            __builtin_nontemporal_store(w, reinterpret_cast<vec *>(yo));
+            tile_store<FULL || !ODD, KEEP>(yo, w, n0 - wc);
         }
     }
     __syncthreads();
 }
 
-template <int V, int EPI> __global__ __launch_bounds__(256) void k_transpose_tiles(const TransposeArgs a) {
+template <bool ODD, bool KEEP, int EPI> __global__ __launch_bounds__(256) void k_transpose_tiles(const TransposeArgs a) {
     __shared__ float tile[kTile0][kTileK + 1];  // [i0 local][ik local]; the pad staggers a column's banks
     __shared__ float s_bias[kTileK];              // the epilogue's bias value per destination line
-    for (uint32_t t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
+    for (uint32_t j = blockIdx.x; j < a.nblocks; j += gridDim.x) {
+        const uint32_t t = a.perxcd != 0 ? (j & 7u) * a.perxcd + (j >> 3) : j;
+        if (t >= a.ntiles) {
+            continue;  // whole block
+        }
         const uint32_t q0   = fastdiv(t, a.tk);
         const uint32_t q1   = fastdiv(q0, a.t0);
         const uint32_t ib   = fastdiv(q1, a.na);
@@ -1349,21 +1387,18 @@ template <int V, int EPI> __global__ __launch_bounds__(256) void k_transpose_til
         const int      n0   = static_cast<int>(a.ne0 - i0 < kTile0 ? a.ne0 - i0 : kTile0);
         const int      nk   = static_cast<int>(a.nek - ik < kTileK ? a.nek - ik : kTileK);
         if (n0 == kTile0 && nk == kTileK) {
-            transpose_tile<V, true, EPI>(tile, s_bias, a, xb, yb, i0, row0, n0, nk);
+            transpose_tile<true, ODD, KEEP, EPI>(tile, s_bias, a, xb, yb, i0, row0, n0, nk);
         } else {
-            transpose_tile<V, false, EPI>(tile, s_bias, a, xb, yb, i0, row0, n0, nk);
+            transpose_tile<false, ODD, KEEP, EPI>(tile, s_bias, a, xb, yb, i0, row0, n0, nk);
         }
     }
 }
 
-// The transposing copy's plan: dims, tiles, strides, and whether 16-byte
-// accesses apply (every line start on both sides 16-byte aligned and both tile
-// extents multiples of 4; the stride of a dimension of extent 1 is never
-// used). SHP_ERR_UNSUPPORTED when x has no contiguous dimension or the tile
-// count passes 2^31.
+// The transposing copy's plan: dims, tiles and strides. SHP_ERR_UNSUPPORTED when
+// x has no contiguous dimension or the tile count passes 2^31.
 struct TransposePlan {
     TransposeArgs args{};
-    bool          v4    = false;
+    bool          keep  = false;  // stores not streamed past L2
     unsigned      grid  = 0;
     int           k     = 0;
     int           da    = 0;
@@ -1413,13 +1448,17 @@ shp_status_t plan_transpose(const shp_tensor * x, const shp_tensor * y, Transpos
     a.rowk                  = rownum[k];
     a.rowa                  = rownum[dims[0]];
     a.rowb                  = rownum[dims[1]];
-    const auto    a16 = [](int64_t ne, int64_t nb) { return ne == 1 || nb % 16 == 0; };
-    const int64_t nea = x->ne[dims[0]], neb = x->ne[dims[1]];
-    pl.v4             = reinterpret_cast<uintptr_t>(x->data) % 16 == 0 &&
-             reinterpret_cast<uintptr_t>(y->data) % 16 == 0 && a16(a.ne0, a.xnb0) && a16(nea, a.xnba) &&
-             a16(neb, a.xnbb) && a16(a.nek, a.ynbk) && a16(nea, a.ynba) && a16(neb, a.ynbb) && a.ne0 % 4 == 0 &&
-             a.nek % 4 == 0;
-    pl.grid = static_cast<unsigned>(nt < (1 << 20) ? nt : (1 << 20));
+    // Rows that are no whole cache lines: a tile's 256-byte stores (512-byte
+    // loads) end inside lines that the next tile along them takes up. Eight
+    // consecutive blocks go to the eight XCDs, each with an L2 of its own, so
+    // every XCD gets a run of consecutive tiles to share those lines in one L2;
+    // and of a large tensor the stores are not streamed past it.
+    const auto lines  = [](const void * p, int64_t ne, int64_t nb) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && (ne == 1 || nb % 128 == 0); };
+    const bool ylines = lines(y->data, a.nek, a.ynbk);
+    a.perxcd          = ylines && lines(x->data, a.ne0, a.xnb0) ? 0 : static_cast<uint32_t>((nt + 7) / 8);
+    pl.keep           = !ylines && nelements(*y) >= kTransposeKeep;
+    a.nblocks         = a.perxcd != 0 ? a.perxcd * 8 : a.ntiles;
+    pl.grid           = a.nblocks < (1u << 20) ? a.nblocks : 1u << 20;
     pl.k    = k;
     pl.da   = dims[0];
     pl.db   = dims[1];
@@ -1427,10 +1466,13 @@ shp_status_t plan_transpose(const shp_tensor * x, const shp_tensor * y, Transpos
 }
 
 template <int EPI> shp_status_t launch_transpose(const TransposePlan & pl, hipStream_t stream) {
-    if (pl.v4) {
-        hipLaunchKernelGGL((k_transpose_tiles<4, EPI>), dim3(pl.grid), dim3(256), 0, stream, pl.args);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(pl.grid), dim3(256), 0, stream, pl.args); };
+    if (pl.keep) {
+        go(k_transpose_tiles<true, true, EPI>);
+    } else if (pl.args.ne0 % 4 == 0 && pl.args.nek % 4 == 0) {
+        go(k_transpose_tiles<false, false, EPI>);
     } else {
-        hipLaunchKernelGGL((k_transpose_tiles<1, EPI>), dim3(pl.grid), dim3(256), 0, stream, pl.args);
+        go(k_transpose_tiles<true, false, EPI>);
     }
     return launch_status();
 }
@@ -1666,9 +1708,6 @@ extern "C" shp_status_t shp_cont_add_leaky_relu(const shp_tensor * x,
     if (!per_row && !per_col) {
         return SHP_ERR_UNSUPPORTED;
     }
-    if (per_col && reinterpret_cast<uintptr_t>(b->data) % 16 != 0) {
-        pl.v4 = false;
-    }
     const auto same_layout = [y](const shp_tensor * t) {
         return same_shape(*t, *y) && t->nb[1] == y->nb[1] && t->nb[2] == y->nb[2] && t->nb[3] == y->nb[3];
     };
@@ -1685,10 +1724,6 @@ extern "C" shp_status_t shp_cont_add_leaky_relu(const shp_tensor * x,
         (r != nullptr && r->data != y->data && !apart(r, y)) ||
         (r != nullptr && sum != nullptr && r->data != sum->data && !apart(r, sum))) {
         return SHP_ERR_UNSUPPORTED;
-    }
-    if ((r != nullptr && reinterpret_cast<uintptr_t>(r->data) % 16 != 0) ||
-        (sum != nullptr && reinterpret_cast<uintptr_t>(sum->data) % 16 != 0)) {
-        pl.v4 = false;
     }
     if (dry_run()) {
         return SHP_OK;
