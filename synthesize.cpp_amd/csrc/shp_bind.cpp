@@ -1,15 +1,18 @@
 // The calling side of the Python binding, for CPython: an entry point of
 // libsynth_hip as a Python callable that takes torch tensors.
 //
-//   bind(handle, name) -> callable(arg, ...) -> status
-//   describe(tensor)   -> the bytes of its shp_tensor
+//   bind(handle, name)  -> callable(arg, ...) -> status
+//   describe(tensor)    -> the bytes of its shp_tensor
+//   types(block, shape) names synth_hip.BlockTensor and its ctypes ShpTensor
 //
 // handle is the loaded library's dlopen handle (ctypes' CDLL._handle), so a
 // process may bind any build of the library. Each C parameter is converted
-// from its Python argument by its type: a tensor pointer from a torch tensor,
-// a synth_hip.BlockTensor, a ctypes ShpTensor or None (an array of them from a
-// list or tuple), numbers from numbers, a stream from its address. The GIL is
-// released while the entry point runs.
+// from its Python argument by its type: a tensor pointer from a torch tensor, a
+// BlockTensor or None, numbers from numbers, a stream from its address. Two
+// entry points start with an array of tensors and its length: there alone a list
+// or tuple is taken, of that length. shp_im2col starts with a kernel of which
+// only the shape is read: that is a ShpTensor too. The GIL is released while the
+// entry point runs.
 //
 // Why native: filling one descriptor field by field through ctypes takes 4 us
 // of Python, ten times an entry point's own host work, and a call has two to
@@ -40,6 +43,9 @@ PyObject * g_ne0  = nullptr;
 PyObject * g_type = nullptr;
 PyObject * g_size = nullptr;
 
+PyObject * g_block = nullptr;  // the classes named by types()
+PyObject * g_shape = nullptr;
+
 // shp_tensor for a torch tensor. Dimensions past the tensor's own have extent
 // 1 and the stride of everything below them.
 bool from_tensor(PyObject * o, shp_tensor & d) {
@@ -58,6 +64,7 @@ bool from_tensor(PyObject * o, shp_tensor & d) {
             d.type = SHP_TYPE_I32;
             break;
         case at::kByte:
+        case at::kChar:
             d.type = -1;  // raw blocks: the caller names the type
             break;
         default: {
@@ -117,21 +124,14 @@ bool to_tensor(PyObject * o, shp_tensor & d) {
         }
         return true;
     }
-    if (PyObject_CheckBuffer(o)) {  // a ctypes ShpTensor
-        Py_buffer b;
-        if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) {
-            return false;
+    const int block = g_block == nullptr ? 0 : PyObject_IsInstance(o, g_block);
+    if (block < 1) {
+        if (block == 0) {
+            PyErr_Format(PyExc_TypeError, "expected a tensor, got %s", Py_TYPE(o)->tp_name);
         }
-        const bool ok = b.len == static_cast<Py_ssize_t>(sizeof(shp_tensor));
-        if (ok) {
-            std::memcpy(&d, b.buf, sizeof(d));
-        } else {
-            PyErr_SetString(PyExc_TypeError, "expected a descriptor");
-        }
-        PyBuffer_Release(&b);
-        return ok;
+        return false;
     }
-    // BlockTensor: raw blocks (..., rows, ne0 / ELEMS * BYTES) with a logical row length
+    // raw blocks (..., rows, ne0 / ELEMS * BYTES) with a logical row length
     int64_t    ne0 = 0, type = 0, bytes = 0, nd = 0;
     PyObject * raw = PyObject_GetAttr(o, g_data);
     if (raw == nullptr) {
@@ -169,25 +169,66 @@ template <class T> struct Arg;
 
 template <> struct Arg<const shp_tensor *> {
     static bool get(PyObject * o, Slot & s, const shp_tensor *& v) {
-        if (o == Py_None) {
-            v = nullptr;
-            return true;
-        }
-        if (PyList_Check(o) || PyTuple_Check(o)) {
-            const Py_ssize_t n = PySequence_Fast_GET_SIZE(o);
-            s.many.resize(static_cast<size_t>(n));
-            for (Py_ssize_t i = 0; i < n; ++i) {
-                if (!to_tensor(PySequence_Fast_GET_ITEM(o, i), s.many[static_cast<size_t>(i)])) {
-                    return false;
-                }
-            }
-            v = s.many.data();
-            return true;
-        }
-        v = &s.one;
-        return to_tensor(o, s.one);
+        v = o == Py_None ? nullptr : &s.one;
+        return o == Py_None || to_tensor(o, s.one);
     }
 };
+
+// What an entry point's first parameter is beside a tensor.
+enum First { kTensor = 0, kArray = 1, kShape = 2 };
+
+// An array of tensors; the entry point reads as many as the parameter after it
+// says.
+bool array_arg(PyObject * o, PyObject * count, Slot & s, const shp_tensor *& v) {
+    if (!PyList_Check(o) && !PyTuple_Check(o)) {
+        PyErr_SetString(PyExc_TypeError, "expected a list of tensors");
+        return false;
+    }
+    PyObject * items = PySequence_Tuple(o);  // (a conversion may run Python code: a list could change under it)
+    if (items == nullptr) {
+        return false;
+    }
+    const Py_ssize_t n  = PyTuple_GET_SIZE(items);
+    const long long  c  = PyLong_AsLongLong(count);
+    bool             ok = !(c == -1 && PyErr_Occurred() != nullptr);
+    if (ok && c != n) {
+        PyErr_Format(PyExc_ValueError, "%zd tensors for a count of %lld", n, c);
+        ok = false;
+    }
+    try {
+        s.many.resize(static_cast<size_t>(n));
+        for (Py_ssize_t i = 0; ok && i < n; ++i) {
+            ok = to_tensor(PyTuple_GET_ITEM(items, i), s.many[static_cast<size_t>(i)]);
+        }
+    } catch (...) {
+        Py_DECREF(items);
+        throw;
+    }
+    Py_DECREF(items);
+    v = s.many.data();
+    return ok;
+}
+
+// A ctypes ShpTensor, for a parameter of which only the shape is read.
+bool shape_arg(PyObject * o, Slot & s, const shp_tensor *& v) {
+    const int shape = g_shape == nullptr ? 0 : PyObject_IsInstance(o, g_shape);
+    if (shape < 1) {
+        return shape == 0 && Arg<const shp_tensor *>::get(o, s, v);
+    }
+    Py_buffer b;
+    if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) {
+        return false;
+    }
+    const bool ok = b.len == static_cast<Py_ssize_t>(sizeof(shp_tensor));
+    if (ok) {
+        std::memcpy(&s.one, b.buf, sizeof(s.one));
+        v = &s.one;
+    } else {
+        PyErr_SetString(PyExc_TypeError, "expected a descriptor");
+    }
+    PyBuffer_Release(&b);
+    return ok;
+}
 
 template <> struct Arg<shp_tensor *> {
     static bool get(PyObject * o, Slot & s, shp_tensor *& v) {
@@ -252,13 +293,24 @@ bool counted(Py_ssize_t got, Py_ssize_t want) {
     return true;
 }
 
-template <class F> struct Call;
+template <class F, First FIRST> struct Call;
 
-template <class... A> struct Call<shp_status_t (*)(A...)> {
+template <First FIRST, class... A> struct Call<shp_status_t (*)(A...), FIRST> {
+    template <size_t I> static bool convert_one(PyObject * const * args, Slot & slot, std::tuple<A...> & vals) {
+        using T = std::tuple_element_t<I, std::tuple<A...>>;
+        if constexpr (I == 0 && FIRST == kArray) {
+            return array_arg(args[0], args[1], slot, std::get<0>(vals));
+        } else if constexpr (I == 0 && FIRST == kShape) {
+            return shape_arg(args[0], slot, std::get<0>(vals));
+        } else {
+            return Arg<T>::get(args[I], slot, std::get<I>(vals));
+        }
+    }
+
     template <size_t... I>
     static bool convert(PyObject * const * args, std::array<Slot, sizeof...(A)> & slots, std::tuple<A...> & vals,
                         std::index_sequence<I...>) {
-        return (Arg<A>::get(args[I], slots[I], std::get<I>(vals)) && ...);
+        return (convert_one<I>(args, slots[I], vals) && ...);
     }
 
     static PyObject * run(void * fn, PyObject * const * args, Py_ssize_t n) {
@@ -316,10 +368,11 @@ struct Entry {
     Runner       run;
 };
 
-#define SHP_ENTRY(f) { #f, &Call<decltype(&f)>::run }
+#define SHP_ENTRY_FIRST(f, first) { #f, &Call<decltype(&f), first>::run }
+#define SHP_ENTRY(f) SHP_ENTRY_FIRST(f, kTensor)
 
 const Entry kEntries[] = {
-    SHP_ENTRY(shp_get_rows), SHP_ENTRY(shp_get_rows_sum), SHP_ENTRY(shp_rms_norm_mul), SHP_ENTRY(shp_add_rms_norm_mul),
+    SHP_ENTRY(shp_get_rows), SHP_ENTRY_FIRST(shp_get_rows_sum, kArray), SHP_ENTRY(shp_rms_norm_mul), SHP_ENTRY(shp_add_rms_norm_mul),
     SHP_ENTRY(shp_rope_ext), SHP_ENTRY(shp_qk_norm_rope), SHP_ENTRY(shp_qk_norm_rope_kv),
     SHP_ENTRY(shp_qk_norm_rope_kv_at), SHP_ENTRY(shp_swiglu), SHP_ENTRY(shp_glu_swiglu), SHP_ENTRY(shp_snake),
     SHP_ENTRY(shp_snake_guarded), SHP_ENTRY(shp_snake_beta), SHP_ENTRY(shp_add_leaky_relu), SHP_ENTRY(shp_add),
@@ -329,9 +382,9 @@ const Entry kEntries[] = {
     SHP_ENTRY(shp_sqrt), SHP_ENTRY(shp_sum_rows), SHP_ENTRY(shp_mean), SHP_ENTRY(shp_mul_sum_rows),
     SHP_ENTRY(shp_inverse_stft), SHP_ENTRY(shp_harmonic_source), SHP_ENTRY(shp_log_mel), SHP_ENTRY(shp_concat),
     SHP_ENTRY(shp_col2im_1d), SHP_ENTRY(shp_pad), SHP_ENTRY(shp_pad_reflect_1d), SHP_ENTRY(shp_repeat),
-    SHP_ENTRY(shp_acc), SHP_ENTRY(shp_im2col), SHP_ENTRY(shp_cont_add_leaky_relu), SHP_ENTRY(shp_soft_max_ext),
+    SHP_ENTRY(shp_acc), SHP_ENTRY_FIRST(shp_im2col, kShape), SHP_ENTRY(shp_cont_add_leaky_relu), SHP_ENTRY(shp_soft_max_ext),
     SHP_ENTRY(shp_diag_mask_inf), SHP_ENTRY(shp_soft_max_causal), SHP_ENTRY(shp_exp), SHP_ENTRY(shp_scale_bias),
-    SHP_ENTRY(shp_sum_scale_leaky_relu), { "shp_layer_nongemm_step", &run_layer },
+    SHP_ENTRY_FIRST(shp_sum_scale_leaky_relu, kArray), { "shp_layer_nongemm_step", &run_layer },
 };
 
 struct Bound {
@@ -399,7 +452,21 @@ PyObject * describe(PyObject *, PyObject * o) {
     return nullptr;
 }
 
-PyMethodDef kMethods[] = { { "describe", describe, METH_O, "describe(tensor) -> the bytes of its shp_tensor" },
+PyObject * types(PyObject *, PyObject * args) {
+    PyObject * block = nullptr;
+    PyObject * shape = nullptr;
+    if (!PyArg_ParseTuple(args, "O!O!", &PyType_Type, &block, &PyType_Type, &shape)) {
+        return nullptr;
+    }
+    Py_INCREF(block);
+    Py_INCREF(shape);
+    Py_XSETREF(g_block, block);
+    Py_XSETREF(g_shape, shape);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef kMethods[] = { { "types", types, METH_VARARGS, "types(BlockTensor, ShpTensor)" },
+                           { "describe", describe, METH_O, "describe(tensor) -> the bytes of its shp_tensor" },
                            { "bind", bind, METH_VARARGS, "bind(handle, name) -> callable" },
                            { nullptr, nullptr, 0, nullptr } };
 

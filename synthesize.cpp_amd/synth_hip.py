@@ -210,6 +210,7 @@ def _binding():
         mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("shp_bind", BIND_PATH,
                                                                                     loader=loader))
         loader.exec_module(mod)
+        mod.types(BlockTensor, ShpTensor)
         _bind = mod
     return _bind
 
@@ -681,7 +682,7 @@ def kernel_shape(k, ic, oc=1):
     return d
 
 
-_kernel_shape = functools.lru_cache(maxsize=64)(kernel_shape)
+_kernel_shape = functools.lru_cache(maxsize=64, typed=True)(kernel_shape)     # (3.0 is not 3: it raises)
 
 
 def im2col(x, k, s0=1, p0=0, d0=1, dtype=None, out=None):
@@ -694,7 +695,7 @@ def im2col(x, k, s0=1, p0=0, d0=1, dtype=None, out=None):
         ow = conv_out_len(iw, k, s0, p0, d0)
         out = torch.empty((n_, max(ow, 1), ic * k), dtype=dtype or torch.float32, device=x.device)
     ic = x.shape[-2]
-    _check(_fn("shp_im2col")(_kernel_shape(int(k), int(ic)), x, int(s0), int(p0), int(d0),
+    _check(_fn("shp_im2col")(_kernel_shape(k, ic), x, int(s0), int(p0), int(d0),
                              out, _stream()), "im2col")
     return out
 

@@ -4,6 +4,7 @@ refuses, and the conversion of call arguments through entry points that refuse
 their arguments before touching a device."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
@@ -75,3 +76,51 @@ def test_calls():
     d = S.kernel_shape(3, 2)                            # a ctypes descriptor without data
     assert S._fn("shp_im2col")(d, a, 1, 0, 1, b, 0) != S.OK
     assert ctypes.sizeof(S.ShpTensor) == len(S._binding().describe(a))
+
+
+@pytest.mark.parametrize("name,args", [
+    ("shp_soft_max_ext", lambda a, bad: (a, bad, 1.0, 0.0, a, 0)),
+    ("shp_swiglu", lambda a, bad: (a, bad, a, 0)),
+    ("shp_swiglu", lambda a, bad: (bad, a, a, 0)),
+    ("shp_add", lambda a, bad: (a, bad, a, 0)),
+    ("shp_add", lambda a, bad: (a, a, bad, 0)),
+    ("shp_sum_rows", lambda a, bad: (bad, a, 0)),
+    ("shp_get_rows_sum", lambda a, bad: ([a, bad], 2, a, a, 0)),
+    ("shp_im2col", lambda a, bad: (bad if not isinstance(bad, S.ShpTensor) else [bad], a, 1, 0, 1, a, 0)),
+    ("shp_im2col", lambda a, bad: (S.kernel_shape(3, 2), bad, 1, 0, 1, a, 0)),
+    ("shp_layer_nongemm_step", lambda a, bad: (a,) * 18 + (bad, 1e-6, 1e6, 128, 0)),
+])
+def test_a_tensor_parameter_takes_nothing_but_a_tensor(name, args):
+    """A list or tuple (also of one tensor, or empty: no mask by mistake), a
+    descriptor, or any object with as many bytes as one, raises."""
+    a = torch.zeros(2, 8)
+    size = ctypes.sizeof(S.ShpTensor)
+    class Alike:
+        data, ne0, TYPE, BYTES = torch.zeros(2, 34, dtype=torch.uint8), 32, S.TYPE_Q8_0, 34
+    for bad in ([], (), [a], (a, a), [None], S.kernel_shape(8, 2), bytes(size), bytearray(size), np.zeros(size, np.uint8),
+                np.zeros((2, 8), np.float32), memoryview(bytes(size)), 3, "x", Alike()):
+        with pytest.raises(TypeError):
+            S._fn(name)(*args(a, bad))
+
+
+@pytest.mark.parametrize("name,rest", [("shp_get_rows_sum", lambda a: (a, a, 0)),
+                                       ("shp_sum_scale_leaky_relu", lambda a: (1.0, 0.1, None, a, 0))])
+def test_an_array_is_a_list_of_the_count_beside_it(name, rest):
+    a, f = torch.zeros(2, 8), S._fn(name)
+    for tables, n, exc in (([a], 2, ValueError), ([a, a], 1, ValueError), ([], 1, ValueError), ((a,), -1, ValueError),
+                           ([a], 2 ** 32 + 1, ValueError), ([a], "1", TypeError), ([a], None, TypeError),
+                           (a, 1, TypeError), (None, 1, TypeError), (iter([a]), 1, TypeError)):
+        with pytest.raises(exc):
+            f(tables, n, *rest(a))
+    b = torch.zeros(2, 8, dtype=torch.float16)              # refused for its type, after the conversion
+    assert f((b, b), 2, *rest(b)) not in (S.OK, S.ERR_BACKEND)
+
+
+def test_public_calls_refuse_what_is_no_tensor(monkeypatch):
+    monkeypatch.setattr(S, "_stream", lambda: 0)
+    a = torch.zeros(2, 8)
+    for call in (lambda: S.soft_max_ext(a, [], 1.0), lambda: S.soft_max_ext(a, [a, a], 1.0), lambda: S.swiglu(a, []),
+                 lambda: S.add(a, [a]), lambda: S.rms_norm_mul(a, (), 1e-6), lambda: S.qk_norm_rope(
+                     a, a, [], a, 1e-6, a, 8, 1e6), lambda: S.im2col(a, 3.0, out=a), lambda: S.get_rows_sum([a, [a]], a, out=a)):
+        with pytest.raises(TypeError):
+            call()
