@@ -83,3 +83,28 @@ def test_codec_encoder_attention_softmax_through_the_executor(gpu):
     g.compute(probs)
     two = _np(gpu.soft_max_ext(gpu.diag_mask_inf(_t(gpu, x), 0), None, scale))
     assert np.array_equal(_bits(_np(probs.t)), _bits(two))
+
+
+@pytest.mark.parametrize("H,T,N,n_past", [(1, 2048, 1025, 0), (1, 2050, 1028, 300), (2, 1100, 1100, 0), (2, 1101, 1101, 0),
+                                          (1, 2049, 2047, 0), (2, 1024, 2048, 1024), (1, 2100, 1537, 5)])
+def test_many_rows_of_1025_to_2048(gpu, H, T, N, n_past):
+    """From 2048 rows, at rows of several waves and at odd ones: bit-identical to
+    the two nodes, infinities and NaN in hidden scores included, and the
+    softmax alone and with a mask tensor within its bound (at most 3 ulp, as
+    test_gpu_softmax_rows.py derives it, > 99 % identical) of the restatement."""
+    rng = np.random.default_rng([SEED, H, T, N])
+    x = (rng.standard_normal((H, T, N)) * 4).astype(np.float32)
+    hidden = np.broadcast_to(np.arange(N)[None, :] > n_past + np.arange(T)[:, None], x.shape)
+    x[hidden] = np.resize(np.float32([np.nan, 1.0, np.inf, -np.inf, 3e38]), int(hidden.sum()))
+    scale = np.float32(1.0 / np.sqrt(64.0))
+    tx = _t(gpu, x)
+    fused = _np(gpu.soft_max_causal(tx, n_past, scale))
+    two = _np(gpu.soft_max_ext(gpu.diag_mask_inf(tx, n_past), None, scale))
+    assert np.array_equal(_bits(fused), _bits(two)) and np.isfinite(fused).all()
+    x[hidden] = 0.5
+    m = np.where(rng.random((T, N)) < 0.3, -np.inf, rng.standard_normal((T, N))).astype(np.float32)
+    m[:, 0] = 0.0
+    for mask in (None, m):
+        got = _np(gpu.soft_max_ext(_t(gpu, x), None if mask is None else _t(gpu, mask), scale))
+        d = _ulps_apart(got, R.run(lambda g: g.soft_max_ext(x, mask, scale)))
+        assert d.max() <= 3 and (d == 0).mean() > 0.99
