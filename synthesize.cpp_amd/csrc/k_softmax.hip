@@ -21,8 +21,8 @@
 // length has odd rows): one wave per row (wave-level reductions only: no LDS,
 // no barrier) where the rows fill the chip, more where they are few or long
 // (the decode step's 16 rows, a short prefill). Longer rows take one block and
-// three passes over the row; rows of up to 128 scores a wave and an element per
-// lane at a time.
+// three passes over the row; rows of up to 128 scores, and odd ones up to 512 of
+// which there are not many, a wave and an element per lane at a time.
 
 #include <cmath>
 
@@ -104,9 +104,9 @@ template <int MK> __device__ __forceinline__ void softmax_args_in_sgprs(const So
     }
 }
 
-// One wave per row of up to 64 K scores (K at most 2), element lane + 64k in
-// register k: a lane then has one or two exps in its chain, not a float4's four
-// (a decode step's 16 rows of 38: 1.71 us, 2.04 by float4).
+// One wave per row of up to 64 K scores (K at most 8), element lane + 64k in
+// register k: a short row's lane then has one or two exps in its chain, not a
+// float4's four (a decode step's 16 rows of 38: 1.71 us, 2.04 by float4).
 template <int K, int MK> __global__ __launch_bounds__(256) void k_soft_max_wave(const SoftMaxArgs a) {
     constexpr bool MASK = MK == kMaskTensor;
     __shared__ double s_tab[256 / kWave][64];
@@ -414,9 +414,9 @@ template <int MK> __global__ __launch_bounds__(kSoftMaxBlock) void k_soft_max_bl
     }
 }
 
-// The form depends on the row count and length only, not on the mask: the causal
-// launch adds a row in the order that the softmax alone does, so diag_mask_inf
-// and soft_max_ext come out bit for bit the same in one launch.
+// The forms' rule reads only the row count and length, so that the causal launch
+// adds a row in the order that the softmax alone does: diag_mask_inf and
+// soft_max_ext come out bit for bit the same in one launch.
 template <int MK, bool ODD, class Go> shp_status_t launch_rows4(const SoftMaxArgs & a, const Go & go) {
     const int nc = (a.ne0 + 3) / 4;
     if (nc <= 64) {
@@ -426,7 +426,9 @@ template <int MK, bool ODD, class Go> shp_status_t launch_rows4(const SoftMaxArg
     // row. The decode step's 16 rows of 512 take one wave each (2.30 us
     // against 2.36 us with two waves and their LDS combine, MI355X), in
     // one-wave blocks: each row on its own CU (2.12 -> 1.99 us warm; the
-    // 28-layer decode graph's layer with the softmax 9.62 -> 9.45 us).
+    // 28-layer decode graph's layer with the softmax 9.62 -> 9.45 us). Rows
+    // of 513-1023 scores: four waves, odd ones below 1024 rows (16 of 601: 2.85
+    // us, one wave 3.2, two 3.0; 1024: 4.6, 4.2, 4.4), whole ones up to 64.
     if (a.nrows < 2048 && nc >= 128) {
         if (nc >= 256) {
             if (a.nrows <= 256 && nc > 512) {
@@ -440,7 +442,10 @@ template <int MK, bool ODD, class Go> shp_status_t launch_rows4(const SoftMaxArg
                    nc <= 2048 ? go(k_soft_max_rows4<4, 8, MK, ODD>, 1, 256) :
                                 go(k_soft_max_rows4<16, 4, MK, ODD>, 1, 1024);
         }
-        if (a.nrows > 64) {
+        if (nc > 128 && a.nrows < (ODD ? 1024 : 65)) {
+            return go(k_soft_max_rows4<4, 1, MK, ODD>, 1, 256);
+        }
+        if (!ODD && a.nrows > 64) {
             return nc <= 128 ? go(k_soft_max_rows4<2, 1, MK, ODD>, 2, 256) : go(k_soft_max_rows4<2, 2, MK, ODD>, 2, 256);
         }
     }
@@ -450,13 +455,22 @@ template <int MK, bool ODD, class Go> shp_status_t launch_rows4(const SoftMaxArg
                                go(k_soft_max_rows4<1, 2, MK, ODD>, 4, 256);
     }
     // Many rows: one wave up to 1024 scores, two up to 2048 (8 heads of 2000 x
-    // 2000, one wave / two / four, MI355X: no mask 46.3 us / 44.5 / 45.1, with a
-    // mask 57.1 / 49.8 / 50.4, causal 39.6 / 35.8 / 40.2; 16 of 1100 x 1100: 36.5 /
-    // 38.5 / 41.8, 41.7 / 40.4 / 45.2, 26.4 / 26.8 / 32.8).
+    // 2000, one wave / two / four: no mask 46.3 us / 44.5 / 45.1, with a mask 57.1
+    // / 49.8 / 50.4, causal 39.6 / 35.8 / 40.2; 16 of 1100 x 1100: 36.5 / 38.5 /
+    // 41.8, 41.7 / 40.4 / 45.2, 26.4 / 26.8 / 32.8).
     return nc <= 256  ? go(k_soft_max_rows4<1, 4, MK, ODD>, 4, 256) :
            nc <= 512  ? go(k_soft_max_rows4<2, 4, MK, ODD>, 2, 256) :
            nc <= 1024 ? go(k_soft_max_rows4<4, 4, MK, ODD>, 1, 256) :
            nc <= 2048 ? go(k_soft_max_rows4<4, 8, MK, ODD>, 1, 256) : go(k_soft_max_rows4<16, 4, MK, ODD>, 1, 1024);
+}
+
+// Up to 128 scores, and odd rows up to 512 where a wave each leaves the chip
+// room, an element per lane at a time: the last float4 of an odd row costs a
+// lane four exps for its one to three scores (16 rows of 301, MI355X: 2.53 us,
+// 2.82 by float4; 1024: 3.0 and 3.6; 2048: 3.6 and 4.1; but 16384: 13.0 and
+// 12.2; of 511, 2048: 4.3 and 4.4, 4096: 6.9 and 5.7).
+inline bool by_elements(const SoftMaxArgs & a) {
+    return a.ne0 <= 2 * kWave || (a.ne0 % 4 != 0 && a.ne0 <= 8 * kWave && a.nrows <= (a.ne0 <= 5 * kWave ? 4096 : 2048));
 }
 
 template <int MK> shp_status_t launch_soft_max(const SoftMaxArgs & a, hipStream_t stream) {
@@ -468,8 +482,12 @@ template <int MK> shp_status_t launch_soft_max(const SoftMaxArgs & a, hipStream_
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(block), 0, stream, a);
         return launch_status();
     };
-    if (a.ne0 <= 2 * kWave) {
-        return a.ne0 <= kWave ? go(k_soft_max_wave<1, MK>, 4, 256) : go(k_soft_max_wave<2, MK>, 4, 256);
+    if (by_elements(a)) {
+        return a.ne0 <= 1 * kWave ? go(k_soft_max_wave<1, MK>, 4, 256) :
+               a.ne0 <= 2 * kWave ? go(k_soft_max_wave<2, MK>, 4, 256) :
+               a.ne0 <= 3 * kWave ? go(k_soft_max_wave<3, MK>, 4, 256) :
+               a.ne0 <= 4 * kWave ? go(k_soft_max_wave<4, MK>, 4, 256) :
+               a.ne0 <= 6 * kWave ? go(k_soft_max_wave<6, MK>, 4, 256) : go(k_soft_max_wave<8, MK>, 4, 256);
     }
     if (a.ne0 > kSoftMaxRegs) {
         return go(k_soft_max_block<MK>, 1, kSoftMaxBlock);

@@ -74,3 +74,11 @@ def test_causal_with_hidden_infinities(gpu, heads, rows, n, past):
     hidden = np.broadcast_to(np.isinf(masked), x.shape)
     x[hidden] = np.resize(np.float32([np.nan, np.inf, 3e38]), int(hidden.sum()))
     assert np.array_equal(_np(gpu.soft_max_causal(_t(gpu, x), past, 0.25)).view(np.uint32), clean.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [129, 191, 193, 301, 321, 383, 385, 509, 511])
+@pytest.mark.parametrize("rows", [1, 2048, 4096, 4097])
+def test_short_odd_rows(gpu, n, rows):
+    """Either side of the row counts from which they go by float4."""
+    x = (np.random.default_rng([SEED, rows, n]).standard_normal((1, rows, n)) * 4).astype(np.float32)
+    _close(_np(gpu.soft_max_ext(_t(gpu, x), None, 0.5)), R.run(lambda g: g.soft_max_ext(x, None, np.float32(0.5))))

@@ -34,3 +34,16 @@ def test_the_causal_softmax_takes_the_form_of_the_softmax_alone():
             del args[mask[kind]]
             forms.append((kind, args, grid, block))
         assert forms[0] == forms[1] == forms[2], calls[i]
+
+
+def _kernels(calls):
+    got = record(calls)
+    assert all(st == 0 for st, _ in got)
+    return [[n for n, *_ in ls] for _, ls in got]
+
+
+def test_short_odd_softmax_rows_go_by_elements_while_they_are_few():
+    sizes = [(16, 129), (1024, 201), (4096, 319), (2048, 321), (1, 511), (4097, 319), (2049, 321), (2049, 511), (16, 513),
+             (16, 300), (100000, 129)]
+    names = _kernels([("shp_soft_max_ext", t(n, rows), None, 0.5, 0.0, t(n, rows)) for rows, n in sizes])
+    assert ["k_soft_max_wave" in k[0] for k in names] == [True] * 5 + [False] * 6
