@@ -525,15 +525,55 @@ template <int K> __global__ __launch_bounds__(256) void k_snake_rows(const EwArg
     }
 }
 
-// Row path: any ggml byte strides. Blocks take rows (x) and runs of
-// kEwRowRun elements of them (y), so that a few long rows fill the chip too;
-// one float4 per lane from any 4-byte boundary, the row's last one to three
-// elements one per lane. A value added to each of 96 strided rows of 24001:
-// 43.9 -> 6.0 us against a block per row and 4-byte accesses (MI355X, cold).
-constexpr int kEwRowRun = 256 * 4;
+// Row path: any ggml byte strides. Blocks take rows (x) and, where the rows are
+// few, runs of them (y), so that a few long rows fill the chip too; one float4
+// per lane from any 4-byte boundary, the row's last one to three elements one
+// per lane, loaded ahead of the float4. A value added to each of 96 strided
+// rows of 24001: 43.9 -> 6.0 us against a block per row and 4-byte accesses
+// (MI355X, cold). Rows of up to a wave's or two waves' float4 take blocks of one
+// or two waves, and those of up to 64 elements, or few rows of up to 512, an
+// element per lane at a time (RowShape): 100000 strided rows of 6 16.8 us, of 128
+// with a value each 28.9, against 42.3 and 76.0 for four waves a row.
+constexpr int kEwRowRun  = 256 * 4;
+constexpr int kEwRowFull = 1024;  // rows that fill the chip with a block each (four per CU)
+constexpr int kEwRowMany = 8192;  // ... and beyond which the longest are not split
 
-template <int OP, bool HAS_B, bool BCAST, bool HAS_S> __global__ __launch_bounds__(256) void k_ew_rows(const EwArgs a) {
-    const int n4 = a.ne0 / 4;
+// A row kernel's threads per block, float4 per row (the rest of a row goes by
+// elements) and grid: every row up to 65536, and of few or long rows their runs,
+// up to kMaxFlatBlocks blocks (the kernels stride over what is left). Split
+// rows, MI355X: 2000 of 12001 39.4 us, whole 42.3; but 20000 SwiGLU rows of 2000
+// 75.6 whole, 82.3 in two runs. Few rows by elements: 300 strided rows of 512 2.41
+// us, 2.78 by float4; 1000 SwiGLU rows of 512 3.42 by float4, 3.88 by elements.
+struct RowShape {
+    int  block;
+    int  n4;
+    dim3 grid;
+
+    RowShape(int64_t nrows, int64_t ne0) {
+        const bool    few      = nrows <= kEwRowFull;
+        const bool    elements = ne0 <= kWave || (few && ne0 <= 256) || (nrows <= kEwRowFull / 2 && ne0 <= 2 * 256);
+        const int64_t quads    = ne0 / 4;
+        block = ne0 <= kWave ? kWave : elements || quads > 2 * kWave ? 256 : quads > kWave ? 2 * kWave : kWave;
+        n4    = elements ? 0 : static_cast<int>(quads);
+        const int64_t x     = nrows < 65536 ? nrows : 65536;
+        const bool    split = few ? !elements : nrows <= kEwRowMany && ne0 > 2 * kEwRowRun;
+        const int64_t runs  = split ? (ne0 + kEwRowRun - 1) / kEwRowRun : 1;
+        const int64_t most  = kMaxFlatBlocks / x < 65535 ? kMaxFlatBlocks / x : 65535;
+        grid                = dim3(static_cast<unsigned>(x), static_cast<unsigned>(runs < most ? runs : most));
+    }
+
+    // go(the block size as a constant)
+    template <class F> shp_status_t with_block(const F & go) const {
+        return block == kWave ? go(std::integral_constant<int, kWave>{}) :
+               block == 256   ? go(std::integral_constant<int, 256>{}) : go(std::integral_constant<int, 2 * kWave>{});
+    }
+};
+
+template <int OP, bool HAS_B, bool BCAST, bool HAS_S, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_ew_rows(const EwArgs a, int n4) {
+    const bool tail = blockIdx.y == 0 && static_cast<int>(threadIdx.x) < a.ne0 - n4 * 4;
+    const int  e    = n4 * 4 + (tail ? static_cast<int>(threadIdx.x) : 0);
+    const int  step = static_cast<int>(gridDim.y) * BLOCK;
     for (int64_t r = blockIdx.x; r < a.nrows; r += gridDim.x) {
         const float * ar = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.a) + row_offset(a.am, r));
         const float * br = nullptr;
@@ -545,37 +585,39 @@ template <int OP, bool HAS_B, bool BCAST, bool HAS_S> __global__ __launch_bounds
         if constexpr (HAS_S) {
             sr = reinterpret_cast<float *>(reinterpret_cast<char *>(a.s) + row_offset(a.sm, r));
         }
-        const int64_t step = static_cast<int64_t>(gridDim.y) * 256;
-        for (int64_t c = static_cast<int64_t>(blockIdx.y) * 256 + threadIdx.x; c < n4; c += step) {
-            const f32x4 av = ld_stream4u(ar + c * 4);
+        float ta = 0.0f, tb = 0.0f;
+        if (tail) {
+            ta = ar[e];
+            tb = HAS_B ? br[e] : 0.0f;
+        }
+        for (int c = static_cast<int>(blockIdx.y) * BLOCK + static_cast<int>(threadIdx.x); c < n4; c += step) {
+            const f32x4 av = ld_stream4u(ar + static_cast<int64_t>(c) * 4);
             f32x4       bv = splat4(0.0f);
             if constexpr (HAS_B) {
-                bv = BCAST ? ld4u(br + c * 4) : ld_stream4u(br + c * 4);
+                bv = BCAST ? ld4u(br + static_cast<int64_t>(c) * 4) : ld_stream4u(br + static_cast<int64_t>(c) * 4);
             }
             f32x4 sv = splat4(0.0f);
-            st_stream4u(yr + c * 4, ew4<OP>(av, bv, a, sv));
+            st_stream4u(yr + static_cast<int64_t>(c) * 4, ew4<OP>(av, bv, a, sv));
             if constexpr (HAS_S) {
-                st_stream4u(sr + c * 4, sv);
+                st_stream4u(sr + static_cast<int64_t>(c) * 4, sv);
             }
         }
-        if (blockIdx.y == 0 && static_cast<int>(threadIdx.x) < a.ne0 % 4) {
-            const int e  = n4 * 4 + static_cast<int>(threadIdx.x);
-            float     sv = 0.0f;
-            yr[e]        = ew<OP>(ar[e], HAS_B ? br[e] : 0.0f, a, sv);
+        if (tail) {
+            float sv = 0.0f;
+            yr[e]    = ew<OP>(ta, tb, a, sv);
             if constexpr (HAS_S) {
                 sr[e] = sv;
             }
+            if (BLOCK == 256 && a.ne0 - e > BLOCK) {  // by elements, two per lane
+                ta = ar[e + BLOCK];
+                tb = HAS_B ? br[e + BLOCK] : 0.0f;
+                yr[e + BLOCK] = ew<OP>(ta, tb, a, sv);
+                if constexpr (HAS_S) {
+                    sr[e + BLOCK] = sv;
+                }
+            }
         }
     }
-}
-
-// The row kernels' grid: every row up to 65536, then the rows' runs up to
-// kMaxFlatBlocks blocks (the kernels stride over what is left).
-inline dim3 row_grid(int64_t nrows, int64_t ne0) {
-    const int64_t x    = nrows < 65536 ? nrows : 65536;
-    const int64_t runs = (ne0 + kEwRowRun - 1) / kEwRowRun;
-    const int64_t most = kMaxFlatBlocks / x < 65535 ? kMaxFlatBlocks / x : 65535;
-    return dim3(static_cast<unsigned>(x), static_cast<unsigned>(runs < most ? runs : most));
 }
 
 // Branch average: summed = t0 + t1 + ... (in term order), current =
@@ -712,8 +754,11 @@ shp_status_t launch_ew(const EwArgs & a, bool flat, hipStream_t stream) {
         }
         return launch_status();
     }
-    hipLaunchKernelGGL((k_ew_rows<OP, HAS_B, BCAST, HAS_S>), row_grid(a.nrows, a.ne0), dim3(256), 0, stream, a);
-    return launch_status();
+    const RowShape shape(a.nrows, a.ne0);
+    return shape.with_block([&](auto block) {
+        hipLaunchKernelGGL((k_ew_rows<OP, HAS_B, BCAST, HAS_S, block()>), shape.grid, dim3(block()), 0, stream, a, shape.n4);
+        return launch_status();
+    });
 }
 
 // Common argument set-up. `b` may be null, may match `a`'s shape, or (when
@@ -1030,26 +1075,30 @@ template <int OP, bool FLAT, int BLOCK, bool ODD> __global__ __launch_bounds__(B
     }
 }
 
-// Any repeat form and any row strides, on k_ew_rows' grid. COL: one value of b
-// per row of a, one float4 per lane; otherwise one element per lane.
-template <int OP, bool COL> __global__ __launch_bounds__(256) void k_repeat_rows(const RepeatArgs g) {
+// Any repeat form and any row strides, in k_ew_rows' shapes. COL: one
+// value of b per row of a, one float4 per lane; otherwise one element per lane.
+template <int OP, bool COL, int BLOCK> __global__ __launch_bounds__(BLOCK) void k_repeat_rows(const RepeatArgs g, int n4) {
+    const bool tail = COL && blockIdx.y == 0 && static_cast<int>(threadIdx.x) < g.ne0 - n4 * 4;
+    const int  e    = n4 * 4 + (tail ? static_cast<int>(threadIdx.x) : 0);
+    const int  step = static_cast<int>(gridDim.y) * BLOCK;
+    const int  i0   = static_cast<int>(blockIdx.y) * BLOCK + static_cast<int>(threadIdx.x);
     for (int64_t r = blockIdx.x; r < g.nrows; r += gridDim.x) {
         const float * ar = reinterpret_cast<const float *>(reinterpret_cast<const char *>(g.a) + row_offset(g.am, r));
         float *       yr = reinterpret_cast<float *>(reinterpret_cast<char *>(g.y) + row_offset(g.ym, r));
         const float * br = reinterpret_cast<const float *>(g.b + repeat_row(g, static_cast<uint32_t>(r)));
-        const int64_t step = static_cast<int64_t>(gridDim.y) * 256;
-        const int64_t i0   = static_cast<int64_t>(blockIdx.y) * 256 + threadIdx.x;
         if constexpr (COL) {
             const float bv = *br;
-            const int   n4 = g.ne0 / 4;
-            for (int64_t c = i0; c < n4; c += step) {
-                const f32x4 av = ld_stream4u(ar + c * 4);
-                st_stream4u(yr + c * 4, f32x4{ binop<OP>(av.x, bv), binop<OP>(av.y, bv), binop<OP>(av.z, bv),
-                                               binop<OP>(av.w, bv) });
+            const float ta = tail ? ar[e] : 0.0f;
+            for (int c = i0; c < n4; c += step) {
+                const f32x4 av = ld_stream4u(ar + static_cast<int64_t>(c) * 4);
+                st_stream4u(yr + static_cast<int64_t>(c) * 4, f32x4{ binop<OP>(av.x, bv), binop<OP>(av.y, bv),
+                                                                     binop<OP>(av.z, bv), binop<OP>(av.w, bv) });
             }
-            if (blockIdx.y == 0 && static_cast<int>(threadIdx.x) < g.ne0 % 4) {
-                const int e = n4 * 4 + static_cast<int>(threadIdx.x);
-                yr[e]       = binop<OP>(ar[e], bv);
+            if (tail) {
+                yr[e] = binop<OP>(ta, bv);
+                if (BLOCK == 256 && g.ne0 - e > BLOCK) {  // by elements, two per lane
+                    yr[e + BLOCK] = binop<OP>(ar[e + BLOCK], bv);
+                }
             }
         } else {
             for (int64_t i = i0; i < g.ne0; i += step) {
@@ -1121,12 +1170,15 @@ shp_status_t repeat_entry(const shp_tensor * a, const shp_tensor * b, shp_tensor
         return odd ? go(k_repeat_col<OP, false, 256, true>, k_repeat_col<OP, false, kWave, true>) :
                      go(k_repeat_col<OP, false, 256, false>, k_repeat_col<OP, false, kWave, false>);
     }
-    if (b->ne[0] == 1) {
-        hipLaunchKernelGGL((k_repeat_rows<OP, true>), row_grid(rows, a->ne[0]), dim3(256), 0, ss, g);
-    } else {
-        hipLaunchKernelGGL((k_repeat_rows<OP, false>), row_grid(rows, a->ne[0]), dim3(256), 0, ss, g);
+    const RowShape shape(rows, a->ne[0]);
+    if (b->ne[0] != 1) {
+        hipLaunchKernelGGL((k_repeat_rows<OP, false, 256>), shape.grid, dim3(256), 0, ss, g, 0);
+        return launch_status();
     }
-    return launch_status();
+    return shape.with_block([&](auto block) {
+        hipLaunchKernelGGL((k_repeat_rows<OP, true, block()>), shape.grid, dim3(block()), 0, ss, g, shape.n4);
+        return launch_status();
+    });
 }
 
 // ggml_add / ggml_mul / ggml_div: b the same shape as a, one row of ne0

@@ -47,3 +47,23 @@ def test_short_odd_softmax_rows_go_by_elements_while_they_are_few():
              (16, 300), (100000, 129)]
     names = _kernels([("shp_soft_max_ext", t(n, rows), None, 0.5, 0.0, t(n, rows)) for rows, n in sizes])
     assert ["k_soft_max_wave" in k[0] for k in names] == [True] * 5 + [False] * 6
+
+
+def test_narrow_rows_take_blocks_of_their_own_width():
+    """Strided rows, a value per row added and a row repeated: rows of up to a
+    wave's or two waves' float4 do not launch four waves each; few short rows go
+    by elements; a row is split over blocks only where the rows are few or long."""
+    #       rows, width, threads, blocks per row
+    shapes = [(100000, 1, 64, 1), (100000, 64, 64, 1), (100000, 65, 64, 1), (100000, 259, 64, 1), (100000, 260, 128, 1),
+              (100000, 515, 128, 1), (100000, 516, 256, 1), (1024, 65, 256, 1), (512, 512, 256, 1), (513, 512, 128, 1),
+              (1024, 513, 128, 1), (7, 64, 64, 1), (96, 24001, 256, 24), (2000, 12001, 256, 12), (20000, 12001, 256, 1),
+              (2000, 2000, 256, 1)]
+    def calls(rows, n):
+        x, y, pad = t(n, rows, nb=[4, 4 * n + 12]), t(n, rows), t(n, rows, nb=[4, 4 * n + 4])
+        return [("shp_sqr", x, pad), ("shp_add", y, t(n), pad), ("shp_add", x, t(1, rows), y),
+                ("shp_glu_swiglu", t(2 * n, rows), 0, y)]
+    got = record([c for rows, n, *_ in shapes for c in calls(rows, n)])
+    for i, (rows, n, block, runs) in enumerate(shapes):
+        for st, ls in got[4 * i:4 * i + 4]:
+            assert st == 0 and len(ls) == 1 and "_rows" in ls[0][0]
+            assert (ls[0][2], ls[0][1]) == ((block, 1, 1), (min(rows, 65536), runs, 1)), (rows, n, ls)
