@@ -284,13 +284,14 @@ template <int TPR> __device__ __forceinline__ double row_sum(double v, double * 
 //
 // HBM-bound: x read once and y written once. A row stays in the registers of
 // the TPR lanes that share it between the two reductions and the store, VPL
-// float4 each (the last ne0 % 4 values one per lane), so both reductions and
-// the store run from one pass over memory. Rows of odd length start on any
+// float4 each (the last ne0 % 4 values, with VPL 0 all, one per lane), so both
+// reductions and the store run from one pass over memory. Rows of odd length start on any
 // 4-byte boundary: the 16-byte accesses are the unaligned form. Measured on
 // MI355X (cold) against one wave per row reading the row three times with
 // 4-byte accesses: 128 rows of 24001 253 -> 8.3 us, 256 of 4001 43 -> 4.5,
 // 1000 of 1024 13.2 -> 4.0, 8192 of 1024 28.2 -> 13.5, 300 of 8192 87.6 -> 5.7,
-// 64 of 65536 646 -> 12.5.
+// 64 of 65536 646 -> 12.5. Rows of up to 64 have no float4: 100000 of 6 25.5 us,
+// 33.5 with one.
 template <int TPR, int VPL> __global__ __launch_bounds__(TPR > 256 ? TPR : 256) void k_layer_norm(const NormArgs a) {
     constexpr int     kBlock = TPR > 256 ? TPR : 256;
     __shared__ double s_mean[kBlock / kWave], s_var[kBlock / kWave];
@@ -298,11 +299,11 @@ template <int TPR, int VPL> __global__ __launch_bounds__(TPR > 256 ? TPR : 256) 
     const int64_t     row  = static_cast<int64_t>(blockIdx.x) * (kBlock / TPR) + row_in_block<TPR>();
     const bool        live = row < a.nrows;
     const int64_t     rr   = live ? row : 0;
-    const int         n4   = live ? a.ne0 / 4 : 0;
-    const int         tail = live ? a.ne0 % 4 : 0;
+    const int         n4   = live && VPL > 0 ? a.ne0 / 4 : 0;
+    const int         tail = live ? (VPL > 0 ? a.ne0 % 4 : a.ne0) : 0;
     const float *     xr = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, rr));
     float *           yr = reinterpret_cast<float *>(reinterpret_cast<char *>(a.y) + row_offset(a.ym, rr));
-    f32x4             v[VPL];
+    f32x4             v[VPL > 0 ? VPL : 1];
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
         const int c = l + TPR * k;
@@ -401,6 +402,9 @@ shp_status_t launch_layer_norm(const NormArgs & a, hipStream_t stream) {
         hipLaunchKernelGGL(k_layer_norm_wide, dim3(static_cast<unsigned>(a.nrows)), dim3(kLayerNormWide), 0, stream, a);
         return launch_status();
     }
+    if (a.ne0 <= 64) {
+        return go(k_layer_norm<64, 0>, 64);
+    }
     if (n4 <= 64) {
         return go(k_layer_norm<64, 1>, 64);
     }
@@ -450,36 +454,64 @@ struct SumRowsArgs {
     int32_t       pad;
 };
 
-template <int MODE, int TPR> __global__ __launch_bounds__(TPR > 256 ? TPR : 256) void k_sum_rows(const SumRowsArgs a) {
+// VPL: float4 of a row that a lane loads before it adds them (0: none, a row of
+// one or two elements per lane).
+template <int MODE, int TPR, int VPL> __global__ __launch_bounds__(TPR > 256 ? TPR : 256) void k_sum_rows(const SumRowsArgs a) {
     constexpr int     kBlock = TPR > 256 ? TPR : 256;
     __shared__ double s_part[kBlock / kWave];
     const int         l    = static_cast<int>(threadIdx.x) % TPR;
     const int64_t     row  = static_cast<int64_t>(blockIdx.x) * (kBlock / TPR) + row_in_block<TPR>();
     const bool        live = row < a.nrows;
     const int64_t     rr   = live ? row : 0;
-    const int         n4   = live ? a.ne0 / 4 : 0;
-    const int         tail = live ? a.ne0 % 4 : 0;
+    const int         n4   = live && VPL > 0 ? a.ne0 / 4 : 0;
+    const int         tail = live ? (VPL > 0 ? a.ne0 % 4 : a.ne0) : 0;
     const float *     xr = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, rr));
     const float *     wr = MODE == kMulSumRows ?
                                reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.w) + row_offset(a.wm, rr)) :
                                nullptr;
-    double            acc = 0.0;
-#pragma unroll 4
-    for (int c = l; c < n4; c += TPR) {
-        f32x4 v = ld_stream4u(xr + c * 4);
-        if constexpr (MODE == kMulSumRows) {
-            const f32x4 u = ld_stream4u(wr + c * 4);
-            v             = f32x4{ v.x * u.x, v.y * u.y, v.z * u.z, v.w * u.w };
+    // the elements past the float4, at most two per lane
+    constexpr int kTail = VPL > 0 ? 1 : 2;
+    float         tv[kTail], tw[kTail];
+#pragma unroll
+    for (int k = 0; k < kTail; ++k) {
+        tv[k] = 0.0f;
+        tw[k] = 0.0f;
+        if (l + TPR * k < tail) {
+            tv[k] = xr[n4 * 4 + l + TPR * k];
+            tw[k] = MODE == kMulSumRows ? wr[n4 * 4 + l + TPR * k] : 0.0f;
         }
-        acc += static_cast<double>(v.x);
-        acc += static_cast<double>(v.y);
-        acc += static_cast<double>(v.z);
-        acc += static_cast<double>(v.w);
     }
-    if (l < tail) {
-        const int   i = n4 * 4 + l;
-        const float v = MODE == kMulSumRows ? xr[i] * wr[i] : xr[i];
-        acc += static_cast<double>(v);
+    double acc = 0.0;
+    if constexpr (VPL > 0) {
+        for (int c0 = l; c0 < n4; c0 += TPR * VPL) {
+            f32x4 v[VPL], u[VPL];
+#pragma unroll
+            for (int k = 0; k < VPL; ++k) {
+                const int64_t i = (static_cast<int64_t>(c0) + TPR * k) * 4;
+                v[k]            = splat4(0.0f);
+                u[k]            = splat4(0.0f);
+                if (c0 + TPR * k < n4) {
+                    v[k] = ld_stream4u(xr + i);
+                    if constexpr (MODE == kMulSumRows) {
+                        u[k] = ld_stream4u(wr + i);
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < VPL; ++k) {  // (past the row's end: 0)
+                if constexpr (MODE == kMulSumRows) {
+                    v[k] = f32x4{ v[k].x * u[k].x, v[k].y * u[k].y, v[k].z * u[k].z, v[k].w * u[k].w };
+                }
+                acc += static_cast<double>(v[k].x);
+                acc += static_cast<double>(v[k].y);
+                acc += static_cast<double>(v[k].z);
+                acc += static_cast<double>(v[k].w);
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kTail; ++k) {
+        acc += static_cast<double>(MODE == kMulSumRows ? tv[k] * tw[k] : tv[k]);  // (past the row's end: 0)
     }
     acc = row_sum<TPR>(acc, s_part);
     if (live && l == 0) {
@@ -491,18 +523,34 @@ template <int MODE, int TPR> __global__ __launch_bounds__(TPR > 256 ? TPR : 256)
     }
 }
 
-// One wave per row fills the chip from 2048 rows (8 waves per CU); fewer rows
-// take 256 lanes each, and up to one row per CU 1024.
+// One wave per row fills the chip from 2048 rows (8 waves per CU) and holds rows
+// of up to 1024 in one batch of loads; fewer long rows take 256 lanes each, and up
+// to one row per CU 1024. Rows of up to 128 go by elements: by float4 the last
+// ones of an odd row are a load of their own behind it (100000 rows of 6 21.5
+// us, of 63 22.9; 13.0 and 16.3 by elements; 20000 of 65 6.8 and 4.6).
 template <int MODE> shp_status_t launch_sum_rows(const SumRowsArgs & a, hipStream_t stream) {
     const int n4 = a.ne0 / 4;
-    if (n4 <= 64 || a.nrows >= 2048) {
-        hipLaunchKernelGGL((k_sum_rows<MODE, 64>), dim3(static_cast<unsigned>((a.nrows + 3) / 4)), dim3(256), 0, stream, a);
-    } else if (n4 <= 512 || a.nrows > kLayerNormFewRows) {
-        hipLaunchKernelGGL((k_sum_rows<MODE, 256>), dim3(static_cast<unsigned>(a.nrows)), dim3(256), 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((k_sum_rows<MODE, 1024>), dim3(static_cast<unsigned>(a.nrows)), dim3(1024), 0, stream, a);
+    auto      go = [&](auto kernel, int rows_per_block, int block) {
+        const int64_t blocks = (a.nrows + rows_per_block - 1) / rows_per_block;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(block), 0, stream, a);
+        return launch_status();
+    };
+    if (a.ne0 <= 128) {
+        return go(k_sum_rows<MODE, 64, 0>, 4, 256);
     }
-    return launch_status();
+    if (n4 <= 64) {
+        return go(k_sum_rows<MODE, 64, 1>, 4, 256);
+    }
+    if (n4 <= 128) {
+        return go(k_sum_rows<MODE, 64, 2>, 4, 256);
+    }
+    if (n4 <= 256 || a.nrows >= 2048) {
+        return go(k_sum_rows<MODE, 64, 4>, 4, 256);
+    }
+    if (n4 <= 512 || a.nrows > kLayerNormFewRows) {
+        return n4 <= 1024 ? go(k_sum_rows<MODE, 256, 4>, 1, 256) : go(k_sum_rows<MODE, 256, 8>, 1, 256);
+    }
+    return go(k_sum_rows<MODE, 1024, 4>, 1, 1024);
 }
 
 template <int MODE> shp_status_t sum_rows_entry(const shp_tensor * x, const shp_tensor * w, shp_tensor * y,

@@ -67,3 +67,17 @@ def test_narrow_rows_take_blocks_of_their_own_width():
         for st, ls in got[4 * i:4 * i + 4]:
             assert st == 0 and len(ls) == 1 and "_rows" in ls[0][0]
             assert (ls[0][2], ls[0][1]) == ((block, 1, 1), (min(rows, 65536), runs, 1)), (rows, n, ls)
+
+
+def test_short_row_sums_and_norms_go_by_elements():
+    """Up to 128 elements a row sum, up to 64 a norm: no float4 (the last template
+    argument), whatever their count; a row of up to 1024 is one wave's batch of loads."""
+    def last(name):
+        return int(re.findall(r"Li(\d+)E", name)[-1])
+    for rows in (1, 300, 2048, 100000):
+        for op, widths in (("shp_sum_rows", {1: 0, 7: 0, 64: 0, 127: 0, 128: 0, 129: 1, 259: 1, 260: 2, 515: 2, 516: 4, 1027: 4}),
+                           ("shp_norm", {1: 0, 6: 0, 63: 0, 64: 0, 65: 1, 259: 1})):
+            extra = (1e-5,) if op == "shp_norm" else ()
+            names = _kernels([(op, t(n, rows), *extra, t(n if extra else 1, rows)) for n in widths])
+            assert [last(k[0]) for k in names] == list(widths.values()), (op, rows, names)
+            assert op == "shp_norm" or all("Li64E" in k[0] for k in names)
