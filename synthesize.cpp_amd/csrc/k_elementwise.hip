@@ -1288,7 +1288,9 @@ struct TransposeArgs {
 constexpr int kTile0 = 64;
 constexpr int kTileK = 128;
 // Elements from which partly written lines are kept in L2: 128 x 24001 (12 MB)
-// 6.9 us streamed, 7.3 kept; 256 x 31999 (33 MB) 18.8 and 16.2 (MI355X, cold).
+// 6.9 us streamed, 7.3 kept; 256 x 31999 (33 MB) 18.8 and 16.2; rows of 2049: 1024
+// of them (8 MB) 5.5 and 6.0, 2048 (17 MB) 9.0 and 8.8, 8192 (67 MB) 47.3 and 33.3
+// (MI355X, cold).
 constexpr int64_t kTransposeKeep = int64_t{ 1 } << 22;
 
 // Epilogue bits: add the bias -- the destination row's value (kEpiBias) or
@@ -1504,10 +1506,19 @@ shp_status_t plan_transpose(const shp_tensor * x, const shp_tensor * y, Transpos
     // loads) end inside lines that the next tile along them takes up. Eight
     // consecutive blocks go to the eight XCDs, each with an L2 of its own, so
     // every XCD gets a run of consecutive tiles to share those lines in one L2;
-    // and of a large tensor the stores are not streamed past it.
+    // and of a large tensor the stores are not streamed past it. Not so where the
+    // other side's rows are whole lines and start a multiple of 4 KB apart (the
+    // loads'), or of 32 KB and the rows are many (the stores'): the XCDs' runs then
+    // meet on the same sets, which costs more than the shared lines. Runs against
+    // tiles in order (MI355X, cold): x rows of 6145 and y rows of 4099, 0.88; of 6400
+    // and 4099, 0.95; but of 4096 and 4099, 1.21; of 8192 and 8193, 1.45; y rows of 8192
+    // and x rows of 513, 0.89; of 1001, 1.00 (with sum and residual 1.10); of 4099,
+    // 1.24; y rows of 12000 and x rows of 4099, 0.96.
     const auto lines  = [](const void * p, int64_t ne, int64_t nb) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && (ne == 1 || nb % 128 == 0); };
     const bool ylines = lines(y->data, a.nek, a.ynbk);
-    a.perxcd          = ylines && lines(x->data, a.ne0, a.xnb0) ? 0 : static_cast<uint32_t>((nt + 7) / 8);
+    const bool xlines = lines(x->data, a.ne0, a.xnb0);
+    const bool sets   = (xlines && a.ne0 > 1 && a.xnb0 % 4096 == 0) || (ylines && a.nek > 768 && a.ynbk % 32768 == 0);
+    a.perxcd          = (xlines && ylines) || sets ? 0 : static_cast<uint32_t>((nt + 7) / 8);
     pl.keep           = !ylines && nelements(*y) >= kTransposeKeep;
     a.nblocks         = a.perxcd != 0 ? a.perxcd * 8 : a.ntiles;
     pl.grid           = a.nblocks < (1u << 20) ? a.nblocks : 1u << 20;

@@ -61,3 +61,14 @@ def test_large_copy(gpu):
     import torch
     x = torch.randn(30011, 143, device="cuda")
     assert torch.equal(gpu.cpy(x.t()), x.t().contiguous())
+
+
+@pytest.mark.parametrize("T,C", [(1027, 1024), (513, 4096), (8192, 771), (8192, 1025), (16384, 769)])
+def test_whole_rows_a_power_of_two_apart(gpu, T, C):
+    """One side's rows start 4 KB or 32 KB apart and the other's share lines:
+    tiles in order."""
+    import torch
+    x, r = torch.randn(T, C, device="cuda"), torch.randn(C, T, device="cuda")
+    assert torch.equal(gpu.cpy(x.t()), x.t().contiguous())
+    col = torch.randn(C, 1, device="cuda")
+    assert torch.equal(gpu.cont_add_leaky_relu(x.t(), col, r), (x.t() + col) + r)
