@@ -24,12 +24,12 @@
 //
 // Bound by the f64 arithmetic and its latency (an exp, a sine and a sincos per
 // bin); every sample taking its frames' whole DFT read each bin n_fft times from
-// LDS. A block's samples are such that its frames times bins are one round of
-// its 512 lanes (two rounds of 256: 8.2 us). Measured on MI355X at n_fft 20, hop 5, 5 seconds (24001
-// frames) 10.1 -> 7.4 us, 20 seconds 23.9 -> 17.9; n_fft 256, hop 64, 2000 frames
-// 44.4 -> 31.0.
+// LDS. Measured on MI355X at n_fft 20, hop 5, 5 seconds (24001 frames) 9.9 -> 7.0
+// us, 20 seconds 22.8 -> 16.4; n_fft 256, hop 64, 2000 frames 44.9 -> 31.9, against
+// k_istft_direct.
 
 #include <cmath>
+#include <numeric>
 
 #include "shp_internal.hpp"
 
@@ -197,6 +197,75 @@ __global__ __launch_bounds__(kIstftDirect) void k_istft_direct(const IstftArgs a
     }
 }
 
+// The kernel and the output samples per block of one call: the least estimated
+// time among k_istft at 64 to 512 samples a block (or as many whole hops as make
+// one round of its lanes) and k_istft_direct at the most samples that the LDS
+// budget holds. Forming each mirrored pair of a frame's samples once is ahead
+// while the chip has room, or where a block's samples are many against its
+// frames' overlap with its neighbours', which every block transforms again; at
+// n_fft 400, hop 100 the budget holds 64 samples a block, whose six frames are
+// 3.3 times the work of taking each sample's four (20 s of 24 kHz, MI355X: 560 us
+// against 187; but 30,000 samples 47 against 56). The estimate is in f64 operations a
+// lane, its weights fitted to 1,871 measured calls (n_fft 20 to 800, hops of an
+// eighth to all of it, 1,500 to 1,920,000 samples): its pick is 0.8 % from the
+// fastest form on average, and at most 1.13 of k_istft_direct's time.
+struct IstftForm {
+    int64_t nfft, hop, kept, bins;
+    int64_t bt     = 0;  // 0: windows too long for their hop
+    bool    direct = true;
+
+    IstftForm(int64_t n, int64_t h, int64_t samples) : nfft(n), hop(h), kept(samples), bins(n / 2 + 1) {
+        for (int64_t cand : { 256, 128, 64 }) {
+            if (lds(cand, true) <= kIstftLds) {
+                bt = cand;
+                break;
+            }
+        }
+        if (bt == 0) {
+            return;
+        }
+        int64_t       least = cost(bt, true);
+        const int64_t whole = (kIstftBlock / bins - (nfft + hop - 1) / hop) * hop;
+        for (int64_t cand : { int64_t{ 64 }, int64_t{ 128 }, int64_t{ 256 }, int64_t{ 512 }, whole }) {
+            if (cand < 64 || cand > 512 || lds(cand, false) > kIstftLds) {
+                continue;
+            }
+            const int64_t c = cost(cand, false);
+            if (c < least) {
+                least  = c;
+                bt     = cand;
+                direct = false;
+            }
+        }
+    }
+
+    // Frames that `samples` consecutive samples overlap, at most.
+    int64_t frames_of(int64_t samples) const { return (samples - 1 + nfft - 1) / hop + 2; }
+
+    size_t lds(int64_t samples, bool whole_dft) const {
+        const int64_t nf = frames_of(samples);
+        return static_cast<size_t>(nf * bins + nfft) * sizeof(double2) +
+               (whole_dft ? size_t{ 0 } : static_cast<size_t>(nf * nfft + nfft) * sizeof(double));
+    }
+
+    int64_t cost(int64_t samples, bool whole_dft) const {
+        const int64_t lanes = whole_dft ? kIstftDirect : kIstftBlock;
+        const int64_t all   = kept / hop + 1;
+        const int64_t align = std::gcd(std::gcd(samples, hop), nfft / 2);  // of every block's first position to a frame's
+        const int64_t upto  = (samples + nfft - align + hop - 1) / hop;
+        const int64_t items = (upto < all ? upto : all) * bins;
+        const int64_t round = (items + lanes - 1) / lanes, turns = (samples + lanes - 1) / lanes;
+        // a bin formed, and a term of a mirrored pair's sums: per round of the
+        // lanes and, for what the waves share, per item
+        const int64_t block = whole_dft ? 547 + round * 47 + items * 74 / lanes + turns * nfft * bins * 16 / hop :
+                                          148 + round * (47 + bins * 6) + items * (74 + bins * 6) / lanes + turns * nfft * 2 / hop;
+        // a CU's blocks share its f64 units, which eight waves fill
+        const int64_t percu = ((kept + samples - 1) / samples + 255) / 256;
+        const int64_t busy  = percu * (lanes / kWave) / 8;
+        return block * (busy > 1 ? busy : 1);
+    }
+};
+
 }  // namespace
 }  // namespace shp
 
@@ -221,36 +290,8 @@ extern "C" shp_status_t shp_inverse_stft(const shp_tensor * spectrum,
     if (spans_overlap(*spectrum, *audio) || frames > INT32_MAX || audio->ne[0] > INT32_MAX) {
         return SHP_ERR_UNSUPPORTED;
     }
-    // Output samples per block: as many whole hops as make a lane's worth of
-    // (frame, bin) items, or the most of 256, 128 and 64 that the LDS budget
-    // holds; without the windowed samples where none does with them.
-    const int64_t bins = n_fft / 2 + 1;
-    int64_t       bt = 0, nf_max = 0;
-    bool          direct = false;
-    auto          frames_of = [&](int64_t samples) { return (samples - 1 + n_fft - 1) / hop + 2; };
-    auto          bytes_of  = [&](int64_t nf, bool with) {
-        return static_cast<size_t>(nf * bins + n_fft) * sizeof(double2) +
-               (with ? static_cast<size_t>(nf * n_fft + n_fft) * sizeof(double) : size_t{ 0 });
-    };
-    const int64_t whole = (kIstftBlock / bins - (n_fft + hop - 1) / hop) * hop;
-    for (bool with : { true, false }) {
-        for (int64_t cand : { whole, int64_t{ 256 }, int64_t{ 128 }, int64_t{ 64 } }) {
-            if (cand < 64 || cand > 512 || (!with && cand == whole && whole != 256 && whole != 128 && whole != 64)) {
-                continue;
-            }
-            const int64_t nf = frames_of(cand);
-            if (bytes_of(nf, with) <= kIstftLds) {
-                bt     = cand;
-                nf_max = nf;
-                direct = !with;
-                break;
-            }
-        }
-        if (bt != 0) {
-            break;
-        }
-    }
-    if (bt == 0) {
+    const IstftForm form{ n_fft, hop, audio->ne[0] };
+    if (form.bt == 0) {
         return SHP_ERR_UNSUPPORTED;  // windows too long for their hop to stage a block's frames
     }
     if (dry_run()) {
@@ -264,14 +305,14 @@ extern "C" shp_status_t shp_inverse_stft(const shp_tensor * spectrum,
     a.kept       = audio->ne[0];
     a.nfft       = n_fft;
     a.hop        = hop;
-    a.bins       = static_cast<int32_t>(bins);
-    a.bt         = static_cast<int32_t>(bt);
-    a.nf_max     = static_cast<int32_t>(nf_max);
+    a.bins       = static_cast<int32_t>(form.bins);
+    a.bt         = static_cast<int32_t>(form.bt);
+    a.nf_max     = static_cast<int32_t>(form.frames_of(form.bt));
     a.fhop       = make_fastdiv(static_cast<uint32_t>(hop));
-    a.fbins      = make_fastdiv(static_cast<uint32_t>(bins));
-    const size_t  lds    = bytes_of(nf_max, !direct);
-    const int64_t blocks = (a.kept + bt - 1) / bt;
-    hipLaunchKernelGGL(direct ? k_istft_direct : k_istft, dim3(static_cast<unsigned>(blocks)),
-                       dim3(direct ? kIstftDirect : kIstftBlock), lds, as_stream(stream), a);
+    a.fbins      = make_fastdiv(static_cast<uint32_t>(form.bins));
+    const size_t  lds    = form.lds(form.bt, form.direct);
+    const int64_t blocks = (a.kept + form.bt - 1) / form.bt;
+    hipLaunchKernelGGL(form.direct ? k_istft_direct : k_istft, dim3(static_cast<unsigned>(blocks)),
+                       dim3(form.direct ? kIstftDirect : kIstftBlock), lds, as_stream(stream), a);
     return launch_status();
 }

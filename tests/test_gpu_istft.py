@@ -52,6 +52,16 @@ def test_istft_block_shapes(gpu, n_fft, hop, frames):
     _close(_np(gpu.inverse_stft(_t(gpu, spec), n_fft, hop)), R.run(lambda g: g.inverse_stft(spec, n_fft, hop)))
 
 
+@pytest.mark.parametrize("n_fft,hop,frames", [(400, 100, 5), (400, 100, 700), (512, 512, 40), (512, 204, 500), (200, 25, 2500),
+                                              (440, 440, 300), (64, 16, 9000), (20, 5, 13000), (128, 85, 1500), (600, 600, 9)])
+def test_istft_forms(gpu, n_fft, hop, frames):
+    """Either side of the estimate's choice: blocks of 64 to 512 samples and of a
+    whole hop, frames formed once or per sample."""
+    rng = np.random.default_rng([SEED, n_fft, hop, frames])
+    spec = rng.uniform(-3, 2, (frames, n_fft + 2)).astype(np.float32)
+    _close(_np(gpu.inverse_stft(_t(gpu, spec), n_fft, hop)), R.run(lambda g: g.inverse_stft(spec, n_fft, hop)))
+
+
 def test_istft_infinite_magnitude(gpu):
     """A log-magnitude past exp's range makes its own frames' samples infinite or NaN and no others."""
     rng = np.random.default_rng(SEED + 5)

@@ -81,3 +81,22 @@ def test_short_row_sums_and_norms_go_by_elements():
             names = _kernels([(op, t(n, rows), *extra, t(n if extra else 1, rows)) for n in widths])
             assert [last(k[0]) for k in names] == list(widths.values()), (op, rows, names)
             assert op == "shp_norm" or all("Li64E" in k[0] for k in names)
+
+
+def _istft(n, hop, frames):
+    return "shp_inverse_stft", t(n + 2, frames), n, hop, t((frames - 1) * hop)
+
+
+def test_inverse_stft_forms_its_frames_once_only_where_the_blocks_are_long_enough():
+    """Windows whose LDS leaves a block few samples go sample by sample once the
+    chip is full; blocks get longer with the utterance."""
+    cases = [((400, 100, 20), False), ((400, 100, 4801), True), ((512, 204, 2400), True), ((200, 25, 80000), True),
+             ((360, 72, 6000), True), ((540, 216, 9000), True), ((600, 600, 800), True), ((20, 5, 24001), False),
+             ((256, 64, 2000), False), ((512, 512, 29), False)]
+    names = _kernels([_istft(*c) for c, _ in cases])
+    assert [("k_istft_direct" in k[0]) for k in names] == [d for _, d in cases]
+    per_block = []
+    for frames in (300, 6000, 24001, 400000):
+        (st, ls), = record([_istft(20, 5, frames)])
+        per_block.append(-(-(frames - 1) * 5 // ls[0][1][0]))
+    assert per_block == sorted(per_block) and per_block[0] <= 64 and per_block[-1] > 400, per_block
