@@ -7,10 +7,13 @@
 // whose butterflies multiply and add in double and round their two results to
 // f32 per stage, the amplitudes sqrt(re^2 + im^2 + 1e-9) (double, rounded),
 // and per mel bin the filterbank-weighted sum in double in frequency order and
-// log(max(energy, 1e-5)). The device's double cos, sin, sqrt and log replace
-// the host library's; sqrt is correctly rounded on both.
+// log(max(energy, 1e-5)). It differs from the host code's in these: one of a
+// butterfly's two products is fused with their sum (a rounding of the double
+// fewer; the two apart: 4-10 % of the time), and the device's double cos, sin,
+// sqrt and log replace the host library's; sqrt is correctly rounded on both.
+// Every form below gives a frame the same bits.
 //
-// A block has kMelWaves transform waves and kMelScan more:
+// A block has 1, 2 or 4 transform waves and kMelScan more:
 //   - a transform wave runs whole frames (one at n_fft 1024, more of a shorter
 //     transform, so that every lane has work): every lane loads 16 samples at
 //     their bit-reversed places straight from memory, runs four stages on them
@@ -28,7 +31,7 @@
 // its 25,000 cycles the transform takes 12,500 (5,120 f64 butterflies a wave),
 // the filterbank read beside it 13,000, the amplitudes 2,800, the mel sums and
 // logs 4,200. Measured on MI355X at the production parameters: a 10-second clip
-// (937 frames) 52.1 -> 12.2 us, one second 40.4 -> 12.3, 20 seconds 93.7 -> 23.0
+// (937 frames) 52.1 -> 12.2 us, one second 40.4 -> 10.9, 20 seconds 93.7 -> 23.0
 // (n_fft 512, hop 160, 80 bins, 10 s: 24.9 -> 11.7; n_fft 2048, hop 512: 54.1 ->
 // 32.2), against a 256-thread block per frame with a barrier per stage, n_fft - 1
 // twiddles evaluated per block and every lane reading a whole filterbank row.
@@ -56,6 +59,11 @@ constexpr int    kMelScan    = 8;    // waves that scan the filterbank
 constexpr int    kMelBins    = 256;  // mel bins whose masks are held at a time
 constexpr int    kMelPerWave = 8;    // frames of a short transform a wave takes at most
 
+constexpr int    kMelUnmasked  = 32;     // n_fft up to which every frequency is summed: no more than four float4 a filter
+constexpr int    kMelFrameNfft = 256;    // the block-per-frame form's n_fft,
+constexpr int    kMelFrameMost = 2048;   // frames (its blocks of one round: eight a CU)
+constexpr int    kMelFrameWork = 98304;  // and samples at most
+
 struct MelArgs {
     const float * pcm;
     const float * fb;  // [bins][n_fft/2 + 1]
@@ -70,7 +78,7 @@ struct MelArgs {
     int32_t       pad;
     int32_t       bins;
     int32_t       lfw;  // log2 of the frames a transform wave takes
-    int32_t       reserved;
+    int32_t       masked;  // the filters' spans are found first
 };
 
 // LDS place of transform element i: one element of padding per 16 spreads the
@@ -268,7 +276,7 @@ template <int WAVES> __global__ __launch_bounds__((WAVES + kMelScan) * kWave) vo
     const int     wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int     fpb  = WAVES << a.lfw;
     uint64_t *    s_mask = reinterpret_cast<uint64_t *>(s_tw + n / 2);
-    const int     words  = mel_words(n);
+    const int     words  = a.masked != 0 ? mel_words(n) : 0;
     float2 *      s_d    = reinterpret_cast<float2 *>(s_mask + kMelBins * words);
     float *       s_win = reinterpret_cast<float *>(s_d + fpb * mel_frame_elems(n));
     float *       s_mag = s_win + n;
@@ -316,7 +324,7 @@ template <int WAVES> __global__ __launch_bounds__((WAVES + kMelScan) * kWave) vo
         if (b0 != 0) {
             __syncthreads();  // the masks of the bins before have been used
         }
-        if (wave >= WAVES) {
+        if (wave >= WAVES && a.masked != 0) {
             mel_masks(rows, nb, nf, words, wave - WAVES, lane, s_mask);
         }
         __syncthreads();
@@ -349,8 +357,9 @@ template <int WAVES> __global__ __launch_bounds__((WAVES + kMelScan) * kWave) vo
                     hi = i * kWave + 64 - __clzll(static_cast<long long>(any));
                 }
             }
-            lo = s_bad[f] != 0 ? 0 : lo;
-            hi = s_bad[f] != 0 ? nf / 4 : hi;
+            const bool every = s_bad[f] != 0 || words == 0;
+            lo               = every ? 0 : lo;
+            hi               = every ? nf / 4 : hi;
             double        e = 0.0;
             // the product of two f32 is exact in double: one rounding either way
 #pragma unroll 4
@@ -369,11 +378,91 @@ template <int WAVES> __global__ __launch_bounds__((WAVES + kMelScan) * kWave) vo
     }
 }
 
+// A block per frame, all its lanes on one stage at a time and a lane per mel bin
+// over every frequency: short transforms of few frames, which leave k_log_mel's
+// waves a few lanes of work each and a long chain (n_fft 64, hop 16, 80 bins: 250
+// frames 4.8 us against 6.3, 1500 frames 7.0 against 7.4, 3750 frames 13.5 against
+// 9.1; MI355X, cold).
+__global__ __launch_bounds__(256) void k_log_mel_frame(const MelArgs a) {
+    extern __shared__ double2 s_tw[];  // [nfft - 1] twiddles, then re, im (f32), then amplitudes
+    float *       s_re  = reinterpret_cast<float *>(s_tw + (a.nfft - 1));
+    float *       s_im  = s_re + a.nfft;
+    float *       s_mag = s_im + a.nfft;
+    const int     tid   = static_cast<int>(threadIdx.x);
+    const int64_t f     = blockIdx.x;
+    const int     n     = a.nfft;
+    const int     nf    = n / 2 + 1;
+    // twiddle idx = len/2 - 1 + k for stage length len and butterfly offset k
+    for (int idx = tid; idx < n - 1; idx += 256) {
+        const int    half  = 1 << (31 - __clz(idx + 1));  // len / 2
+        const int    len   = half * 2;
+        const int    k     = idx - (half - 1);
+        const double angle = -2.0 * kMelPi / static_cast<double>(len);
+        double       sn, cs;
+        sincos(angle * static_cast<double>(k), &sn, &cs);
+        s_tw[idx] = double2{ cs, sn };
+    }
+    const int wpl = (n - a.win) / 2;
+    for (int i = tid; i < n; i += 256) {
+        // the padded signal at frame start + i: reflect-padded by `pad`
+        const int64_t p = f * a.hop + i;
+        float         x;
+        if (p < a.pad) {
+            x = a.pcm[a.pad - p];
+        } else if (p < a.pad + a.ns) {
+            x = a.pcm[p - a.pad];
+        } else {
+            x = a.pcm[a.ns - 2 - (p - a.pad - a.ns)];
+        }
+        float w = 0.0f;
+        if (i >= wpl && i < wpl + a.win) {
+            const double phase = 2.0 * kMelPi * static_cast<double>(i - wpl) / static_cast<double>(a.win);
+            w                  = static_cast<float>(0.5 - 0.5 * cos(phase));
+        }
+        const int r = static_cast<int>(__brev(static_cast<unsigned>(i)) >> (32 - a.log2n));
+        s_re[r]     = x * w;
+        s_im[r]     = 0.0f;
+    }
+    __syncthreads();
+    for (int half = 1; half < n; half *= 2) {
+        for (int t = tid; t < n / 2; t += 256) {
+            const int     k   = t & (half - 1);
+            const int     ia  = (t - k) * 2 + k;  // start + k, start = (t / half) * 2 * half
+            const int     ib  = ia + half;
+            const double2 tw  = s_tw[half - 1 + k];
+            const double  br  = s_re[ib], bi = s_im[ib];
+            const double  xr  = fma(br, tw.x, -(bi * tw.y));
+            const double  xi  = fma(br, tw.y, bi * tw.x);
+            const double  ar  = s_re[ia];
+            const double  ai  = s_im[ia];
+            s_re[ib]          = static_cast<float>(ar - xr);
+            s_im[ib]          = static_cast<float>(ai - xi);
+            s_re[ia]          = static_cast<float>(ar + xr);
+            s_im[ia]          = static_cast<float>(ai + xi);
+        }
+        __syncthreads();
+    }
+    for (int k = tid; k < nf; k += 256) {
+        const double sq = static_cast<double>(s_re[k]) * static_cast<double>(s_re[k]) +
+                          static_cast<double>(s_im[k]) * static_cast<double>(s_im[k]);
+        s_mag[k]        = static_cast<float>(sqrt(sq + 1e-9));
+    }
+    __syncthreads();
+    for (int b = tid; b < a.bins; b += 256) {
+        const float * row = a.fb + static_cast<int64_t>(b) * nf;
+        double        e   = 0.0;
+        for (int k = 0; k < nf; ++k) {
+            e += static_cast<double>(row[k]) * static_cast<double>(s_mag[k]);
+        }
+        a.y[f * a.bins + b] = static_cast<float>(log(e < 1e-5 ? 1e-5 : e));  // std::max(e, 1e-5)
+    }
+}
+
 template <int WAVES> shp_status_t launch_mel(const MelArgs & a, hipStream_t stream) {
     const int    n   = a.nfft, nf = n / 2 + 1;
     const int    fpb = WAVES << a.lfw;
     const size_t lds = static_cast<size_t>(n / 2) * sizeof(double2) + static_cast<size_t>(fpb) * mel_frame_elems(n) * sizeof(float2) +
-                       static_cast<size_t>(n + fpb * nf) * sizeof(float) + static_cast<size_t>(kMelBins * mel_words(n)) * sizeof(uint64_t) +
+                       static_cast<size_t>(n + fpb * nf) * sizeof(float) + static_cast<size_t>(a.masked != 0 ? kMelBins * mel_words(n) : 0) * sizeof(uint64_t) +
                        static_cast<size_t>(fpb) * sizeof(int);
     const int64_t blocks = (a.frames + fpb - 1) / fpb;
     hipLaunchKernelGGL((k_log_mel<WAVES>), dim3(static_cast<unsigned>(blocks)), dim3((WAVES + kMelScan) * kWave), lds, stream, a);
@@ -478,9 +567,35 @@ extern "C" shp_status_t shp_log_mel(const shp_tensor * pcm,
     a.pad    = static_cast<int32_t>(pad);
     a.bins   = static_cast<int32_t>(bins);
     a.fnf    = make_fastdiv(static_cast<uint32_t>(n_fft / 2 + 1));
-    // 16 samples a lane: a wave takes 1024 of them
-    for (a.lfw = 0; (n_fft << (a.lfw + 1)) <= 1024 && (2 << a.lfw) <= kMelPerWave; ++a.lfw) {
+    if (n_fft > 1 && n_fft <= kMelFrameNfft && frames <= kMelFrameMost && n_fft * frames <= kMelFrameWork) {
+        const size_t lds = static_cast<size_t>(n_fft - 1) * sizeof(double2) + static_cast<size_t>(2 * n_fft + n_fft / 2 + 1) * sizeof(float);
+        hipLaunchKernelGGL(k_log_mel_frame, dim3(static_cast<unsigned>(frames)), dim3(256), lds, as_stream(stream), a);
+        return launch_status();
     }
-    // four waves' elements and tables are 58 KB of LDS at n_fft 1024
-    return n_fft <= 1024 ? launch_mel<kMelWaves>(a, as_stream(stream)) : launch_mel<1>(a, as_stream(stream));
+    a.masked = n_fft > kMelUnmasked;
+    // The fewest frames a block that leave one block a CU, more of a short
+    // transform to a wave (16 samples a lane: a wave takes 1024 of them) before
+    // more waves (four waves' elements and tables are 58 KB of LDS at n_fft 1024).
+    // n_fft 1024, hop 256, 80 bins: 234 frames one a block 10.3 us, four 11.6; 937
+    // frames 35 and 12.2. n_fft 64, 128 bins: 1500 frames in eights 9.4, in 32s 14.7.
+    int most = 0;
+    while ((n_fft << (most + 1)) <= 1024 && (2 << most) <= kMelPerWave) {
+        ++most;
+    }
+    const int waves = n_fft <= 1024 ? kMelWaves : 1;
+    int       fpb   = 1;
+    while (fpb < waves << most && (frames + fpb - 1) / fpb > 256) {
+        fpb *= 2;
+    }
+    while (a.lfw < most && (2 << a.lfw) <= fpb) {
+        ++a.lfw;
+    }
+    switch (fpb >> a.lfw) {
+        case 1:
+            return launch_mel<1>(a, as_stream(stream));
+        case 2:
+            return launch_mel<2>(a, as_stream(stream));
+        default:
+            return launch_mel<kMelWaves>(a, as_stream(stream));
+    }
 }

@@ -111,3 +111,24 @@ def test_log_mel_infinite_amplitudes(gpu, value):
     assert np.array_equal(np.isinf(got), np.isinf(ref))
     ok = np.isfinite(ref)
     _close(got[ok], ref[ok])
+
+
+@pytest.mark.parametrize("n_fft,hop,bins", [(2, 1, 5), (16, 4, 30), (32, 8, 80), (64, 16, 80), (256, 64, 128), (512, 128, 80),
+                                            (1024, 256, 128)])
+def test_log_mel_frames_do_not_depend_on_the_clip(gpu, n_fft, hop, bins):
+    """A frame's bits are the same alone, in a short clip and in one of thousands
+    of frames: a block per frame, one to four waves, one to eight frames each."""
+    rng = np.random.default_rng([SEED, n_fft, 3])
+    pad = (n_fft - hop) // 2
+    pcm = _t(gpu, (rng.standard_normal(hop * 8500 if n_fft <= 64 else 400000) * 0.2).astype(np.float32))
+    fb = _t(gpu, gpu.mel_filterbank(24000, n_fft, bins, 0.0, 12000.0))
+    long = _np(gpu.log_mel(pcm, fb, n_fft, hop, n_fft))
+    for frames in (3, 20, 150, 300, 600, 1200, 2049, 3000):
+        ns = frames * hop + n_fft
+        if ns > pcm.numel():
+            break
+        got = _np(gpu.log_mel(pcm[:ns], fb, n_fft, hop, n_fft))
+        inside = frames - pad // hop - 1            # frames that the end's reflection does not reach
+        assert np.array_equal(got[:inside].view(np.uint32), long[:inside].view(np.uint32)), frames
+    ref = R.run(lambda g: g.log_mel(_np(pcm)[:50 * hop + n_fft], _np(fb), n_fft, hop, n_fft))
+    _close(long[:49 - pad // hop], ref[:49 - pad // hop])

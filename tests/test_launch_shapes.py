@@ -100,3 +100,21 @@ def test_inverse_stft_forms_its_frames_once_only_where_the_blocks_are_long_enoug
         (st, ls), = record([_istft(20, 5, frames)])
         per_block.append(-(-(frames - 1) * 5 // ls[0][1][0]))
     assert per_block == sorted(per_block) and per_block[0] <= 64 and per_block[-1] > 400, per_block
+
+
+def test_log_mel_spreads_its_frames_over_the_chip():
+    """Few frames go a block each (a short transform in the block-per-frame form),
+    more in as few blocks as one a CU."""
+    def call(n, hop, frames, bins=80):
+        ns = (frames - 1) * hop + n - 2 * ((n - hop) // 2)
+        return "shp_log_mel", t(ns), t(n // 2 + 1, bins), n, hop, n, t(bins, frames)
+    #        n_fft, hop, frames, frame form, blocks
+    cases = [(64, 16, 250, True, 250), (64, 16, 1536, True, 1536), (64, 16, 1537, False, 193), (256, 64, 384, True, 384),
+             (256, 64, 385, False, 193), (16, 4, 2049, False, 129), (1024, 256, 15, False, 15), (1024, 256, 256, False, 256),
+             (1024, 256, 257, False, 129), (1024, 256, 937, False, 235), (1024, 256, 2000, False, 500), (2048, 512, 900, False, 900),
+             (1, 1, 100, False, 100), (512, 128, 1875, False, 235)]
+    got = record([call(*c[:3]) for c in cases])
+    for (n, hop, frames, form, blocks), (st, ls) in zip(cases, got):
+        assert st == 0 and len(ls) == 1
+        assert (("k_log_mel_frame" in ls[0][0]), ls[0][1][0]) == (form, blocks), (n, frames, ls)
+        assert ls[0][3] <= 64 * 1024
