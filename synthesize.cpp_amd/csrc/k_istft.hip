@@ -55,6 +55,7 @@ struct IstftArgs {
     int32_t      pad;
     FastDiv      fhop;
     FastDiv      fbins;
+    int64_t      block0;  // the launch's first block
 };
 
 __global__ __launch_bounds__(kIstftBlock) void k_istft(const IstftArgs a) {
@@ -64,7 +65,7 @@ __global__ __launch_bounds__(kIstftBlock) void k_istft(const IstftArgs a) {
     double *      win  = reinterpret_cast<double *>(fb + a.nf_max * a.bins);
     double *      vw   = win + a.nfft;
     const int     tid  = static_cast<int>(threadIdx.x);
-    const int64_t t0   = static_cast<int64_t>(blockIdx.x) * a.bt;
+    const int64_t t0   = (a.block0 + blockIdx.x) * a.bt;
     const int     nt   = static_cast<int>(a.kept - t0 < a.bt ? a.kept - t0 : a.bt);
     const int     half = a.nfft / 2;
     // frames overlapping positions [t0 + half, t0 + nt - 1 + half]
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(kIstftDirect) void k_istft_direct(const IstftArgs a
     double2 *     tw   = sm;
     double2 *     fb   = sm + a.nfft;
     const int     tid  = static_cast<int>(threadIdx.x);
-    const int64_t t0   = static_cast<int64_t>(blockIdx.x) * a.bt;
+    const int64_t t0   = (a.block0 + blockIdx.x) * a.bt;
     const int64_t t1   = t0 + a.bt < a.kept ? t0 + a.bt : a.kept;
     const int     half = a.nfft / 2;
     // frames overlapping positions [t0 + half, t1 - 1 + half]
@@ -312,7 +313,9 @@ extern "C" shp_status_t shp_inverse_stft(const shp_tensor * spectrum,
     a.fbins      = make_fastdiv(static_cast<uint32_t>(form.bins));
     const size_t  lds    = form.lds(form.bt, form.direct);
     const int64_t blocks = (a.kept + form.bt - 1) / form.bt;
-    hipLaunchKernelGGL(form.direct ? k_istft_direct : k_istft, dim3(static_cast<unsigned>(blocks)),
-                       dim3(form.direct ? kIstftDirect : kIstftBlock), lds, as_stream(stream), a);
-    return launch_status();
+    const int     block  = form.direct ? kIstftDirect : kIstftBlock;
+    return in_launches(blocks, block, [&](int64_t first, dim3 grid) {
+        a.block0 = first;
+        hipLaunchKernelGGL(form.direct ? k_istft_direct : k_istft, grid, dim3(block), lds, as_stream(stream), a);
+    });
 }

@@ -79,6 +79,7 @@ struct MelArgs {
     int32_t       bins;
     int32_t       lfw;  // log2 of the frames a transform wave takes
     int32_t       masked;  // the filters' spans are found first
+    int64_t       block0;  // the launch's first block
 };
 
 // LDS place of transform element i: one element of padding per 16 spreads the
@@ -281,7 +282,7 @@ template <int WAVES> __global__ __launch_bounds__((WAVES + kMelScan) * kWave) vo
     float *       s_win = reinterpret_cast<float *>(s_d + fpb * mel_frame_elems(n));
     float *       s_mag = s_win + n;
     int *         s_bad = reinterpret_cast<int *>(s_mag + fpb * nf);
-    const int64_t f0    = static_cast<int64_t>(blockIdx.x) * fpb;
+    const int64_t f0    = (a.block0 + blockIdx.x) * fpb;
     const int     nfr   = static_cast<int>(a.frames - f0 < fpb ? a.frames - f0 : fpb);  // the block's frames
 
     for (int k = tid; k < n / 2; k += kThreads) {
@@ -464,9 +465,12 @@ template <int WAVES> shp_status_t launch_mel(const MelArgs & a, hipStream_t stre
     const size_t lds = static_cast<size_t>(n / 2) * sizeof(double2) + static_cast<size_t>(fpb) * mel_frame_elems(n) * sizeof(float2) +
                        static_cast<size_t>(n + fpb * nf) * sizeof(float) + static_cast<size_t>(a.masked != 0 ? kMelBins * mel_words(n) : 0) * sizeof(uint64_t) +
                        static_cast<size_t>(fpb) * sizeof(int);
-    const int64_t blocks = (a.frames + fpb - 1) / fpb;
-    hipLaunchKernelGGL((k_log_mel<WAVES>), dim3(static_cast<unsigned>(blocks)), dim3((WAVES + kMelScan) * kWave), lds, stream, a);
-    return launch_status();
+    constexpr int kThreads = (WAVES + kMelScan) * kWave;
+    return in_launches((a.frames + fpb - 1) / fpb, kThreads, [&](int64_t first, dim3 grid) {
+        MelArgs part = a;
+        part.block0  = first;
+        hipLaunchKernelGGL((k_log_mel<WAVES>), grid, dim3(kThreads), lds, stream, part);
+    });
 }
 
 double slaney_step() {

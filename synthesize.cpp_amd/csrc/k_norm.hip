@@ -34,6 +34,7 @@ struct NormArgs {
     int64_t       nrows;
     int32_t       ne0;
     float         eps;
+    int64_t       block0;  // k_layer_norm: the launch's first block
 };
 
 enum NormMode { kPlain = 0, kAdd = 1, kAddSum = 2 };
@@ -296,7 +297,7 @@ template <int TPR, int VPL> __global__ __launch_bounds__(TPR > 256 ? TPR : 256) 
     constexpr int     kBlock = TPR > 256 ? TPR : 256;
     __shared__ double s_mean[kBlock / kWave], s_var[kBlock / kWave];
     const int         l    = static_cast<int>(threadIdx.x) % TPR;
-    const int64_t     row  = static_cast<int64_t>(blockIdx.x) * (kBlock / TPR) + row_in_block<TPR>();
+    const int64_t     row  = (a.block0 + blockIdx.x) * (kBlock / TPR) + row_in_block<TPR>();
     const bool        live = row < a.nrows;
     const int64_t     rr   = live ? row : 0;
     const int         n4   = live && VPL > 0 ? a.ne0 / 4 : 0;
@@ -349,7 +350,7 @@ constexpr int kLayerNormWide = 1024;
 __global__ __launch_bounds__(kLayerNormWide) void k_layer_norm_wide(const NormArgs a) {
     __shared__ double s_mean[kLayerNormWide / kWave], s_var[kLayerNormWide / kWave];
     const int         l    = static_cast<int>(threadIdx.x);
-    const int64_t     row  = blockIdx.x;
+    const int64_t     row  = a.block0 + blockIdx.x;
     const int         n4   = a.ne0 / 4;
     const int         tail = a.ne0 % 4;
     const float *     xr = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, row));
@@ -392,15 +393,16 @@ constexpr int64_t kLayerNormManyRows = 2048;
 
 shp_status_t launch_layer_norm(const NormArgs & a, hipStream_t stream) {
     auto go = [&](auto kernel, int tpr) {
-        const int     block  = tpr > 256 ? tpr : 256;
-        const int64_t blocks = (a.nrows + block / tpr - 1) / (block / tpr);
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(block), 0, stream, a);
-        return launch_status();
+        const int block = tpr > 256 ? tpr : 256;
+        return in_launches((a.nrows + block / tpr - 1) / (block / tpr), block, [&](int64_t first, dim3 grid) {
+            NormArgs part = a;
+            part.block0   = first;
+            hipLaunchKernelGGL(kernel, grid, dim3(block), 0, stream, part);
+        });
     };
     const int n4 = a.ne0 / 4;
     if (a.ne0 > kLayerNormMax) {
-        hipLaunchKernelGGL(k_layer_norm_wide, dim3(static_cast<unsigned>(a.nrows)), dim3(kLayerNormWide), 0, stream, a);
-        return launch_status();
+        return go(k_layer_norm_wide, kLayerNormWide);
     }
     if (a.ne0 <= 64) {
         return go(k_layer_norm<64, 0>, 64);
@@ -1763,8 +1765,8 @@ shp_status_t layer_step_launch(const shp_layer_step & s, hipStream_t stream, boo
     const bool dec = t <= kRopeDecMaxPos;
     a.chunks       = static_cast<int32_t>((rows + kLayerDecRows - 1) / kLayerDecRows);
     const int64_t rope = dec ? t * a.chunks : t, act = (a.act4 + kLayerBlock - 1) / kLayerBlock;
-    if (t + rope + act > INT32_MAX) {
-        return SHP_OK;
+    if (t + rope + act > int64_t{ UINT32_MAX } / kLayerBlock) {
+        return SHP_OK;  // more blocks than a launch takes
     }
     a.rope_first   = static_cast<uint32_t>(t);
     a.swiglu_first = static_cast<uint32_t>(t + rope);

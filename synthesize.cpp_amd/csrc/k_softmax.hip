@@ -52,6 +52,7 @@ struct SoftMaxArgs {
     // from multiply-shift divisions (FastDiv) instead of 64-bit divisions.
     int32_t       mfast;
     int32_t       pad;
+    int64_t       block0;  // the launch's first block
     int64_t       n_past;  // causal form: element i of row r is masked when i > n_past + r % ne1
     FastDiv       fne1;
     FastDiv       fne2;
@@ -112,7 +113,7 @@ template <int K, int MK> __global__ __launch_bounds__(256) void k_soft_max_wave(
     __shared__ double s_tab[256 / kWave][64];
     softmax_args_in_sgprs<MK>(a);
     const int     lane = threadIdx.x % kWave;
-    const int64_t r    = static_cast<int64_t>(blockIdx.x) * (256 / kWave) +
+    const int64_t r    = (a.block0 + blockIdx.x) * (256 / kWave) +
                       __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     if (r >= a.nrows) {
         return;  // whole wave
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(BLOCK) void k_soft_max_rows4(const SoftMaxArgs a) {
     const int     q    = threadIdx.x % kLanes;
     const int     wv   = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     const int     slot = wv / WPR;  // row of this block
-    const int64_t r    = static_cast<int64_t>(blockIdx.x) * (BLOCK / kLanes) + slot;
+    const int64_t r    = (a.block0 + blockIdx.x) * (BLOCK / kLanes) + slot;
     const bool    live = r < a.nrows;
     if (WPR == 1 && !live) {
         return;  // whole wave; the one-wave form has no barrier
@@ -344,7 +345,7 @@ template <int MK> __global__ __launch_bounds__(kSoftMaxBlock) void k_soft_max_bl
     __shared__ float  s_max[kWaves];
     __shared__ double s_sum[kWaves];
     __shared__ double s_tab[kWaves][64];
-    const int64_t  r    = blockIdx.x;
+    const int64_t  r    = a.block0 + blockIdx.x;
     const int      lane = threadIdx.x % kWave;
     const int      wv   = threadIdx.x / kWave;
     const float *  xr   = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.x) + row_offset(a.xm, r));
@@ -478,9 +479,11 @@ template <int MK> shp_status_t launch_soft_max(const SoftMaxArgs & a, hipStream_
         return SHP_OK;
     }
     auto go = [&](auto kernel, int rows_per_block, int block) {
-        const int64_t blocks = (a.nrows + rows_per_block - 1) / rows_per_block;
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(block), 0, stream, a);
-        return launch_status();
+        return in_launches((a.nrows + rows_per_block - 1) / rows_per_block, block, [&](int64_t first, dim3 grid) {
+            SoftMaxArgs part = a;
+            part.block0      = first;
+            hipLaunchKernelGGL(kernel, grid, dim3(block), 0, stream, part);
+        });
     };
     if (by_elements(a)) {
         return a.ne0 <= 1 * kWave ? go(k_soft_max_wave<1, MK>, 4, 256) :

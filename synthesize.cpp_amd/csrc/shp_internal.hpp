@@ -557,6 +557,20 @@ inline shp_status_t launch_status() {
     return hipGetLastError() == hipSuccess ? SHP_OK : SHP_ERR_BACKEND;
 }
 
+// `blocks` blocks of `threads` in as few launches as their size allows (a launch
+// ends below 2^32 threads a dimension): go(first block, blocks of this launch).
+template <class Go> shp_status_t in_launches(int64_t blocks, int threads, const Go & go) {
+    const int64_t most = int64_t{ UINT32_MAX } / threads;
+    for (int64_t first = 0; first < blocks; first += most) {
+        go(first, dim3(static_cast<unsigned>(blocks - first < most ? blocks - first : most)));
+        const shp_status_t st = launch_status();
+        if (st != SHP_OK) {
+            return st;
+        }
+    }
+    return SHP_OK;
+}
+
 // A checked layer step in one launch (k_norm.hip). `taken` is false when the
 // step's layouts are not that launch's: nothing was enqueued then.
 shp_status_t layer_step_launch(const shp_layer_step & s, hipStream_t stream, bool & taken);

@@ -3,7 +3,7 @@ import re
 
 import pytest
 
-from launches import record, t
+from launches import layer, record, t
 
 ROWS = [1, 8, 64, 65, 250, 256, 257, 640, 1023, 1024, 2047, 2048, 2049, 4096, 4097, 16384, 40000]
 WIDTHS = [1, 3, 63, 64, 65, 100, 127, 128, 129, 192, 200, 255, 256, 257, 301, 320, 321, 384, 500, 511, 512, 513, 700, 767,
@@ -118,3 +118,38 @@ def test_log_mel_spreads_its_frames_over_the_chip():
         assert st == 0 and len(ls) == 1
         assert (("k_log_mel_frame" in ls[0][0]), ls[0][1][0]) == (form, blocks), (n, frames, ls)
         assert ls[0][3] <= 64 * 1024
+
+
+def _layer_step(T, hidden=4, heads=1, kv=1, ffn=4):
+    x = lambda n: t(n, T)
+    w = lambda n: t(n, type_=30)
+    q, k = lambda: t(128, heads, T), lambda: t(128, kv, T)
+    return "shp_layer_nongemm_step", layer(x(hidden), w(hidden), x(hidden), q(), k(), w(128), w(128), t(T, type_=26), q(), k(),
+                                           x(hidden), w(hidden), x(hidden), x(hidden), x(ffn), x(ffn), x(ffn), x(hidden), x(hidden))
+
+
+def test_a_launch_ends_below_two_to_the_32_threads():
+    """Tensors of more rows, samples or positions than one launch's threads: several
+    launches that together have a block for all of it (the step: its five). Those
+    of 2^26 rows and more ended in an error before any split."""
+    def soft(n, rows, causal):
+        x, y = t(n, rows), t(n, rows)
+        return ("shp_soft_max_causal", x, 0, 0.5, y) if causal else ("shp_soft_max_ext", x, None, 0.5, 0.0, y)
+    #        call, blocks in all
+    cases = [(("shp_norm", t(300, 50000001), 1e-5, t(300, 50000001)), 25000001),
+             (("shp_norm", t(700, 20000000), 1e-5, t(700, 20000000)), 5000000),
+             (("shp_norm", t(70000, 5000001), 1e-5, t(70000, 5000001)), 5000001),
+             (soft(9001, 5000003, False), 5000003), (soft(9001, 5000003, True), 5000003),
+             (soft(2047, 60000001, False), 30000001), (soft(17000, 4500000, False), 4500000), (soft(130, 80000001, False), 20000001),
+             (("shp_log_mel", t(9000000), t(1025, 8), 2048, 1, 2048, t(8, 8999999)), 8999999),
+             (_istft(160, 20, 100000001), None), (_istft(20, 5, 400000001), None), (_istft(400, 100, 20000001), None)]
+    for (call, blocks), (st, ls) in zip(cases, record([c for c, _ in cases])):
+        assert st == 0 and ls, (call[0], st)
+        for _, grid, block, _ in ls:
+            assert grid[0] * block[0] < 2 ** 32 and grid[1:] == block[1:] == (1, 1), (call, ls)
+        assert blocks is None or sum(g[0] for _, g, *_ in ls) == blocks, (call, ls)
+        assert len({n for n, *_ in ls}) == 1 and len(ls) == -(-sum(g[0] for _, g, *_ in ls) // ((2 ** 32 - 1) // ls[0][2][0]))
+    for T in (100, 8388607, 8388608, 9000000):
+        (st, ls), = record([_layer_step(T)])
+        assert st == 0 and all(g[0] * b[0] < 2 ** 32 for _, g, b, _ in ls)
+        assert len(ls) == (1 if T <= 8380000 else 5), (T, ls)
