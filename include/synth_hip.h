@@ -613,7 +613,7 @@ shp_status_t shp_cont_add_leaky_relu(const shp_tensor * x,
  * and the layouts are the 128-wide rope's and whole aligned float4 rows of up
  * to 4096 values; otherwise five, each the launch of shp_rms_norm_mul,
  * shp_qk_norm_rope, shp_add_rms_norm_mul, shp_swiglu and shp_add, in this
- * order. The same results either way. Every tensor's presence, type and shape is checked first:
+ * order. The same bits either way. Every tensor's presence, type and shape is checked first:
  * a malformed step returns SHP_ERR_INVALID_ARG with nothing enqueued.
  * x, normed, attn_out, resid, mlp_in, mlp_out, out: F32 [hidden, T];
  * q, q_out: F32 [head_dim, q_heads, T]; k, k_out: F32 [head_dim, kv_heads, T];

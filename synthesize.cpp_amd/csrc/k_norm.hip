@@ -587,6 +587,39 @@ template <int MODE> shp_status_t sum_rows_entry(const shp_tensor * x, const shp_
     return launch_sum_rows<MODE>(a, stream);
 }
 
+// Lanes that share an RMSNorm row of nvec float4 (at most kRmsMaxVec; PLAIN: no
+// residual add), and so the order in which its squares are added: whoever adds
+// them otherwise gives other bits. Rows of 1024 / 2048: by row count.
+// Measured on MI355X (cold, us; 4 waves per row first, then the pick):
+//   plain 1024: 4 waves up to 2048 rows; two waves per row below
+//     6144 rows ([1024,3072] 6.37 -> 5.67, [1024,4096] 8.15 -> 6.68);
+//     one wave per row from 6144 ([1024,8192] 13.4 -> 11.5);
+//   plain 2048: 4 waves (2 float4 each) up to 2048 rows, then two
+//     waves per row ([2048,3072] 10.3 -> 9.65, [2048,8192] 25.1 ->
+//     22.9, at the same-size copy's speed);
+//   add forms 1024: 4 waves below 1024 rows (more loads in flight);
+//     two waves per row below 4096 ([1024,2048] 7.67 -> 6.51); one
+//     wave per row below 16384 ([1024,4096] 13.8 -> 11.4, [1024,8192]
+//     about even); 4 waves again from 16384 ([1024,16384] 44.0
+//     against 46.0 for one wave);
+//   add forms 2048: 4 waves below 2048 rows; two waves per row below
+//     4096 ([2048,2048] 13.5 -> 11.5); one wave per row from 4096
+//     ([2048,4096] 23.9 -> 21.9).
+constexpr int kRmsMaxVec = 256 * 8;
+
+int rms_lanes(int nvec, bool plain, int64_t nr) {
+    if (nvec <= 128) {
+        return nvec <= 16 ? 16 : nvec <= 32 ? 32 : nvec <= 64 ? 64 : 128;
+    }
+    if (nvec == 256) {
+        return plain ? (nr <= 2048 ? 256 : nr < 6144 ? 128 : 64) : (nr < 1024 || nr >= 16384 ? 256 : nr < 4096 ? 128 : 64);
+    }
+    if (nvec == 512) {
+        return plain ? (nr <= 2048 ? 256 : 128) : (nr < 2048 ? 256 : nr < 4096 ? 128 : 64);
+    }
+    return 256;
+}
+
 template <int WT, int MODE> shp_status_t launch_norm(const NormArgs & a, bool vec, hipStream_t stream) {
     if (dry_run()) {
         return SHP_OK;
@@ -597,7 +630,8 @@ template <int WT, int MODE> shp_status_t launch_norm(const NormArgs & a, bool ve
         return launch_status();
     };
     const int nvec = a.ne0 / 4;
-    if (vec && nvec <= 256 * 8) {
+    if (vec && nvec <= kRmsMaxVec) {
+        const int lanes = rms_lanes(nvec, MODE == kPlain, a.nrows);
         if (nvec <= 16) {
             return go(k_rms_norm_vec<16, 1, WT, MODE>, 16);
         }
@@ -610,34 +644,12 @@ template <int WT, int MODE> shp_status_t launch_norm(const NormArgs & a, bool ve
         if (nvec <= 128) {
             return go(k_rms_norm_vec<128, 1, WT, MODE>, 2);
         }
-        // Rows of 1024 / 2048: how many waves share a row, by row count.
-        // Measured on MI355X (cold, us; 4 waves per row first, then the pick):
-        //   plain 1024: 4 waves up to 2048 rows; two waves per row below
-        //     6144 rows ([1024,3072] 6.37 -> 5.67, [1024,4096] 8.15 -> 6.68);
-        //     one wave per row from 6144 ([1024,8192] 13.4 -> 11.5);
-        //   plain 2048: 4 waves (2 float4 each) up to 2048 rows, then two
-        //     waves per row ([2048,3072] 10.3 -> 9.65, [2048,8192] 25.1 ->
-        //     22.9, at the same-size copy's speed);
-        //   add forms 1024: 4 waves below 1024 rows (more loads in flight);
-        //     two waves per row below 4096 ([1024,2048] 7.67 -> 6.51); one
-        //     wave per row below 16384 ([1024,4096] 13.8 -> 11.4, [1024,8192]
-        //     about even); 4 waves again from 16384 ([1024,16384] 44.0
-        //     against 46.0 for one wave);
-        //   add forms 2048: 4 waves below 2048 rows; two waves per row below
-        //     4096 ([2048,2048] 13.5 -> 11.5); one wave per row from 4096
-        //     ([2048,4096] 23.9 -> 21.9).
-        const int64_t nr = a.nrows;
-        if (nvec == 256 && MODE == kPlain && nr > 2048) {
-            return nr < 6144 ? go(k_rms_norm_vec<128, 2, WT, MODE>, 2) : go(k_rms_norm_vec<64, 4, WT, MODE>, 4);
+        // (fewer than 256 lanes from here on: rows of 256 or 512 float4)
+        if (lanes == 128) {
+            return nvec == 256 ? go(k_rms_norm_vec<128, 2, WT, MODE>, 2) : go(k_rms_norm_vec<128, 4, WT, MODE>, 2);
         }
-        if (nvec == 256 && MODE != kPlain && nr >= 1024 && nr < 16384) {
-            return nr < 4096 ? go(k_rms_norm_vec<128, 2, WT, MODE>, 2) : go(k_rms_norm_vec<64, 4, WT, MODE>, 4);
-        }
-        if (nvec == 512 && MODE == kPlain && nr > 2048) {
-            return go(k_rms_norm_vec<128, 4, WT, MODE>, 2);
-        }
-        if (nvec == 512 && MODE != kPlain && nr >= 2048) {
-            return nr < 4096 ? go(k_rms_norm_vec<128, 4, WT, MODE>, 2) : go(k_rms_norm_vec<64, 8, WT, MODE>, 4);
+        if (lanes == 64) {
+            return nvec == 256 ? go(k_rms_norm_vec<64, 4, WT, MODE>, 4) : go(k_rms_norm_vec<64, 8, WT, MODE>, 4);
         }
         switch ((nvec + 255) / 256) {
             case 1:
@@ -1486,7 +1498,11 @@ bool cache_view(const shp_tensor * cache, const shp_tensor * src, int64_t filled
 //     and rope, as k_rope128 and k_rope128_dec do;
 //   - 256 consecutive float4 of SwiGLU (512, two per lane: 205 us against 198 at
 //     [2048,8192], 10.4 against 9.8 at [1024,509]).
-// The arithmetic is the single kernels' (the double row sums in another order).
+// The arithmetic is the single kernels', the order of the double row sums
+// included: where those share a row among fewer lanes (rms_lanes), a row's
+// squares go through LDS and are added as those lanes add them (REGROUP: rows of
+// 1024 or 2048, many positions; 8192 at 2048 197.1 us, 196.9 with the sums in this
+// kernel's own order).
 // HBM-bound for a prefill, one kernel's latency for a decode step. Measured on
 // MI355X (cold) against the five launches: one token at 1024 8.7 -> 2.2 us, 64
 // 11.5 -> 3.3, 509 17.1 -> 9.8, 4000 70.7 -> 58.8; 8192 at 2048 219.9 -> 198 (6.45
@@ -1518,6 +1534,8 @@ struct LayerArgs {
     int32_t       ne0;
     int32_t       chunks;       // DEC: blocks per position
     float         eps;
+    int32_t       lanes_in;     // REGROUP: lanes that add a row's squares for w_in's norm,
+    int32_t       lanes_post;   // and for w_post's
     int32_t       pad;
 };
 
@@ -1526,7 +1544,20 @@ constexpr int kLayerDecRows = (kLayerBlock - kWave) / kRopeLanes;  // head rows 
 constexpr int kLayerPasses  = 2;                                   // head rows per 16-lane group otherwise
 constexpr int kLayerMaxRows = kLayerPasses * kLayerBlock / kRopeLanes;
 
-template <int WT, int VPL> __device__ __forceinline__ void layer_row(const LayerArgs & a, int64_t row, double (&part)[2][4]) {
+// Wave w's share of a row's squares sq[0, nvec) added by `lanes` lanes: 0 for
+// the waves past them.
+__device__ __forceinline__ double regrouped(const double * sq, int lanes, int nvec) {
+    double acc = 0.0;
+    if (static_cast<int>(threadIdx.x) < lanes) {
+        for (int c = static_cast<int>(threadIdx.x); c < nvec; c += lanes) {
+            acc += sq[c];
+        }
+    }
+    return group_sum<kWave>(acc);
+}
+
+template <int WT, int VPL, bool REGROUP>
+__device__ __forceinline__ void layer_row(const LayerArgs & a, int64_t row, double (&part)[2][4], double (*sq)[VPL * kLayerBlock]) {
     args_in_sgprs(a.x, a.attn, a.mlp, a.w_in, a.w_post, a.xs, a.attns, a.mlps, a.ne0);
     const int     l    = static_cast<int>(threadIdx.x);
     const int     nvec = a.ne0 / 4;
@@ -1559,15 +1590,26 @@ template <int WT, int VPL> __device__ __forceinline__ void layer_row(const Layer
     for (int k = 0; k < VPL; ++k) {
         const int c = k * kLayerBlock + l;
         r[k]        = add4v(v[k], r[k]);
-        accx += sq4v(v[k]);
-        accr += sq4v(r[k]);
+        if constexpr (REGROUP) {  // (c < nvec: whole rows of VPL * 256 float4)
+            sq[0][c] = sq4v(v[k]);
+            sq[1][c] = sq4v(r[k]);
+        } else {
+            accx += sq4v(v[k]);
+            accr += sq4v(r[k]);
+        }
         if (c < nvec) {
             st_stream(rp + c, r[k]);
             st_stream(op + c, add4v(r[k], m[k]));
         }
     }
-    accx           = group_sum<kWave>(accx);
-    accr           = group_sum<kWave>(accr);
+    if constexpr (REGROUP) {
+        __syncthreads();
+        accx = regrouped(sq[0], a.lanes_in, nvec);
+        accr = regrouped(sq[1], a.lanes_post, nvec);
+    } else {
+        accx = group_sum<kWave>(accx);
+        accr = group_sum<kWave>(accr);
+    }
     const int wave = l / kWave;
     if (l % kWave == 0) {
         part[0][wave] = accx;
@@ -1658,12 +1700,14 @@ __device__ __forceinline__ void layer_rope(const RopeArgs & a, int64_t pi, int r
     }
 }
 
-template <int WT, int VPL, bool DEC> __global__ __launch_bounds__(kLayerBlock) void k_layer_step(const LayerArgs a) {
+template <int WT, int VPL, bool DEC, bool REGROUP = false>
+__global__ __launch_bounds__(kLayerBlock) void k_layer_step(const LayerArgs a) {
     __shared__ double s_part[2][4];
+    __shared__ double s_sq[REGROUP ? 2 : 1][REGROUP ? VPL * kLayerBlock : 1];
     __shared__ f32x4  s_cos[16], s_sin[16];
     const uint32_t    b = blockIdx.x;
     if (b < a.rope_first) {
-        layer_row<WT, VPL>(a, b, s_part);
+        layer_row<WT, VPL, REGROUP>(a, b, s_part, reinterpret_cast<double(*)[VPL * kLayerBlock]>(s_sq));
     } else if (b < a.swiglu_first) {
         const uint32_t j = b - a.rope_first;
         if constexpr (DEC) {
@@ -1688,6 +1732,11 @@ template <int WT> shp_status_t launch_layer(const LayerArgs & a, bool dec, int64
         hipLaunchKernelGGL(dec ? dk : bk, dim3(static_cast<unsigned>(blocks)), dim3(kLayerBlock), 0, stream, a);
         return launch_status();
     };
+    // (many positions: not a decode step's)
+    if (a.lanes_in < kLayerBlock || a.lanes_post < kLayerBlock) {
+        return nvec == kLayerBlock ? go(k_layer_step<WT, 1, false, true>, k_layer_step<WT, 1, false, true>) :
+                                     go(k_layer_step<WT, 2, false, true>, k_layer_step<WT, 2, false, true>);
+    }
     if (nvec <= kLayerBlock) {
         return go(k_layer_step<WT, 1, true>, k_layer_step<WT, 1, false>);
     }
@@ -1762,6 +1811,10 @@ shp_status_t layer_step_launch(const shp_layer_step & s, hipStream_t stream, boo
     a.rope         = plan.args;
     a.ne0          = static_cast<int32_t>(ne0);
     a.eps          = s.eps;
+    // a row of up to 128 float4 is added by as many lanes in both (the others add 0)
+    const int  nvec  = static_cast<int>(ne0 / 4);
+    a.lanes_in       = nvec <= 128 ? kLayerBlock : rms_lanes(nvec, true, t);
+    a.lanes_post     = nvec <= 128 ? kLayerBlock : rms_lanes(nvec, false, t);
     const bool dec = t <= kRopeDecMaxPos;
     a.chunks       = static_cast<int32_t>((rows + kLayerDecRows - 1) / kLayerDecRows);
     const int64_t rope = dec ? t * a.chunks : t, act = (a.act4 + kLayerBlock - 1) / kLayerBlock;

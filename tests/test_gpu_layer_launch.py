@@ -3,8 +3,8 @@ to past the decode form's 64, hidden sizes of one to four float4 a lane, head
 counts that end inside a block and past what the launch takes (the five
 launches then), every gain type, strided rows, and outputs laid over inputs,
 where the step keeps the five launches' order. Every output equals the single
-entry points' bit for bit (the row sums are double: their order may show only
-on an f32 rounding boundary, which these fixed inputs do not meet)."""
+entry points' bit for bit, also where the single norms share a row among fewer
+lanes and rows lie on an f32 rounding boundary of their sum of squares."""
 import numpy as np
 import pytest
 
@@ -83,3 +83,36 @@ def test_outputs_over_inputs_keep_the_launch_order(gpu, over):
         if n in over.values():
             continue        # overwritten by the later output
         assert_bitexact(_np(got[n]), ref[n])
+
+
+def _boundary_rows(H):
+    """Rows whose sum of squares is halfway between two f32, and moves off it only
+    if the two smallest squares (0.3 ulp of the double sum each) meet before they
+    meet the largest: at float4 64 and 192 if 128 lanes share the row, not if 64 or
+    256 do; at 65 and 193 if 64 or 128 do. 1.25^2 has an even f32 mantissa, and at
+    eps 1e-6 (512 float4: other leading values too) the scale shows the step."""
+    rows = []
+    for big in (1.0, 1.25, 1.375, 1.125):
+        for p, q in ((64, 192), (65, 193), (64, 128), (65, 129), (128, 192), (3, 67)):
+            x = np.zeros(H, np.float32)
+            x[0], x[1] = big, np.sqrt(np.spacing(np.float32(big) * np.float32(big)) / 2)
+            x[4 * p], x[4 * q] = (np.sqrt(0.3 * 2.0 ** -52),) * 2
+            rows.append(x)
+    return np.stack(rows)
+
+
+@pytest.mark.parametrize("H,T", [(1024, t) for t in (1023, 1024, 2048, 2049, 4095, 4096, 6143, 6144, 16383, 16384)] +
+                         [(2048, t) for t in (2047, 2048, 2049, 4095, 4096)] + [(512, 2100), (256, 1025), (1020, 3000)])
+def test_many_positions_add_their_rows_as_the_single_norms_do(gpu, H, T):
+    import torch
+    a = _inputs(T, H, 4, 1, 1, torch.float32, T)
+    rows = torch.from_numpy(_boundary_rows(H)).cuda() if H >= 1020 else a["x"][:8].clone()
+    n = rows.shape[0]
+    a["w_in"].fill_(1.0)
+    a["w_post"].fill_(1.0)
+    for at in (0, T // 2, T - n):
+        a["x"][at:at + n] = rows
+        a["attn_out"][at:at + n] = 0.0
+    got, ref = _step(gpu, a), _singles(gpu, a)
+    for name in ref:
+        assert_bitexact(_np(got[name]), _np(ref[name]))
