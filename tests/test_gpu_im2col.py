@@ -216,3 +216,19 @@ def test_im2col_window_walks(gpu, IC, IW, K, s0, p0, d0, layout):
     view = pick(torch.full(shape, 7.0, device="cuda"))
     view.copy_(_t(gpu, x))
     _check(gpu.im2col(view, K, s0, p0, d0), _cols_ref(x, K, s0, p0, d0, R.F32), R.F32)
+
+
+@pytest.mark.parametrize("N,IC,IW,K,s0,p0,d0", [(1, 131, 64037, 3, 1, 1, 1), (1, 33, 254203, 3, 1, 5, 5), (2, 70, 59921, 4, 3, 2, 1),
+                                                (1, 4099, 2047, 3, 2, 300, 1), (1, 5, 1700003, 5, 1, 2, 1), (3, 64, 43691, 7, 1, 9, 3)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_im2col_window_by_four_samples(gpu, N, IC, IW, K, s0, p0, d0, f16):
+    """Inputs large enough for it: rows of every remainder, in a wider tensor
+    whose neighbours (7) must not show; every value is a copy (F16: rounded)."""
+    import torch
+    buf = torch.full((N, IC + 1, IW + 3), 7.0, device="cuda")
+    x = buf[:, 1:, 2:2 + IW]
+    x.normal_()
+    dt = torch.float16 if f16 else torch.float32
+    got = gpu.im2col(x, K, s0, p0, d0, dt)
+    taps = torch.nn.functional.pad(x.to(dt), (p0, p0)).unfold(2, (K - 1) * d0 + 1, s0)[..., ::d0]      # N, IC, OW, K
+    assert torch.equal(got, taps.permute(0, 2, 1, 3).reshape(got.shape))

@@ -153,3 +153,16 @@ def test_a_launch_ends_below_two_to_the_32_threads():
         (st, ls), = record([_layer_step(T)])
         assert st == 0 and all(g[0] * b[0] < 2 ** 32 for _, g, b, _ in ls)
         assert len(ls) == (1 if T <= 8380000 else 5), (T, ls)
+
+
+def test_im2col_reads_a_small_time_major_input_by_value():
+    """The window walk (the last template argument: 0 by value, 1 four samples, 2 four
+    channels) by the input's size and layout."""
+    def walk(x, k, ow, type_=0):
+        kernel = t(k, x["ne"][1])
+        (st, ls), = record([("shp_im2col", kernel, x, 1, 0, 1, t(x["ne"][1] * k, ow, type_=type_))])
+        assert st == 0
+        return int(re.findall(r"Li(\d+)E", ls[0][0])[-1])
+    assert [walk(t(L, C), 3, L - 2, ty) for L, C in ((4136, 256), (65536, 64), (131072, 64)) for ty in (0, 1)] == [0, 0, 0, 0, 1, 1]
+    assert walk(t(1000, 80, nb=[4 * 80, 4]), 3, 998) == 2       # channel-major
+    assert walk(t(1000, 80, nb=[8, 8000]), 3, 998) == 0         # every other sample
