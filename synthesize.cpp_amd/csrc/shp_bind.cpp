@@ -3,12 +3,14 @@
 //
 //   bind(handle, name)  -> callable(arg, ...) -> status
 //   describe(tensor)    -> the bytes of its shp_tensor
-//   types(block, shape) names synth_hip.BlockTensor and its ctypes ShpTensor
 //
 // handle is the loaded library's dlopen handle (ctypes' CDLL._handle), so a
 // process may bind any build of the library. Each C parameter is converted
 // from its Python argument by its type: a tensor pointer from a torch tensor, a
-// BlockTensor or None, numbers from numbers, a stream from its address. Two
+// BlockTensor or None, numbers from numbers, a stream from its address. A
+// BlockTensor and a ctypes ShpTensor are known by an attribute of their class
+// (SHP_BLOCKS, SHP_TENSOR), not by the class: a program that loads or reloads the
+// Python half twice has two of each, and tensors of both. Two
 // entry points start with an array of tensors and its length: there alone a list
 // or tuple is taken, of that length. shp_im2col starts with a kernel of which
 // only the shape is read: that is a ShpTensor too. The GIL is released while the
@@ -38,13 +40,27 @@
 
 namespace {
 
-PyObject * g_data = nullptr;  // interned attribute names of BlockTensor
-PyObject * g_ne0  = nullptr;
-PyObject * g_type = nullptr;
-PyObject * g_size = nullptr;
+PyObject * g_data   = nullptr;  // interned attribute names of BlockTensor
+PyObject * g_ne0    = nullptr;
+PyObject * g_type   = nullptr;
+PyObject * g_size   = nullptr;
+PyObject * g_blocks = nullptr;  // ... and the class attributes that mark it and ShpTensor
+PyObject * g_tensor = nullptr;
 
-PyObject * g_block = nullptr;  // the classes named by types()
-PyObject * g_shape = nullptr;
+// 1 if o's class has the attribute `mark` (as True), 0 if not, -1 with an error set.
+int marked(PyObject * o, PyObject * mark) {
+    PyObject * v = PyObject_GetAttr(reinterpret_cast<PyObject *>(Py_TYPE(o)), mark);
+    if (v == nullptr) {
+        if (!PyErr_ExceptionMatches(PyExc_AttributeError)) {
+            return -1;
+        }
+        PyErr_Clear();
+        return 0;
+    }
+    const int yes = v == Py_True ? 1 : 0;
+    Py_DECREF(v);
+    return yes;
+}
 
 // shp_tensor for a torch tensor. Dimensions past the tensor's own have extent
 // 1 and the stride of everything below them.
@@ -124,7 +140,7 @@ bool to_tensor(PyObject * o, shp_tensor & d) {
         }
         return true;
     }
-    const int block = g_block == nullptr ? 0 : PyObject_IsInstance(o, g_block);
+    const int block = marked(o, g_blocks);
     if (block < 1) {
         if (block == 0) {
             PyErr_Format(PyExc_TypeError, "expected a tensor, got %s", Py_TYPE(o)->tp_name);
@@ -211,7 +227,7 @@ bool array_arg(PyObject * o, PyObject * count, Slot & s, const shp_tensor *& v) 
 
 // A ctypes ShpTensor, for a parameter of which only the shape is read.
 bool shape_arg(PyObject * o, Slot & s, const shp_tensor *& v) {
-    const int shape = g_shape == nullptr ? 0 : PyObject_IsInstance(o, g_shape);
+    const int shape = marked(o, g_tensor);
     if (shape < 1) {
         return shape == 0 && Arg<const shp_tensor *>::get(o, s, v);
     }
@@ -452,21 +468,7 @@ PyObject * describe(PyObject *, PyObject * o) {
     return nullptr;
 }
 
-PyObject * types(PyObject *, PyObject * args) {
-    PyObject * block = nullptr;
-    PyObject * shape = nullptr;
-    if (!PyArg_ParseTuple(args, "O!O!", &PyType_Type, &block, &PyType_Type, &shape)) {
-        return nullptr;
-    }
-    Py_INCREF(block);
-    Py_INCREF(shape);
-    Py_XSETREF(g_block, block);
-    Py_XSETREF(g_shape, shape);
-    Py_RETURN_NONE;
-}
-
-PyMethodDef kMethods[] = { { "types", types, METH_VARARGS, "types(BlockTensor, ShpTensor)" },
-                           { "describe", describe, METH_O, "describe(tensor) -> the bytes of its shp_tensor" },
+PyMethodDef kMethods[] = { { "describe", describe, METH_O, "describe(tensor) -> the bytes of its shp_tensor" },
                            { "bind", bind, METH_VARARGS, "bind(handle, name) -> callable" },
                            { nullptr, nullptr, 0, nullptr } };
 
@@ -475,10 +477,16 @@ PyModuleDef kModule = { PyModuleDef_HEAD_INIT, "shp_bind", nullptr, -1, kMethods
 }  // namespace
 
 PyMODINIT_FUNC PyInit_shp_bind() {
-    g_data = PyUnicode_InternFromString("data");
-    g_ne0  = PyUnicode_InternFromString("ne0");
-    g_type = PyUnicode_InternFromString("TYPE");
-    g_size = PyUnicode_InternFromString("BYTES");
-    return g_data == nullptr || g_ne0 == nullptr || g_type == nullptr || g_size == nullptr ? nullptr :
-                                                                                           PyModule_Create(&kModule);
+    g_data   = PyUnicode_InternFromString("data");
+    g_ne0    = PyUnicode_InternFromString("ne0");
+    g_type   = PyUnicode_InternFromString("TYPE");
+    g_size   = PyUnicode_InternFromString("BYTES");
+    g_blocks = PyUnicode_InternFromString("SHP_BLOCKS");
+    g_tensor = PyUnicode_InternFromString("SHP_TENSOR");
+    for (PyObject * name : { g_data, g_ne0, g_type, g_size, g_blocks, g_tensor }) {
+        if (name == nullptr) {
+            return nullptr;
+        }
+    }
+    return PyModule_Create(&kModule);
 }

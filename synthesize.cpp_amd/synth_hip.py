@@ -31,6 +31,7 @@ Q5_K_BLOCK_BYTES, Q5_K_BLOCK_ELEMS = 176, 256
 
 
 class ShpTensor(ctypes.Structure):
+    SHP_TENSOR = True  # how csrc/shp_bind.cpp knows it
     _fields_ = [("type", ctypes.c_int32), ("reserved", ctypes.c_int32), ("ne", ctypes.c_int64 * 4),
                 ("nb", ctypes.c_size_t * 4), ("data", ctypes.c_void_p)]
 
@@ -174,6 +175,7 @@ class BlockTensor:
     """A block-quantized tensor held as raw blocks: `data` is a uint8 torch
     tensor of shape (..., rows, ne0/ELEMS*BYTES); ne0 is the logical row length."""
     TYPE = ELEMS = BYTES = None
+    SHP_BLOCKS = True  # how csrc/shp_bind.cpp knows it
 
     def __init__(self, data, ne0):
         assert ne0 % self.ELEMS == 0
@@ -210,7 +212,6 @@ def _binding():
         mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("shp_bind", BIND_PATH,
                                                                                     loader=loader))
         loader.exec_module(mod)
-        mod.types(BlockTensor, ShpTensor)
         _bind = mod
     return _bind
 

@@ -124,3 +124,19 @@ def test_public_calls_refuse_what_is_no_tensor(monkeypatch):
                      a, a, [], a, 1e-6, a, 8, 1e6), lambda: S.im2col(a, 3.0, out=a), lambda: S.get_rows_sum([a, [a]], a, out=a)):
         with pytest.raises(TypeError):
             call()
+
+
+def test_tensors_of_another_load_of_the_binding():
+    """A reload, or a second copy of the module, has classes of its own; tensors
+    made with either go through both, in any order of loading."""
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("synth_hip_again", S.__file__)
+    again = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(again)
+    raw, a = torch.zeros(3, 68, dtype=torch.uint8), torch.zeros(2, 8)
+    for first, second in ((S, again), (again, S)):
+        want = bytes(first.desc(first.Q8Tensor(raw, 64)))
+        assert bytes(second.desc(second.Q8Tensor(raw, 64))) == want
+        assert bytes(first.desc(second.Q8Tensor(raw, 64))) == want and bytes(second.desc(first.Q8Tensor(raw, 64))) == want
+        for shape in (first.kernel_shape(3, 2), second.kernel_shape(3, 2)):
+            assert first._fn("shp_im2col")(shape, a, 1, 0, 1, a, 0) != S.OK
