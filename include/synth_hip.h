@@ -602,7 +602,11 @@ shp_status_t shp_cont_add_leaky_relu(const shp_tensor * x,
  * The non-GEMM node runs of one Qwen3 decoder layer,
  * src/arch/qwen3-tts/operations.cpp:84-147, in the layer's order. The
  * layer's matrix products and its attention run between these node runs in
- * a model, so their outputs are inputs here:
+ * a model, so their outputs are inputs here; they in turn depend on this call's
+ * own outputs (q and k on normed, attn_out on q_out and k_out, gate and up on
+ * mlp_in, mlp_out on act), so a model that computes a layer calls the single
+ * entry points between its products, and this call is for a caller that holds
+ * every input of the step:
  *   normed       = rms_norm(x)*w_in                        (:85-86)
  *   q_out, k_out = rope(rms_norm(q)*wq), rope(rms_norm(k)*wk)  (:98-104)
  *   resid        = x + attn_out                            (:143)
@@ -613,8 +617,9 @@ shp_status_t shp_cont_add_leaky_relu(const shp_tensor * x,
  * and the layouts are the 128-wide rope's and whole aligned float4 rows of up
  * to 4096 values; otherwise five, each the launch of shp_rms_norm_mul,
  * shp_qk_norm_rope, shp_add_rms_norm_mul, shp_swiglu and shp_add, in this
- * order. The same bits either way. Every tensor's presence, type and shape is checked first:
- * a malformed step returns SHP_ERR_INVALID_ARG with nothing enqueued.
+ * order. The same bits either way. Every tensor's presence, type and shape is
+ * checked first: a malformed step returns SHP_ERR_INVALID_ARG with nothing
+ * enqueued.
  * x, normed, attn_out, resid, mlp_in, mlp_out, out: F32 [hidden, T];
  * q, q_out: F32 [head_dim, q_heads, T]; k, k_out: F32 [head_dim, kv_heads, T];
  * gate, up, act: F32 [ffn, T]; pos: I32 [T]; w_in, w_post: [hidden] and

@@ -18,9 +18,11 @@
 //      to f32, or 0 where the envelope is below 1e-11.
 // The window is the periodic Hann window rounded to f32, the value the host
 // code tabulates. The turn of bin b at sample s is taken from the twiddle of
-// (b*s) mod n_fft, and A and B are summed apart, each product fused with its
-// sum: the host computes cos(2 pi b s / n_fft) of the unreduced product and one
-// sum, which differs in the last bits of the double.
+// (b*s) mod n_fft, A and B are summed apart, each product fused with its sum,
+// and the division by n_fft is a product with its reciprocal: the host computes
+// cos(2 pi b s / n_fft) of the unreduced product, one sum and its quotient, which
+// differ in the last bits of the double. (k_istft_direct keeps the one sum and
+// the division.)
 //
 // Bound by the f64 arithmetic and its latency (an exp, a sine and a sincos per
 // bin); every sample taking its frames' whole DFT read each bin n_fft times from

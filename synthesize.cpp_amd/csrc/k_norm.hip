@@ -383,11 +383,20 @@ __global__ __launch_bounds__(kLayerNormWide) void k_layer_norm_wide(const NormAr
 }
 
 // Lanes per row: enough that a lane holds one float4 where the rows are many
-// (the RMSNorm rule), and 1024 where they are too few to fill the chip with
-// 256-thread blocks (kLayerNormFewRows: one block per CU) or too long for one.
-// From kLayerNormManyRows rows of up to 2048 values the chip is full either way
-// and fewer lanes per row, with more loads in flight each, are ahead, as for
-// the RMSNorm (8192 rows of 1024: 256 lanes 15.7 us, 64 lanes 13.5).
+// (the RMSNorm rule), and 1024 where they are at most kLayerNormFewRows (a block
+// per CU) or too long for 256. From kLayerNormManyRows rows of up to 2048 values
+// the chip is full either way and fewer lanes per row, with more loads in flight
+// each, are ahead, as for the RMSNorm (8192 rows of 1024: 256 lanes 15.7 us, 64
+// lanes 13.5). Both sides of each line (MI355X, cold, us), rows x values:
+//   - past kLayerNormFewRows: 300 x 4096 256 lanes 4.3, 1024 5.4; 600 x 8192 7.7
+//     and 10.3; 1024 x 2048 4.9 and 8.0. Below it the blocks' ramps differ less,
+//     and 256 lanes stay ahead up to 8192 values (16 x 2048 2.7 and 3.3, 256 x
+//     4096 4.1 and 4.6, 256 x 8192 5.3 and 5.6); longer rows need the 1024;
+//   - past kLayerNormManyRows: 3000 x 1024 128 lanes 6.0, 256 7.0, 64 5.8; 8000 x
+//     1024 12.8, 14.7, 13.2; 3000 x 2048 128 lanes 10.9, 256 11.0, 64 9.0; 8000 x
+//     2048 23.9, 22.8, 23.7;
+//   - 257-512 values: 128 lanes; 64 with two float4 are ahead (1024 x 512 3.2 and
+//     3.4, 8000 x 300 5.6 and 8.5).
 constexpr int64_t kLayerNormFewRows  = 256;
 constexpr int64_t kLayerNormManyRows = 2048;
 
@@ -1487,8 +1496,12 @@ bool cache_view(const shp_tensor * cache, const shp_tensor * src, int64_t filled
 // ---------------------------------------------------------------------------
 
 // shp_layer_nongemm_step's five node runs (qwen3-tts/operations.cpp:84-147)
-// have the GEMM and attention outputs as inputs, so none of them waits for
-// another but the adds, which work row by row: one launch takes them all. Its
+// in one call have the GEMM and attention outputs as inputs, so none of them
+// waits for another but the adds, which work row by row: one launch takes them
+// all. (Within a model's layer they do wait: q and k are products of normed,
+// attn_out needs q_out and k_out, gate and up are products of mlp_in, mlp_out of
+// act. A synthesis issues the single runs between its matrix products and gains
+// nothing here; this is for a caller that holds all of a step's inputs.) Its
 // blocks have one of three jobs:
 //   - a row each: x, the attention output and the MLP output read once;
 //     rms(x)*w_in, x + attn, rms(x + attn)*w_post and (x + attn) + mlp written.

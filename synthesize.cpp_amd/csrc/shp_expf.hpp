@@ -8,7 +8,7 @@
 //   T[j] = 2^(j/64) rounded to double, p(r) = 1 + c1 r + c2 r^2 + c3 r^3 + c4 r^4
 //   with c_n = (ln2/64)^n / n!, the Taylor series of e^(r ln2/64).
 // Error of the double result before the f32 rounding: truncation
-// (|r ln2/64| <= 0.0055)^5/5! < 4e-14, z's rounding (|z| < 9600) < 2e-14 in
+// (|r ln2/64| <= 0.0055)^5/5! < 4e-14, z's rounding (|z| < 9603) < 2e-14 in
 // the result, table and product roundings ~2^-52: about 2^-44 relative, so
 // the f32 rounding is the correct one unless e^x lies within ~2^-44 of an f32
 // rounding boundary. tests/host/expf_check.cpp compares every f32 input with
@@ -77,7 +77,7 @@ template <class Tab> SHP_HD inline float exp_f32_rn(float x, const Tab & tab) {
     const bool   nan = x != x;
     const float  xc  = std::fmin(std::fmax(x, -104.0f), 89.0f);  // max/min instructions; a NaN gives -104
     const double z  = static_cast<double>(xc) * kExp64OverLn2;
-    const double m  = z + kExpRound;  // rint(z) in the low bits (|z| < 9600)
+    const double m  = z + kExpRound;  // rint(z) in the low bits (|z| < 9603)
     const double r  = z - (m - kExpRound);
     double       p  = std::fma(r, kExpC4, kExpC3);
     p               = std::fma(p, r, kExpC2);
