@@ -1271,7 +1271,10 @@ PMC_OPS = [
     ("im2col K=7 d=3 f16 [128,131072]", 301989888), ("col2im_1d K=4 s=2 [128,131072]", 201326592),
     ("pad: spread x2 [128,1,65536]", 100663296), ("repeat: frames x2 [128,1,65536]", 100663296),
     ("pad_ext: time +3/+4 [131072,128]", 134221312),
-    ("acc: codec run +8176@16 into text [2048,8192]", 201195520)]
+    ("acc: codec run +8176@16 into text [2048,8192]", 201195520),
+    ("layer non-GEMM step, one launch [2048,8192]", 1275109888), ("norm [24001,128]", 24577024),
+    ("sum_rows [24001,128]", 12289024), ("soft_max_ext+mask [1021,1021,16]", 137602212),
+    ("cont(transpose) [256,31999]", 65533952), ("add bias[1,C] time-major [24001,128]", 24577536)]
 
 
 def pmc_large(S, torch):
@@ -1302,6 +1305,10 @@ def pmc_large(S, torch):
     sp_x, sp_y = randn(65536, 1, 128), empty(65536, 2, 128)   # the spread and the frame doubling
     ed_x, ed_y = randn(128, 131072), empty(128, 131079)        # edge padding +3/+4 along time
     ac_a, ac_b, ac_y = randn(8192, 2048), randn(8176, 2048), empty(8192, 2048)
+    ly_m, ly_o = randn(8192, 2048), {n: empty(8192, 2048) for n in ("normed", "resid", "mlp_in", "out")}
+    ly_o.update(q_out=empty(8192, 16, 128), k_out=empty(8192, 8, 128), act=empty(8192, 6144))
+    od_x, od_s, od_t = randn(128, 24001), randn(16, 1021, 1021), randn(31999, 256)   # odd rows
+    od_m = torch.triu(torch.full((1, 1021, 1021), float("-inf"), device="cuda"), 1)
     fns = [lambda: S.rms_norm_mul(x2, w2, 1e-6), lambda: S.add_rms_norm_mul(x2, x2b, w2, 1e-6),
            lambda: S.qk_norm_rope(q, k, wq, wk, 1e-6, pos, 128, 1e6), lambda: S.swiglu(gt, up),
            lambda: S.add(x2, x2b), lambda: S.snake(xs, al), lambda: S.snake_beta(xs, la, lb),
@@ -1314,7 +1321,10 @@ def pmc_large(S, torch):
            lambda: S.im2col(tr, 7, 1, 9, 3, out=cols7), lambda: S.col2im_1d(c2i, 2, 128, 1, out=ty),
            lambda: S.pad_ext(sp_x, [0, 0], [0, 1], out=sp_y), lambda: S.repeat(sp_x, (65536, 2, 128), out=sp_y),
            lambda: S.pad_ext(ed_x, [3], [4], out=ed_y),
-           lambda: S.acc(ac_a, ac_b, 8192, 8192 * 8192, 8192 * 8192, 16 * 8192, out=ac_y)]
+           lambda: S.acc(ac_a, ac_b, 8192, 8192 * 8192, 8192 * 8192, 16 * 8192, out=ac_y),
+           lambda: S.layer_nongemm_step(x2, w2, q, k, wq, wk, pos, x2b, w2, gt, up, ly_m, 1e-6, 128, 1e6, outs=ly_o),
+           lambda: S.norm(od_x, 1e-5), lambda: S.sum_rows(od_x), lambda: S.soft_max_ext(od_s, od_m, 0.0884),
+           lambda: S.cpy(od_t.t()), lambda: S.add(od_x, tb)]
     n = CALIB_BYTES // 4
     src = torch.randn(n, device="cuda")
     dst = torch.empty_like(src)
