@@ -415,9 +415,14 @@ template <int MK> __global__ __launch_bounds__(kSoftMaxBlock) void k_soft_max_bl
     }
 }
 
-// The forms' rule reads only the row count and length, so that the causal launch
-// adds a row in the order that the softmax alone does: diag_mask_inf and
-// soft_max_ext come out bit for bit the same in one launch.
+// Rows of 257 to 512 float4 in one wave (launch_rows4).
+inline bool one_wave(int64_t nrows, int nc, bool mask) {
+    return nrows > (nc > 400 ? 2688 : 4608) && nrows <= (mask ? 3328 : 6144);
+}
+
+// The forms' rule reads the row count and length, and whether a mask tensor is
+// added, so that the causal launch adds a row in the order that the softmax alone
+// does: diag_mask_inf and soft_max_ext come out bit for bit the same in one launch.
 template <int MK, bool ODD, class Go> shp_status_t launch_rows4(const SoftMaxArgs & a, const Go & go) {
     const int nc = (a.ne0 + 3) / 4;
     if (nc <= 64) {
@@ -458,7 +463,16 @@ template <int MK, bool ODD, class Go> shp_status_t launch_rows4(const SoftMaxArg
     // Many rows: one wave up to 1024 scores, two up to 2048 (8 heads of 2000 x
     // 2000, one wave / two / four: no mask 46.3 us / 44.5 / 45.1, with a mask 57.1
     // / 49.8 / 50.4, causal 39.6 / 35.8 / 40.2; 16 of 1100 x 1100: 36.5 / 38.5 /
-    // 41.8, 41.7 / 40.4 / 45.2, 26.4 / 26.8 / 32.8).
+    // 41.8, 41.7 / 40.4 / 45.2, 26.4 / 26.8 / 32.8), but one where two waves a
+    // row begin a second round of the chip that one does not, until the rounds even
+    // out: rows past 1600 scores from some 2700, shorter ones from 4600 (no mask and
+    // causal, one wave / two: 2560 x 1800 9.6 / 8.3 and 10.3 / 9.1, 3072 x 2000 10.2 /
+    // 13.4 and 11.3 / 10.7, 4096 x 2000 12.7 / 14.0 and 13.0 / 13.7, 5120 x 1200 12.4 / 12.5
+    // and 10.9 / 12.5, 8192 x 2000 25.6 / 24.6 and 25.5 / 24.3; with a mask 3072 x 2000
+    // 11.1 / 12.8, 5120 x 1800 18.4 / 17.8).
+    if (nc > 256 && nc <= 512 && one_wave(a.nrows, nc, MK == kMaskTensor)) {
+        return go(k_soft_max_rows4<1, 8, MK, ODD>, 4, 256);
+    }
     return nc <= 256  ? go(k_soft_max_rows4<1, 4, MK, ODD>, 4, 256) :
            nc <= 512  ? go(k_soft_max_rows4<2, 4, MK, ODD>, 2, 256) :
            nc <= 1024 ? go(k_soft_max_rows4<4, 4, MK, ODD>, 1, 256) :

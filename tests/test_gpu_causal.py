@@ -86,7 +86,8 @@ def test_codec_encoder_attention_softmax_through_the_executor(gpu):
 
 
 @pytest.mark.parametrize("H,T,N,n_past", [(1, 2048, 1025, 0), (1, 2050, 1028, 300), (2, 1100, 1100, 0), (2, 1101, 1101, 0),
-                                          (1, 2049, 2047, 0), (2, 1024, 2048, 1024), (1, 2100, 1537, 5)])
+                                          (1, 2049, 2047, 0), (2, 1024, 2048, 1024), (1, 2100, 1537, 5), (1, 2690, 2047, 3),
+                                          (2, 1500, 1700, 200), (1, 6144, 1601, 0), (1, 4609, 1026, 0)])
 def test_many_rows_of_1025_to_2048(gpu, H, T, N, n_past):
     """From 2048 rows, at rows of several waves and at odd ones: bit-identical to
     the two nodes, infinities and NaN in hidden scores included, and the

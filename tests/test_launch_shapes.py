@@ -5,7 +5,7 @@ import pytest
 
 from launches import layer, record, t
 
-ROWS = [1, 8, 64, 65, 250, 256, 257, 640, 1023, 1024, 2047, 2048, 2049, 4096, 4097, 16384, 40000]
+ROWS = [1, 8, 64, 65, 250, 256, 257, 640, 1023, 1024, 2047, 2048, 2049, 2689, 3329, 4096, 4097, 6144, 6145, 16384, 40000]
 WIDTHS = [1, 3, 63, 64, 65, 100, 127, 128, 129, 192, 200, 255, 256, 257, 301, 320, 321, 384, 500, 511, 512, 513, 700, 767,
           1000, 1021, 1023, 1024, 1025, 1100, 1500, 2000, 2047, 2048, 2049, 4095, 4096, 4097, 8191, 8193, 16383, 16384,
           16385, 20000]
@@ -19,21 +19,32 @@ def test_the_causal_softmax_takes_the_form_of_the_softmax_alone():
     for rows in ROWS:
         for n in WIDTHS:
             x, y = t(n, rows), t(n, rows)
-            calls += [("shp_soft_max_ext", x, None, 0.5, 0.0, y), ("shp_soft_max_causal", x, 0, 0.5, y),
-                      ("shp_soft_max_ext", x, t(n, rows), 0.5, 0.0, y)]
+            calls += [("shp_soft_max_ext", x, None, 0.5, 0.0, y), ("shp_soft_max_causal", x, 0, 0.5, y)]
     got = record(calls)
     # k_soft_max_wave<K, MK>, k_soft_max_rows4<WPR, K4, MK, ODD, BLOCK>, k_soft_max_block<MK>
     mask = {"wave": 1, "rows4": 2, "block": 0}
-    for i in range(0, len(got), 3):
+    for i in range(0, len(got), 2):
         forms = []
-        for st, launches in got[i:i + 3]:
+        for st, launches in got[i:i + 2]:
             assert st == 0 and len(launches) == 1
             name, grid, block, _ = launches[0]
             kind, args = re.search(r"k_soft_max_(wave|rows4|block)I((?:L[ib]\d+E)+)E", name).groups()
             args = re.findall(r"L[ib](\d+)E", args)
             del args[mask[kind]]
             forms.append((kind, args, grid, block))
-        assert forms[0] == forms[1] == forms[2], calls[i]
+        assert forms[0] == forms[1], calls[i]
+
+
+def test_many_long_softmax_rows_take_one_wave_where_two_begin_another_round():
+    """k_soft_max_rows4<waves, ...> of 1025 to 2048 scores, each side of every line."""
+    def waves(rows, n, mask):
+        x = t(n, rows)
+        return ("shp_soft_max_ext", x, t(n, rows) if mask else None, 0.5, 0.0, x)
+    cases = [(2688, 1601, False, 2), (2689, 1601, False, 1), (2689, 1600, False, 2), (4608, 1600, False, 2), (4609, 1025, False, 1),
+             (6144, 2048, False, 1), (6145, 2048, False, 2), (4609, 1600, True, 2),
+             (2688, 2048, True, 2), (2689, 1601, True, 1), (3328, 2048, True, 1), (3329, 2048, True, 2), (40000, 1025, False, 2)]
+    names = _kernels([waves(*c[:3]) for c in cases])
+    assert [int(re.search(r"rows4ILi(\d+)E", k[0]).group(1)) for k in names] == [c[3] for c in cases]
 
 
 def _kernels(calls):
