@@ -16,11 +16,13 @@
 // entry (no loop: a block's stores never wait at a barrier):
 //   1. the tile's input window (ICT channel rows of (OWT-1)*s0 + (K-1)*d0 + 1
 //      samples, zeros past the input's ends) goes to LDS, consecutive lanes on
-//      consecutive addresses: along time for a time-contiguous x, along
-//      channels for a channel-contiguous x (the transposed view of a
-//      channel-major activation, so the ggml_cont the reference puts in front
-//      of im2col is not needed); four values a lane for the latter and for a
-//      large x (kIm2colTimeQuads), one a lane otherwise;
+//      consecutive addresses, four values a lane (by_value's calls: one): along time
+//      for a time-contiguous x, along channels for a channel-contiguous x (the
+//      transposed view of a channel-major activation, so the ggml_cont the
+//      reference puts in front of im2col is not needed). Value by value, behind
+//      a leaky-ReLU that has just written x (MI355X, both launches): K = 3
+//      [128,131072] 75.3 -> 72.5 us, [256,4136] 10.4 -> 9.1; K = 7 d = 3 F16
+//      [128,131072] 101 -> 89.7;
 //   2. the tile's outputs are written in y's order, V values (16 bytes) per
 //      store. The LDS offsets of the values a store takes repeat with a short
 //      period -- one position's run of ICT*K values, or for a tile of every
@@ -43,13 +45,6 @@ constexpr int kIm2colBlock = 256;
 constexpr int kIm2colLds   = 4480;   // floats of LDS window per block at most (17.5 KB; with the table, 8 blocks per CU)
 constexpr int kIm2colBatch = 8;      // window loads a lane issues before its LDS writes
 constexpr int kIm2colQuads = 4;      // the same for float4 loads
-// Values of a time-contiguous x from which its window is read four at a time: x
-// no longer fits the L2s (32 MB). Behind a leaky-ReLU that has just written it,
-// both launches (MI355X, cold), by value and by four: K = 3 [128,131072] 83.9 and 79.0
-// us, F16 [512,16384] 37.0 and 33.4, K = 7 d = 3 F16 [256,32768] 51.1 and 46.9; but K = 3
-// [256,4136] 8.4 and 9.5, F16 [64,65536] 16.6 and 20.0, d = 5 F16 [512,4096] 11.6 and
-// 15.1. (K = 11 F16 alone [256,4136] 11.4 and 9.0, behind the leaky-ReLU 15.0 and 14.8.)
-constexpr int64_t kIm2colTimeQuads = int64_t{ 1 } << 23;
 constexpr int kIm2colTab   = 1024;   // int16 LDS offsets of the store table (one period)
 
 // Tile shape: ict channels; at least owt positions, or enough for `elems`
@@ -173,7 +168,8 @@ __device__ __forceinline__ int tap_offset(const Im2colArgs & a, uint32_t f, cons
 template <bool FLAT, int V, bool F16, int WALK>
 __global__ __launch_bounds__(kIm2colBlock) void k_im2col(const Im2colArgs a) {
     typedef int16_t         tv __attribute__((ext_vector_type(V > 1 ? V : 2)));  // one store's offsets
-    extern __shared__ float lds[];
+    extern __shared__ f32x4 lds4[];
+    float *                 lds = reinterpret_cast<float *>(lds4);
     __shared__ tv           tabv[V > 1 ? kIm2colTab / V : 1];
     int16_t *               tab = reinterpret_cast<int16_t *>(tabv);
     const int               tid = static_cast<int>(threadIdx.x);
@@ -234,7 +230,7 @@ __global__ __launch_bounds__(kIm2colBlock) void k_im2col(const Im2colArgs a) {
         }
     } else {
         // four at a time from any 4-byte boundary: whole where the row goes on
-        // in memory (past the window's last sample too)
+        // in memory (past the window's last sample too: its row of LDS has room)
         const int most = WALK == kWalkTime ? static_cast<int>(a.iw - iw0 < a.wt + 4 ? a.iw - iw0 : a.wt + 4) : nic;
         const int from = WALK == kWalkTime ? wlo : 0;
         while (s < a.ns) {
@@ -261,10 +257,14 @@ __global__ __launch_bounds__(kIm2colBlock) void k_im2col(const Im2colArgs a) {
 #pragma unroll
             for (int u = 0; u < kIm2colQuads; ++u) {
                 if (at[u] >= 0) {
+                    if constexpr (WALK == kWalkTime) {
+                        *reinterpret_cast<f32x4 *>(lds + at[u]) = v[u];
+                    } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (WALK == kWalkTime ? ch[u] + e < a.wt : ch[u] + e < a.ict) {
-                            lds[at[u] + e * (WALK == kWalkTime ? 1 : a.wtp)] = v[u][e];
+                        for (int e = 0; e < 4; ++e) {
+                            if (ch[u] + e < a.ict) {
+                                lds[at[u] + e * a.wtp] = v[u][e];
+                            }
                         }
                     }
                 }
@@ -371,8 +371,48 @@ inline int64_t window(int64_t owt, int64_t s0, int64_t k, int64_t d0) {
     return (owt - 1) * s0 + (k - 1) * d0 + 1;
 }
 
-inline int64_t padded(int64_t w) {
-    return w | 1;  // an odd row stride spreads a column of the window over the banks
+// LDS row stride of a window of w samples: odd, which spreads a column of the
+// window over the banks; for rows written 16 bytes at a time, an odd number of
+// float4, which spreads 16 channels' taps over all of them.
+inline int64_t padded(int64_t w, bool quads) {
+    return quads ? ((w + 3) / 4 | 1) * 4 : w | 1;
+}
+
+// The most of a wave's 64 lanes that read one LDS bank for the first value of
+// their stores (the others' counts are alike), at a row stride of wtp.
+int bank_depth(const Im2colArgs & a, int v, int64_t wtp) {
+    uint8_t depth[64] = {};
+    int     most = 0, ch = 0, tap = 0, pos = 0;
+    for (int l = 0; l < kWave; ++l) {
+        uint8_t & n = depth[(ch * wtp + static_cast<int64_t>(tap) * a.d0 + static_cast<int64_t>(pos) * a.s0) & 63];
+        most        = ++n > most ? n : most;
+        for (tap += v; tap >= a.k; tap -= a.k) {
+            ch  = ch + 1 < a.ict ? ch + 1 : 0;
+            pos = ch == 0 ? pos + 1 : pos;
+        }
+    }
+    return most;
+}
+
+// Whether F16 columns of a time-contiguous x read the window by value all the
+// same. Eight LDS reads a store make them sensitive to bank conflicts, and at some
+// tap distances the quads' row stride has them: K = 3 with d = 3 or 5, six lanes a
+// bank against two at the odd stride. And few columns a sample leave the launch to
+// its loads where x is between the L2s' size and the memory's. Both launches
+// behind a leaky-ReLU that has just written x, by four and by value (MI355X, cold):
+// K = 3 d = 5 [512,4000] 14.4 us and 11.5, im2col alone 8.4 and 7.0; K = 3 [256,4000]
+// 10.8 and 9.8, alone 6.2 and 6.5; [64,65536] 20.0 and 16.6, alone 10.5 and 9.7; but
+// K = 11 [256,4000] 13.6 and 14.2, alone 8.4 and 10.7, K = 3 [256,1000] alone 5.7 and
+// 6.2, and F32 K = 3 [256,4000] 7.9 and 8.1, alone 4.7 and 5.0.
+bool by_value(const Im2colArgs & a, int64_t n) {
+    const int64_t values = n * a.ic * a.iw;
+    if (a.ict < 32) {  // tiles of fewer channels: by four in all of these
+        return false;
+    }
+    if (bank_depth(a, 8, padded(a.wt, true)) >= 3 * bank_depth(a, 8, padded(a.wt, false))) {
+        return true;
+    }
+    return a.k <= 4 * static_cast<int64_t>(a.s0) && values < (int64_t{ 1 } << 23) && n * a.ow * a.row >= (int64_t{ 3 } << 20);
 }
 
 inline int64_t gcd64(int64_t a, int64_t b) {
@@ -498,8 +538,8 @@ shp_status_t plan_im2col(const shp_tensor * kernel, const shp_tensor * x, int32_
     a.ict              = static_cast<int32_t>(ict);
     a.owt              = static_cast<int32_t>(owt);
     a.wt               = static_cast<int32_t>(wt);
-    pl.walk            = pl.chfast ? kWalkChannels : (nb0 == 4 && N * IC * IW >= kIm2colTimeQuads ? kWalkTime : kWalkValues);
-    a.wtp              = static_cast<int32_t>(padded(wt));
+    pl.walk            = pl.chfast ? kWalkChannels : (nb0 == 4 && !(pl.f16 && by_value(a, N)) ? kWalkTime : kWalkValues);
+    a.wtp              = static_cast<int32_t>(padded(wt, pl.walk == kWalkTime));
     a.tic              = make_fastdiv(static_cast<uint32_t>(tic));
     a.tow              = make_fastdiv(static_cast<uint32_t>(tow));
     a.kdiv             = make_fastdiv(static_cast<uint32_t>(K));

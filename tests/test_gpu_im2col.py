@@ -219,11 +219,13 @@ def test_im2col_window_walks(gpu, IC, IW, K, s0, p0, d0, layout):
 
 
 @pytest.mark.parametrize("N,IC,IW,K,s0,p0,d0", [(1, 131, 64037, 3, 1, 1, 1), (1, 33, 254203, 3, 1, 5, 5), (2, 70, 59921, 4, 3, 2, 1),
-                                                (1, 4099, 2047, 3, 2, 300, 1), (1, 5, 1700003, 5, 1, 2, 1), (3, 64, 43691, 7, 1, 9, 3)])
+                                                (1, 4099, 2047, 3, 2, 300, 1), (1, 5, 1700003, 5, 1, 2, 1), (3, 64, 43691, 7, 1, 9, 3),
+                                                (1, 67, 16411, 3, 1, 1, 1), (2, 96, 1003, 3, 1, 5, 5), (1, 33, 501, 3, 1, 3, 3), (1, 70, 30011, 16, 4, 7, 1)])
 @pytest.mark.parametrize("f16", [False, True])
-def test_im2col_window_by_four_samples(gpu, N, IC, IW, K, s0, p0, d0, f16):
-    """Inputs large enough for it: rows of every remainder, in a wider tensor
-    whose neighbours (7) must not show; every value is a copy (F16: rounded)."""
+def test_im2col_window_walks_by_size(gpu, N, IC, IW, K, s0, p0, d0, f16):
+    """Windows read by four samples, and by value (F16 columns of some taps and
+    sizes): rows of every remainder, in a wider tensor whose neighbours (7) must not
+    show; every value is a copy (F16: rounded)."""
     import torch
     buf = torch.full((N, IC + 1, IW + 3), 7.0, device="cuda")
     x = buf[:, 1:, 2:2 + IW]

@@ -166,14 +166,21 @@ def test_a_launch_ends_below_two_to_the_32_threads():
         assert len(ls) == (1 if T <= 8380000 else 5), (T, ls)
 
 
-def test_im2col_reads_a_small_time_major_input_by_value():
+def test_im2col_reads_a_window_by_value_only_where_that_is_ahead():
     """The window walk (the last template argument: 0 by value, 1 four samples, 2 four
-    channels) by the input's size and layout."""
-    def walk(x, k, ow, type_=0):
-        kernel = t(k, x["ne"][1])
-        (st, ls), = record([("shp_im2col", kernel, x, 1, 0, 1, t(x["ne"][1] * k, ow, type_=type_))])
+    channels) by layout, and for F16 columns by bank conflicts, taps and size."""
+    def walk(x, k, d, ow, type_=0, s0=1):
+        c = x["ne"][1]
+        (st, ls), = record([("shp_im2col", t(k, c), x, s0, 0, d, t(c * k, ow, type_=type_))])
         assert st == 0
         return int(re.findall(r"Li(\d+)E", ls[0][0])[-1])
-    assert [walk(t(L, C), 3, L - 2, ty) for L, C in ((4136, 256), (65536, 64), (131072, 64)) for ty in (0, 1)] == [0, 0, 0, 0, 1, 1]
-    assert walk(t(1000, 80, nb=[4 * 80, 4]), 3, 998) == 2       # channel-major
-    assert walk(t(1000, 80, nb=[8, 8000]), 3, 998) == 0         # every other sample
+    for L, C, k, d, s0, f16, want in [(4136, 256, 3, 1, 1, 0, 1), (65536, 64, 3, 1, 1, 0, 1), (4097, 256, 3, 1, 1, 1, 1), (4098, 256, 3, 1, 1, 1, 0),
+                                      (65536, 127, 3, 1, 1, 1, 0), (65536, 128, 3, 1, 1, 1, 1), (4136, 256, 4, 1, 1, 1, 0), (4136, 256, 5, 1, 1, 1, 1),
+                                      (65536, 64, 16, 1, 4, 1, 0), (65536, 47, 1, 1, 1, 1, 1), (65536, 48, 1, 1, 1, 1, 0), (65536, 64, 11, 1, 1, 1, 1), (500, 64, 3, 5, 1, 1, 0), (500, 64, 3, 3, 1, 1, 0),
+                                      (500, 64, 3, 2, 1, 1, 1), (500, 64, 3, 5, 1, 0, 1), (500, 31, 3, 5, 1, 1, 1), (500, 32, 3, 5, 1, 1, 0),
+                                      (250000, 31, 3, 1, 1, 1, 1),
+                                      (24000, 1, 16, 1, 8, 1, 1)]:
+        assert walk(t(L, C), k, d, (L - (k - 1) * d - 1) // s0 + 1, f16, s0) == want, (L, C, k, d, s0, f16)
+    for f16 in (0, 1):
+        assert walk(t(1000, 80, nb=[4 * 80, 4]), 3, 1, 998, f16) == 2       # channel-major
+        assert walk(t(1000, 80, nb=[8, 8000]), 3, 1, 998, f16) == 0         # every other sample
